@@ -165,6 +165,7 @@ int Engine::reserve(int64_t capacity) {
     d_run = nullptr;
     dtpart = nullptr; dtpart_cap = 0;
     nbr = nullptr; nbr_ovf = nullptr; nbr_bcap = 0; prec = nullptr; fbal = nullptr;
+    no_list_mem = false;
     cap = 0;
     n = 0;
     R = 0;
@@ -184,17 +185,37 @@ int Engine::reserve(int64_t capacity) {
     SPHX_CHECK(alloc((void **)&hist, sizeof(uint32_t) * hist_cap));
     SPHX_CHECK(alloc((void **)&counters, sizeof(int64_t) * CNT_SLOTS));
     SPHX_HIP(hipMemset(counters, 0, sizeof(int64_t) * CNT_SLOTS));
-    if (want_lists && mode == SPHX_MIXED) {
-        // every run has at most one partial bucket
-        int64_t bc = capacity / SPHX_BUCKET + std::max(max_runs, 1) + 1;
-        SPHX_CHECK(alloc((void **)&nbr, sizeof(int32_t) * (size_t)bc * SPHX_NBR_MAX * 64));
-        SPHX_CHECK(alloc((void **)&nbr_ovf, sizeof(int32_t) * 2 * (size_t)bc));
-        SPHX_CHECK(alloc((void **)&prec, sizeof(PairRec) * (size_t)capacity));
-        SPHX_CHECK(alloc((void **)&fbal, sizeof(float) * (size_t)capacity));
-        nbr_bcap = bc;
-    }
+    if (want_lists && mode == SPHX_MIXED) SPHX_CHECK(alloc_lists(capacity));
     cap = capacity;
     return SPHX_OK;
+}
+
+int Engine::alloc_lists(int64_t capacity) {
+    // every run has at most one partial bucket
+    int64_t bc = capacity / SPHX_BUCKET + std::max(max_runs, 1) + 1;
+    SPHX_CHECK(alloc((void **)&nbr, sizeof(int32_t) * (size_t)bc * SPHX_NBR_MAX * 64));
+    SPHX_CHECK(alloc((void **)&nbr_ovf, sizeof(int32_t) * 4 * (size_t)bc));
+    SPHX_CHECK(alloc((void **)&prec, sizeof(PairRec) * (size_t)capacity));
+    SPHX_CHECK(alloc((void **)&fbal, sizeof(float) * (size_t)capacity));
+    nbr_bcap = bc;
+    return SPHX_OK;
+}
+
+// The stateless calls take the lists when there is memory for them and walk
+// otherwise (the results are the same).
+bool Engine::ensure_lists() {
+    if (!nbr_bcap && !no_list_mem) {
+        const size_t held = owned.size();
+        if (alloc_lists(cap) < 0) {
+            for (size_t k = held; k < owned.size(); ++k) hipFree(owned[k]);
+            owned.resize(held);
+            nbr = nullptr; nbr_ovf = nullptr; prec = nullptr; fbal = nullptr;
+            nbr_bcap = 0;
+            no_list_mem = true;  // until the capacity changes
+            (void)hipGetLastError();
+        }
+    }
+    return lists_ready();
 }
 
 int Engine::set_runs(const std::vector<int64_t> &sizes, hipStream_t st) {
@@ -745,7 +766,7 @@ extern "C" int sphx_getDensity(sphx_ctx *ctx, int mode, int64_t n, const double 
     SPHX_CHECK(ctx_load(ctx, n, pos, m, h, nullptr, true, st));
     SPHX_CHECK(E.build_boxes(st, true));
     k_fill_d<<<gu(n), UT, 0, st>>>(E.s.u, 0.0, n);
-    SPHX_CHECK(E.density_eos(st));
+    SPHX_CHECK(E.density_eos(st, E.ensure_lists()));
     SPHX_CHECK(scatter_out(E, E.s.rho, row_beg, row_end, rho, st));
     SPHX_CHECK(scatter_out_i(E, E.tmpi, row_beg, row_end, nngb, st));
     return SPHX_OK;
@@ -854,7 +875,9 @@ extern "C" int sphx_div_curlVel(sphx_ctx *ctx, int mode, int64_t n, const double
     SPHX_CHECK(ctx_load(ctx, n, pos, m, h, v, true, st));
     SPHX_CHECK(gather_in(E, rho, E.s.rho, st));
     SPHX_CHECK(E.build_boxes(st, true));
-    SPHX_CHECK(E.divcurl(st));
+    const bool lists = E.ensure_lists();
+    if (lists) SPHX_CHECK(E.build_lists(st));
+    SPHX_CHECK(E.divcurl(st, lists));
     SPHX_CHECK(scatter_out(E, E.s.divv, row_beg, row_end, divV, st));
     SPHX_CHECK(scatter_out(E, E.s.curlv, row_beg, row_end, curlV, st));
     return SPHX_OK;
@@ -889,7 +912,12 @@ extern "C" int sphx_getAcc_sph(sphx_ctx *ctx, int mode, int64_t n, const double 
         SPHX_CHECK(plain_du(E.s, *p, n, 0, n, E.s.du, st));
     } else {
         SPHX_CHECK(E.build_boxes(st, true));
-        SPHX_CHECK(E.hydro(st));
+        const bool lists = E.ensure_lists();
+        if (lists) {
+            SPHX_CHECK(E.build_lists(st));
+            SPHX_CHECK(E.fill_records(st));
+        }
+        SPHX_CHECK(E.hydro(st, lists));
     }
     SPHX_CHECK(scatter_out_aos(E, E.s.ax, E.s.ay, E.s.az, row_beg, row_end, acc, st));
     SPHX_CHECK(scatter_out(E, E.s.du, row_beg, row_end, dudt, st));

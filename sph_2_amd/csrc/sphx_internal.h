@@ -365,10 +365,12 @@ struct Engine {
     bool want_lists = false;
     bool use_lists = true;      // tuning knob: the walks give the same bits
     int32_t *nbr = nullptr;     // nbr_bcap buckets x SPHX_NBR_MAX x 64
-    int32_t *nbr_ovf = nullptr; // two per bucket (one per half of a half-bucket walk)
+    int32_t *nbr_ovf = nullptr; // four per bucket (one per quarter)
     int64_t nbr_bcap = 0;
     PairRec *prec = nullptr;    // per particle of capacity
     float *fbal = nullptr;      // per particle of capacity
+    bool no_list_mem = false;   // ensure_lists found no memory for them at this capacity
+    int alloc_lists(int64_t capacity);
     bool lists_ready() const;
     int32_t *cand_off = nullptr, *cand_cnt = nullptr, *cand = nullptr;
     int64_t cand_cap = 0;
@@ -457,8 +459,13 @@ struct Engine {
     int smoothing(hipStream_t st, bool predictor);
     int build_candidates(hipStream_t st);
     int density_eos(hipStream_t st, bool lists = false);
-    // groups per bucket of the density walk (1 or 2)
-    int walk_halves() const;
+    // groups per bucket of the smoothing and list walks (1, 2 or 4)
+    int smooth_parts() const;
+    int list_parts() const;
+    int build_lists(hipStream_t st);
+    int fill_records(hipStream_t st);
+    // allocate the lists if they are not; false (and no error) without the memory
+    bool ensure_lists();
     int gravity(hipStream_t st, bool with_pot);
     int divcurl(hipStream_t st, bool lists = false);
     int hydro(hipStream_t st, bool lists = false);

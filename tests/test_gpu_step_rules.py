@@ -1,0 +1,50 @@
+"""The step rules of the smoothing length (h_mode 2-5) where the window of
+distances that replaces their walks is hardest to find: starts far from the
+band, more particles at one distance than the window holds, a run smaller than
+the band, passes that end outside the window.  Every h, count and pass count
+bit for bit the oracle's."""
+import numpy as np
+import pytest
+
+import oracle
+from sph_2_amd import ic
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(name):
+    e = ic.evrard(1500, seed=4)
+    if name == "guess":
+        return e.pos, e.h
+    if name == "starts":  # from a fifth to five times the length
+        return e.pos, e.h * np.geomspace(0.2, 5.0, e.n)
+    if name == "lattice":  # shells of up to 48 particles at one distance
+        g = np.arange(11.0)
+        pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+        return pos, np.full(len(pos), 1.3)
+    if name == "coincident":  # 80 particles on one point among others
+        pos = e.pos[:700].copy()
+        pos[100:180] = pos[100]
+        return pos, e.h[:700]
+    if name == "few":  # fewer particles than the band asks for
+        return e.pos[:50], np.full(50, 0.3)
+    if name == "just_enough":  # 65: the band can be met, never passed
+        return e.pos[:65], np.full(65, 0.9)
+    raise AssertionError(name)
+
+
+@pytest.mark.parametrize("h_mode", [2, 3, 4, 5])
+@pytest.mark.parametrize("name", ["guess", "starts", "lattice", "coincident", "few", "just_enough"])
+def test_step_rules_match_the_oracle(gpu, name, h_mode):
+    import warnings
+
+    from sph_2_amd import libsx
+
+    pos, h0 = _case(name)
+    ho, ko, ito, _ = oracle.smoothing(pos, h0, p=oracle.Params(h_mode=h_mode))
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", RuntimeWarning)  # the pass limit, as in the oracle
+        h, k, it = libsx.smoothing_h(pos, h0, h_mode=h_mode)
+    assert np.array_equal(h, ho)
+    assert np.array_equal(k, ko)
+    assert np.array_equal(it, ito)

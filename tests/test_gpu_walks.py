@@ -1,0 +1,79 @@
+"""The candidate walks at the sizes where their shape changes (a quarter, a half
+or a whole bucket per group: 384 / 385, 1,536 / 1,537 and 3,072 / 3,073 buckets),
+with a partial last bucket, and where the FP32 screen of the FP64 distance test
+is hardest: coordinates far from the origin, units far from one, distances that
+equal the radius.  Counts and smoothing lengths bit for bit the oracle's."""
+import numpy as np
+import pytest
+
+import oracle
+from sph_2_amd import ic
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 1000, 24576, 24577, 98304, 98305, 196608, 196650])
+def test_walk_shapes(gpu, n):
+    from sph_2_amd import libsx
+
+    e = ic.evrard(n, seed=11)
+    rows = np.unique(np.r_[0:min(n, 200), np.linspace(0, n - 1, min(n, 300)).astype(int)])
+    h, k, it = libsx.smoothing_h(e.pos, e.h)
+    ho, ko, ito, _ = oracle.smoothing(e.pos, e.h, rows=rows)
+    assert np.array_equal(h[rows], ho) and np.array_equal(k[rows], ko)
+    assert np.array_equal(it[rows], ito)
+    rho, cnt = libsx.getDensity(e.pos, e.m, h, return_count=True)
+    rho_o, cnt_o = oracle.density(e.pos, e.m, h, rows=rows)
+    assert np.array_equal(cnt[rows], cnt_o)
+    assert np.max(np.abs(rho[rows] / rho_o - 1.0)) < 1e-6
+
+
+@pytest.mark.parametrize("shift,scale", [(1e6, 1.0), (0.0, 3.0e21), (0.0, 1e-150), (0.0, 1e150)])
+def test_walk_frames(gpu, shift, scale):
+    """Offsets and units: the counts only compare distances, so any scale does."""
+    from sph_2_amd import libsx
+
+    e = ic.evrard(3000, seed=12)
+    pos, h0 = e.pos * scale + shift, e.h * scale
+    h, k, _ = libsx.smoothing_h(pos, h0)
+    ho, ko, _, _ = oracle.smoothing(pos, h0)
+    assert np.array_equal(h, ho) and np.array_equal(k, ko)
+
+
+def test_walk_distances_at_the_radius(gpu):
+    """A cubic lattice with h = 1 and 1.5: thousands of pairs lie exactly at r =
+    h_i + h_j, which counts them, and every batch holds one."""
+    from sph_2_amd import libsx
+
+    g = np.arange(14.0)
+    pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    m = np.full(len(pos), 1.0 / len(pos))
+    for h in (1.0, 1.5):
+        hh = np.full(len(pos), h)
+        rho, cnt = libsx.getDensity(pos, m, hh, return_count=True)
+        rho_o, cnt_o = oracle.density(pos, m, hh)
+        assert np.array_equal(cnt, cnt_o)
+        assert np.max(np.abs(rho / rho_o - 1.0)) < 1e-6
+
+
+def test_lists_of_the_stateless_calls_overflow(gpu):
+    """Particles with more neighbours than a list holds beside others without:
+    the stateless density, div/curl and hydro take the walk for those buckets."""
+    from sph_2_amd import libsx
+
+    e = ic.evrard(6000, seed=13)
+    rng = np.random.default_rng(5)
+    v = rng.standard_normal((e.n, 3))
+    h = np.where(e.pos[:, 0] > 0.4, 2.0 * e.h, e.h)
+    rho, cnt = libsx.getDensity(e.pos, e.m, h, return_count=True)
+    rho_o, cnt_o = oracle.density(e.pos, e.m, h)
+    assert cnt_o.max() > 128 and cnt_o.min() < 128
+    assert np.array_equal(cnt, cnt_o)
+    assert np.max(np.abs(rho / rho_o - 1.0)) < 1e-6
+    dv, cv = libsx.div_curlVel(e.pos, v, rho_o, e.m, h)
+    dvo, cvo = oracle.divcurl(e.pos, v, rho_o, e.m, h)
+    P, c = (2.0 / 3.0) * rho_o * e.u, np.sqrt(10.0 / 9.0 * e.u)
+    acc, du = libsx.getAcc_sph_dU(e.pos, v, rho_o, P, c, h, e.m, balsara=1, divV=dvo, curlV=cvo)
+    acco, duo = oracle.hydro(e.pos, v, rho_o, P, c, h, e.m, dvo, cvo, oracle.Params(balsara=1))
+    for a, b in ((dv, dvo), (cv, cvo), (acc, acco), (du, duo)):
+        assert np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum()) < 1e-5
