@@ -181,8 +181,6 @@ int Engine::reserve(int64_t capacity) {
     for (int32_t **q : iptr) SPHX_CHECK(alloc((void **)q, I));
     SPHX_CHECK(alloc((void **)&keys, sizeof(uint64_t) * capacity));
     SPHX_CHECK(alloc((void **)&keys2, sizeof(uint64_t) * capacity));
-    hist_cap = 256 * ((capacity + SPHX_RS_TILE - 1) / SPHX_RS_TILE + 1);
-    SPHX_CHECK(alloc((void **)&hist, sizeof(uint32_t) * hist_cap));
     SPHX_CHECK(alloc((void **)&counters, sizeof(int64_t) * CNT_SLOTS));
     SPHX_HIP(hipMemset(counters, 0, sizeof(int64_t) * CNT_SLOTS));
     if (want_lists && mode == SPHX_MIXED) SPHX_CHECK(alloc_lists(capacity));
@@ -295,6 +293,7 @@ int Engine::set_runs(const std::vector<int64_t> &sizes, hipStream_t st) {
         SPHX_CHECK(alloc((void **)&d_run, sizeof(RunParams) * std::max(nr, 1)));
     }
     drop_graph();
+    sorted_boxes = false;
     int32_t *q = tab_i32;
     t.nb = nb; t.ns = ns; t.R = nr;
     t.boff = 0;

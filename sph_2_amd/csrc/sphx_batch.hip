@@ -114,11 +114,7 @@ static int sort_segment(Engine &E, int r, hipStream_t st) {
     if (n <= 1) return SPHX_OK;
     // keys for the whole packed set are cheap; only the segment is sorted
     SPHX_CHECK(sphx_launch_morton(E, st));
-    int rb = 0;
-    while ((1 << rb) < E.max_runs) ++rb;
-    int bits = 3 * sphx_morton_bits(E.max_runs) + rb;
-    SPHX_CHECK(sphx_radix_sort(E.keys + p0, E.perm + p0, E.keys2 + p0, E.perm2 + p0, E.hist, n,
-                               bits, st));
+    SPHX_CHECK(sphx_sort_keys(E.keys + p0, E.perm + p0, E.keys2 + p0, E.perm2 + p0, n, (int32_t)p0, st));
     for (double *a : moving_d(E)) {
         kb_gather_d<<<gb(n), BT, 0, st>>>(a + p0, E.perm + p0, (int32_t)p0, E.tmpd, n);
         kb_copy_d<<<gb(n), BT, 0, st>>>(E.tmpd, a + p0, n);

@@ -22,8 +22,6 @@
 #include "../../include/sphx.h"
 
 #define SPHX_BUCKET 64
-// keys per workgroup tile of the radix sort (its histograms: 256 per tile)
-#define SPHX_RS_TILE 1024
 #define SPHX_SUPER 64
 #define SPHX_NBR_MAX 128  // entries of a particle's neighbour list (more: its bucket walks)
 
@@ -342,8 +340,6 @@ struct Engine {
     int32_t *perm = nullptr, *perm2 = nullptr;
     double *tmpd = nullptr;   // n doubles
     int32_t *tmpi = nullptr;  // n int32
-    uint32_t *hist = nullptr; // radix histograms
-    int64_t hist_cap = 0;
     double *bbox = nullptr;   // per-run bounding boxes (6 per run) + chunk partials
     int64_t bbox_cap = 0;
     int32_t *h_iters = nullptr;
@@ -360,6 +356,7 @@ struct Engine {
     double *tab_d = nullptr;     // box arrays
     int64_t tab_d_cap = 0;
     Tables t{};
+    bool sorted_boxes = false;  // the bucket boxes in t are those of the sort just done
     // neighbour lists of the density pass for the div/curl and hydro passes
     // (plans and batches; allocated with the capacity when want_lists is set)
     bool want_lists = false;
@@ -526,8 +523,8 @@ int sphx_bh_run(Engine &E, BhHost &H, double theta, bool with_pot, hipStream_t s
 int sphx_gravity_run(Engine &E, const GravConfig &cfg, bool with_pot, hipStream_t st);
 int sphx_gravity_prepare(Engine &E, const GravConfig &cfg, hipStream_t st);
 int sphx_launch_morton(Engine &E, hipStream_t st);
-int sphx_radix_sort(uint64_t *keys, int32_t *vals, uint64_t *keys_tmp, int32_t *vals_tmp,
-                    uint32_t *hist, int64_t n, int key_bits, hipStream_t st);
+int sphx_sort_keys(uint64_t *keys, int32_t *vals, uint64_t *keys_tmp, int32_t *vals_tmp, int64_t n,
+                   int32_t v0, hipStream_t st);
 // Time-step criterion over n particles (acc and acc_g with element strides
 // as/gs); out[0..4] = dt, dt_f, dt_kin, dt_cfl, dt_dens.
 int sphx_global_dt_launch(const double *h, const double *c, const double *acc, int64_t as,

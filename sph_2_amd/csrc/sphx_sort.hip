@@ -1,4 +1,4 @@
-// Morton keys, stable LSD radix sort, permutation gather and bucket boxes.
+// Morton keys, stable merge sort, permutation gather and bucket boxes.
 //
 // Replaces the reference's neighbour structures (counting-sort cells of
 // Particles_in_BH_Tree_II/Evrard_test/ngb_v3.h:58-117, atomics-filled grid
@@ -10,11 +10,6 @@
 #include "sphx_internal.h"
 
 namespace {
-
-constexpr int RS_THREADS = 256;
-constexpr int RS_TILE = SPHX_RS_TILE;
-constexpr int RS_ITEMS = RS_TILE / RS_THREADS;
-static_assert(RS_ITEMS * RS_THREADS == RS_TILE, "a tile is whole rounds of the workgroup");
 
 __device__ __forceinline__ uint64_t spread3(uint64_t v) {
     // Spread the low 21 bits of v so bit b lands at bit 3b.
@@ -29,18 +24,18 @@ __device__ __forceinline__ uint64_t spread3(uint64_t v) {
 
 // Bounding box of each super-bucket straight from the particles (before the
 // sort, in the current order; supers never straddle runs).
-__global__ __launch_bounds__(256) void k_super_box_pos(Tables t, const double *__restrict__ x,
+__global__ __launch_bounds__(1024) void k_super_box_pos(Tables t, const double *__restrict__ x,
                                                        const double *__restrict__ y,
                                                        const double *__restrict__ z,
                                                        double *__restrict__ out /* 6 per super */) {
-    __shared__ double part[4][6];
+    __shared__ double part[16][6];
     const int sidx = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int b0 = t.s_bbeg[sidx], b1 = t.s_bend[sidx];
     const int p0 = t.b_beg[b0];
     const int p1 = t.b_beg[b1 - 1] + t.b_cnt[b1 - 1];
     double v[6] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY};
-    for (int i = p0 + tid; i < p1; i += 256) {
+    for (int i = p0 + tid; i < p1; i += 1024) {
         const double a = x[i], b = y[i], c = z[i];
         v[0] = fmin(v[0], a); v[1] = fmax(v[1], a);
         v[2] = fmin(v[2], b); v[3] = fmax(v[3], b);
@@ -55,7 +50,7 @@ __global__ __launch_bounds__(256) void k_super_box_pos(Tables t, const double *_
     __syncthreads();
     if (tid < 6) {
         double r = part[0][tid];
-        for (int q = 1; q < 4; ++q) r = (tid & 1) ? fmax(r, part[q][tid]) : fmin(r, part[q][tid]);
+        for (int q = 1; q < 16; ++q) r = (tid & 1) ? fmax(r, part[q][tid]) : fmin(r, part[q][tid]);
         out[6 * sidx + tid] = r;
     }
 }
@@ -82,21 +77,22 @@ __global__ void k_run_box(Tables t, const double *__restrict__ sbox, double *__r
 // key = run << (3*bits) | interleave(ix, iy, iz); ix = floor((x - lo) * scale)
 // clamped to [0, 2^bits - 1], scale = 2^bits / (extent * (1 + 2^-30)) over the
 // run's cubic box.  All FP64, separately rounded.
-__global__ void k_morton(const double *__restrict__ x, const double *__restrict__ y,
-                         const double *__restrict__ z, const int32_t *__restrict__ run,
-                         const double *__restrict__ rbox, int64_t n, int bits,
-                         uint64_t *__restrict__ keys, int32_t *__restrict__ vals) {
+struct MortonIn {
+    const double *x, *y, *z;
+    const int32_t *run;  // null: one run
+    const double *rbox;
+    int bits;
+};
+__device__ __forceinline__ uint64_t morton_key(const MortonIn &in, int64_t i) {
 #pragma clang fp contract(off)
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int r = run ? run[i] : 0;
-    const double *b = rbox + 6 * r;
+    int r = in.run ? in.run[i] : 0;
+    const double *b = in.rbox + 6 * r;
     double ex = b[1] - b[0], ey = b[3] - b[2], ez = b[5] - b[4];
     double ext = fmax(ex, fmax(ey, ez));
-    double cells = (double)(1ull << bits);
+    double cells = (double)(1ull << in.bits);
     double scale = ext > 0.0 ? cells / (ext * (1.0 + 0x1p-30)) : 0.0;
-    uint64_t maxc = (1ull << bits) - 1ull;
-    double fx = (x[i] - b[0]) * scale, fy = (y[i] - b[2]) * scale, fz = (z[i] - b[4]) * scale;
+    uint64_t maxc = (1ull << in.bits) - 1ull;
+    double fx = (in.x[i] - b[0]) * scale, fy = (in.y[i] - b[2]) * scale, fz = (in.z[i] - b[4]) * scale;
     uint64_t ix = fx <= 0.0 ? 0ull : (uint64_t)fx;
     uint64_t iy = fy <= 0.0 ? 0ull : (uint64_t)fy;
     uint64_t iz = fz <= 0.0 ? 0ull : (uint64_t)fz;
@@ -104,127 +100,179 @@ __global__ void k_morton(const double *__restrict__ x, const double *__restrict_
     iy = iy > maxc ? maxc : iy;
     iz = iz > maxc ? maxc : iz;
     uint64_t key = (spread3(ix) << 2) | (spread3(iy) << 1) | spread3(iz);
-    key |= ((uint64_t)r) << (3 * bits);
-    keys[i] = key;
-    vals[i] = (int32_t)i;
+    return key | ((uint64_t)r) << (3 * in.bits);
 }
 
-__global__ __launch_bounds__(RS_THREADS) void k_rs_hist(const uint64_t *__restrict__ keys,
-                                                        int64_t n, int shift,
-                                                        uint32_t *__restrict__ hist,
-                                                        int nblocks) {
-    __shared__ uint32_t h[256];
-    int tid = threadIdx.x;
-    h[tid] = 0;
-    __syncthreads();
-    int64_t base = (int64_t)blockIdx.x * RS_TILE;
-    for (int r = 0; r < RS_ITEMS; ++r) {
-        int64_t i = base + r * RS_THREADS + tid;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    hist[(int64_t)tid * nblocks + blockIdx.x] = h[tid];
+__global__ void k_morton(MortonIn in, int64_t n, uint64_t *__restrict__ keys) {
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) keys[i] = morton_key(in, i);
 }
 
-// The scatter offsets are the exclusive scan of the block histograms in
-// digit-major order (entry d * nblocks + b counts digit d in block b).  Two
-// kernels with one workgroup per digit: the first sums each digit's row, the
-// second scans its row on top of the totals of the digits before it.
-__global__ __launch_bounds__(256) void k_rs_digit_total(const uint32_t *__restrict__ hist,
-                                                        int nblocks, uint32_t *__restrict__ tot) {
-    __shared__ uint32_t red[256];
-    const int d = blockIdx.x, tid = threadIdx.x;
-    uint32_t s = 0;
-    for (int b = tid; b < nblocks; b += 256) s += hist[(int64_t)d * nblocks + b];
-    red[tid] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) red[tid] += red[tid + o];
-        __syncthreads();
+// ---------------------------------------------------------------------------
+// Stable sort of (key, value) by the 63-bit key: tiles of 4,096 sorted in LDS,
+// then merged pairwise.  What bounds the sort of a run is launches and the
+// chain of dependent memory trips, not bandwidth (24 bytes a particle and pass),
+// so it is a merge sort: one launch for the tiles, which also make the keys
+// from the positions, and one per doubling, against the 32 of an eight-pass
+// radix sort (histogram, two scans and scatter each).  Half kick, drift, keys,
+// sort and gather together: 141 -> 49 us at 4,096 particles, 153 -> 78 at
+// 65,752, 162 -> 83 at 131,072, 360 -> 213 at 1,048,576.
+// ---------------------------------------------------------------------------
+constexpr int ST_TILE = 4096, ST_THREADS = 1024, ST_ITEMS = ST_TILE / ST_THREADS;
+constexpr int MG_CHUNK = 1024, MG_THREADS = 256, MG_ITEMS = MG_CHUNK / MG_THREADS;
+static_assert(ST_ITEMS == 4 && MG_ITEMS == 4, "four items a thread");
+static_assert((2 * ST_TILE) % MG_CHUNK == 0, "a chunk lies inside one pair of runs");
+
+// How many of the first d outputs of the stable merge of A[0, nA) and B[0, nB)
+// come from A (equal keys: A first).
+__device__ __forceinline__ int merge_split(const uint64_t *A, int nA, const uint64_t *B, int nB, int d) {
+    int lo = d > nB ? d - nB : 0, hi = d < nA ? d : nA;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (A[mid] <= B[d - 1 - mid]) lo = mid + 1;
+        else hi = mid;
     }
-    if (tid == 0) tot[d] = red[0];
+    return lo;
 }
 
-__global__ __launch_bounds__(256) void k_rs_scan_rows(uint32_t *__restrict__ hist, int nblocks,
-                                                      const uint32_t *__restrict__ tot) {
-    __shared__ uint32_t part[256];
-    const int d = blockIdx.x, tid = threadIdx.x;
-    part[tid] = tid < d ? tot[tid] : 0u;  // the digits before this one
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) part[tid] += part[tid + o];
-        __syncthreads();
-    }
-    const uint32_t base = part[0];
-    __syncthreads();
-    // each thread a consecutive piece of the row
-    const int per = (nblocks + 255) / 256;
-    const int b0 = min(nblocks, tid * per), b1 = min(nblocks, b0 + per);
-    uint32_t *row = hist + (int64_t)d * nblocks;
-    uint32_t s = 0;
-    for (int b = b0; b < b1; ++b) s += row[b];
-    part[tid] = s;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        uint32_t v = tid >= off ? part[tid - off] : 0u;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
-    }
-    uint32_t run = base + (tid > 0 ? part[tid - 1] : 0u);
-    for (int b = b0; b < b1; ++b) {
-        uint32_t v = row[b];
-        row[b] = run;
-        run += v;
-    }
-}
-
-// Stable scatter: items keep their order inside each digit.  Items of a tile
-// are taken in rounds of 256 (thread order); inside a wavefront, peers with
-// the same digit are found by matching the 8 digit bits with ballots.
-__global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
-    const uint64_t *__restrict__ kin, const int32_t *__restrict__ vin, uint64_t *__restrict__ kout,
-    int32_t *__restrict__ vout, int64_t n, int shift, const uint32_t *__restrict__ hist,
-    int nblocks) {
-    __shared__ uint32_t base[256];
-    __shared__ uint32_t runc[256];
-    __shared__ uint32_t wcnt[RS_THREADS / 64][256];
-    int tid = threadIdx.x;
-    int lane = tid & 63;
-    int w = tid >> 6;
-    base[tid] = hist[(int64_t)tid * nblocks + blockIdx.x];
-    runc[tid] = 0;
-    uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    int64_t tile = (int64_t)blockIdx.x * RS_TILE;
-    for (int r = 0; r < RS_ITEMS; ++r) {
-        for (int q = 0; q < RS_THREADS / 64; ++q) wcnt[q][tid] = 0;
-        __syncthreads();
-        int64_t i = tile + r * RS_THREADS + tid;
-        bool valid = i < n;
-        uint64_t key = valid ? kin[i] : 0ull;
-        int32_t val = valid ? vin[i] : 0;
-        uint32_t d = (uint32_t)((key >> shift) & 255u);
-        uint64_t peers = __ballot(valid);
+// Four consecutive outputs of the merge from (a, b) on: their indices into
+// [A | B], with B at offset offB of the same array.
+__device__ __forceinline__ void merge_four(const uint64_t *A, int nA, const uint64_t *B, int nB, int a,
+                                           int b, int offB, uint64_t *key, int *at) {
+    uint64_t ka = a < nA ? A[a] : ~0ull, kb = b < nB ? B[b] : ~0ull;
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
-            uint64_t m = __ballot(valid && ((d >> b) & 1u));
-            peers &= ((d >> b) & 1u) ? m : ~m;
+    for (int k = 0; k < 4; ++k) {
+        const bool ta = b >= nB || (a < nA && ka <= kb);
+        key[k] = ta ? ka : kb;
+        at[k] = ta ? a : offB + b;
+        if (ta) {
+            ++a;
+            ka = a < nA ? A[a] : ~0ull;
+        } else {
+            ++b;
+            kb = b < nB ? B[b] : ~0ull;
         }
-        uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && rank == 0) wcnt[w][d] = (uint32_t)__popcll(peers);
+    }
+}
+
+// One tile per workgroup, four items a thread: sorted in registers, then merged
+// in LDS, doubling from runs of four.  Item i's value is v0 + i; MAKE makes the
+// keys from the positions, else they come from kin (which may be kout: a
+// workgroup has its tile in LDS before it writes it).
+template <bool MAKE>
+__global__ __launch_bounds__(ST_THREADS) void k_sort_tiles(MortonIn in, const uint64_t *kin, int64_t n,
+                                                           int32_t v0, uint64_t *kout,
+                                                           int32_t *__restrict__ vout) {
+    __shared__ uint64_t K[ST_TILE];
+    __shared__ uint16_t P[ST_TILE];  // position in the tile
+    const int tid = threadIdx.x;
+    const int64_t base = (int64_t)blockIdx.x * ST_TILE;
+    const int cnt = (int)(n - base < ST_TILE ? n - base : ST_TILE);
+    uint64_t key[4];
+    int at[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int q = 4 * tid + k;
+        at[k] = q;
+        key[k] = ~0ull;  // past the end: after every key (keys have 63 bits)
+        if (q < cnt) key[k] = MAKE ? morton_key(in, base + q) : kin[base + q];
+    }
+    auto order = [&](int i, int j) {
+        const bool sw = key[j] < key[i] || (key[j] == key[i] && at[j] < at[i]);
+        const uint64_t ki = sw ? key[j] : key[i], kj = sw ? key[i] : key[j];
+        const int pi = sw ? at[j] : at[i], pj = sw ? at[i] : at[j];
+        key[i] = ki; key[j] = kj; at[i] = pi; at[j] = pj;
+    };
+    order(0, 1); order(2, 3); order(0, 2); order(1, 3); order(1, 2);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        K[4 * tid + k] = key[k];
+        P[4 * tid + k] = (uint16_t)at[k];
+    }
+    __syncthreads();
+    for (int w = 4; w < cnt; w <<= 1) {
+        const int s = (4 * tid) / (2 * w) * (2 * w), d = 4 * tid - s;
+        const uint64_t *A = K + s, *B = K + s + w;
+        const int a = merge_split(A, w, B, w, d);
+        int idx[4];
+        merge_four(A, w, B, w, a, d - a, w, key, idx);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) at[k] = P[s + idx[k]];
         __syncthreads();
-        if (valid) {
-            uint32_t off = base[d] + runc[d] + rank;
-            for (int q = 0; q < w; ++q) off += wcnt[q][d];
-            kout[off] = key;
-            vout[off] = val;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            K[4 * tid + k] = key[k];
+            P[4 * tid + k] = (uint16_t)at[k];
         }
         __syncthreads();
-        uint32_t add = 0;
-        for (int q = 0; q < RS_THREADS / 64; ++q) add += wcnt[q][tid];
-        runc[tid] += add;
-        // next round's clearing of wcnt follows a barrier at its top
-        __syncthreads();
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int q = 4 * tid + k;
+        if (q < cnt) {
+            kout[base + q] = key[k];
+            vout[base + q] = v0 + (int32_t)base + at[k];
+        }
+    }
+}
+
+// merge_split over global memory by one wavefront, 64 probes at a time.
+__device__ __forceinline__ int merge_split_wave(const uint64_t *A, int nA, const uint64_t *B, int nB,
+                                                int d, int lane) {
+    int lo = d > nB ? d - nB : 0, hi = d < nA ? d : nA;
+    while (lo < hi) {
+        const int step = (hi - lo + 63) / 64;
+        const int b = lo + lane * step;                    // this lane's piece of [lo, hi)
+        const int e = (b + step < hi ? b + step : hi) - 1;  // its last index
+        // pieces whose last element is among A's come first
+        const int c = __popcll(__ballot(b < hi && A[b < hi ? e : lo] <= B[d - 1 - (b < hi ? e : lo)]));
+        lo += c * step;
+        if (lo >= hi) return hi;
+        hi = (lo + step < hi ? lo + step : hi) - 1;  // known not to be among A's
+    }
+    return lo;
+}
+
+// One pass: runs of `len` merged pairwise, 1,024 outputs per workgroup.
+__global__ __launch_bounds__(MG_THREADS) void k_merge(const uint64_t *__restrict__ kin,
+                                                      const int32_t *__restrict__ vin, int64_t n,
+                                                      int64_t len, uint64_t *__restrict__ kout,
+                                                      int32_t *__restrict__ vout) {
+    __shared__ uint64_t K[MG_CHUNK];
+    __shared__ int32_t V[MG_CHUNK];
+    __shared__ int split[2];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int64_t base = (int64_t)blockIdx.x * MG_CHUNK;
+    const int64_t s = base / (2 * len) * (2 * len);
+    const int nA = (int)(n - s < len ? n - s : len);
+    const int64_t rest = n - s - nA;
+    const int nB = (int)(rest < len ? rest : len);
+    const uint64_t *A = kin + s, *B = A + nA;
+    const int d0 = (int)(base - s), d1 = d0 + MG_CHUNK < nA + nB ? d0 + MG_CHUNK : nA + nB;
+    if (w < 2) {
+        const int a = merge_split_wave(A, nA, B, nB, w == 0 ? d0 : d1, lane);
+        if (lane == 0) split[w] = a;
+    }
+    __syncthreads();
+    const int a0 = split[0], ca = split[1] - a0, b0 = d0 - a0, cb = (d1 - d0) - ca;
+    for (int q = tid; q < ca + cb; q += MG_THREADS) {
+        const int64_t g = s + (q < ca ? a0 + q : nA + b0 + (q - ca));
+        K[q] = kin[g];
+        V[q] = vin[g];
+    }
+    __syncthreads();
+    const int d = 4 * tid;
+    if (d >= ca + cb) return;
+    const int a = merge_split(K, ca, K + ca, cb, d);
+    uint64_t key[4];
+    int idx[4];
+    merge_four(K, ca, K + ca, cb, a, d - a, ca, key, idx);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (d + k < ca + cb) {
+            kout[base + d + k] = key[k];
+            vout[base + d + k] = V[idx[k]];
+        }
     }
 }
 
@@ -236,12 +284,33 @@ struct GatherList {
     int nd, ni;
 };
 
-__global__ void k_gather(GatherList g, const int32_t *__restrict__ perm, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    int32_t p = perm[i];
-    for (int a = 0; a < g.nd; ++a) g.dst[a][i] = g.src[a][p];
-    for (int a = 0; a < g.ni; ++a) g.idst[a][i] = g.isrc[a][p];
+// The gather of the sort, one wave per bucket, with the bucket's box from the
+// positions it has in hand (the boxes the smoothing walk reads; a launch less).
+__global__ __launch_bounds__(64) void k_gather(GatherList g, const int32_t *__restrict__ perm,
+                                               Tables t) {
+    const int b = blockIdx.x, lane = threadIdx.x;
+    const bool ok = lane < t.b_cnt[b];
+    const int i = t.b_beg[b] + lane;
+    const int32_t p = ok ? perm[i] : 0;
+    double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+    if (ok) {
+        for (int a = 0; a < 3; ++a) {  // x, y, z
+            const double v = g.src[a][p];
+            g.dst[a][i] = v;
+            lo[a] = hi[a] = v;
+        }
+        for (int a = 3; a < g.nd; ++a) g.dst[a][i] = g.src[a][p];
+        for (int a = 0; a < g.ni; ++a) g.idst[a][i] = g.isrc[a][p];
+    }
+    for (int a = 0; a < 3; ++a) {
+        lo[a] = wave_min_d(lo[a]);
+        hi[a] = wave_max_d(hi[a]);
+    }
+    if (lane == 0) {
+        t.bxl[b] = lo[0]; t.bxh[b] = hi[0];
+        t.byl[b] = lo[1]; t.byh[b] = hi[1];
+        t.bzl[b] = lo[2]; t.bzh[b] = hi[2];
+    }
 }
 
 // Box and largest h and softening of each 64-particle bucket: one wave each.
@@ -329,31 +398,37 @@ int sphx_soa_to_aos(const double *x, const double *y, const double *z, int64_t n
     return SPHX_OK;
 }
 
-// hist holds 256 x (nblocks + 1) entries: the block histograms, then the
-// digit totals.
-int sphx_radix_sort(uint64_t *keys, int32_t *vals, uint64_t *keys_tmp, int32_t *vals_tmp,
-                    uint32_t *hist, int64_t n, int key_bits, hipStream_t st) {
-    if (n <= 1) return SPHX_OK;
-    int nblocks = (int)((n + RS_TILE - 1) / RS_TILE);
-    uint32_t *tot = hist + (int64_t)256 * nblocks;
-    int passes = (key_bits + 7) / 8;
-    uint64_t *ka = keys, *kb = keys_tmp;
-    int32_t *va = vals, *vb = vals_tmp;
-    for (int p = 0; p < passes; ++p) {
-        int shift = 8 * p;
-        k_rs_hist<<<nblocks, RS_THREADS, 0, st>>>(ka, n, shift, hist, nblocks);
-        k_rs_digit_total<<<256, 256, 0, st>>>(hist, nblocks, tot);
-        k_rs_scan_rows<<<256, 256, 0, st>>>(hist, nblocks, tot);
-        k_rs_scatter<<<nblocks, RS_THREADS, 0, st>>>(ka, va, kb, vb, n, shift, hist, nblocks);
-        SPHX_HIP(hipGetLastError());
-        uint64_t *tk = ka; ka = kb; kb = tk;
-        int32_t *tv = va; va = vb; vb = tv;
+// Passes of pairwise merges over n items.
+static int merge_passes(int64_t n) {
+    int m = 0;
+    while (((int64_t)ST_TILE << m) < n) ++m;
+    return m;
+}
+
+// Merge the sorted tiles in (ka, va) until one run is left; it ends in ka / va
+// after an even number of passes, else in kb / vb.
+static int merge_tiles(uint64_t *ka, int32_t *va, uint64_t *kb, int32_t *vb, int64_t n, hipStream_t st) {
+    const unsigned grid = grid_for(n, MG_CHUNK);
+    for (int64_t len = ST_TILE; len < n; len <<= 1) {
+        k_merge<<<grid, MG_THREADS, 0, st>>>(ka, va, n, len, kb, vb);
+        std::swap(ka, kb);
+        std::swap(va, vb);
     }
-    if (ka != keys) {
-        SPHX_HIP(hipMemcpyAsync(keys, ka, sizeof(uint64_t) * n, hipMemcpyDeviceToDevice, st));
-        SPHX_HIP(hipMemcpyAsync(vals, va, sizeof(int32_t) * n, hipMemcpyDeviceToDevice, st));
-    }
+    SPHX_HIP(hipGetLastError());
     return SPHX_OK;
+}
+
+// Sort n keys in place with their indices, counted from v0, in vals; the other
+// two arrays are scratch.
+int sphx_sort_keys(uint64_t *keys, int32_t *vals, uint64_t *keys_tmp, int32_t *vals_tmp, int64_t n,
+                   int32_t v0, hipStream_t st) {
+    if (n <= 0) return SPHX_OK;
+    const bool odd = merge_passes(n) & 1;
+    uint64_t *ka = odd ? keys_tmp : keys, *kb = odd ? keys : keys_tmp;
+    int32_t *va = odd ? vals_tmp : vals, *vb = odd ? vals : vals_tmp;
+    k_sort_tiles<false><<<grid_for(n, ST_TILE), ST_THREADS, 0, st>>>(MortonIn{}, keys, n, v0, ka, va);
+    SPHX_HIP(hipGetLastError());
+    return merge_tiles(ka, va, kb, vb, n, st);
 }
 
 static int run_bits(int max_runs) {
@@ -370,17 +445,24 @@ int sphx_morton_bits(int max_runs) {
     return b > 21 ? 21 : b;
 }
 
-static int run_key_bits(int max_runs) { return 3 * sphx_morton_bits(max_runs) + run_bits(max_runs); }
-
-int sphx_launch_morton(Engine &E, hipStream_t st) {
+// Boxes of the runs (E.bbox), and where their keys come from.
+static int morton_in(Engine &E, MortonIn *in, hipStream_t st) {
     Tables &t = E.t;
     double *sbox = E.bbox;                 // 6 per super
     double *rbox = E.bbox + 6 * (int64_t)t.ns;  // 6 per run
-    k_super_box_pos<<<t.ns, 256, 0, st>>>(t, E.s.x, E.s.y, E.s.z, sbox);
+    k_super_box_pos<<<t.ns, 1024, 0, st>>>(t, E.s.x, E.s.y, E.s.z, sbox);
     k_run_box<<<t.R, 64, 0, st>>>(t, sbox, rbox);
-    k_morton<<<grid_for(E.n, 256), 256, 0, st>>>(E.s.x, E.s.y, E.s.z,
-                                                E.max_runs > 1 ? E.s.run : nullptr, rbox, E.n,
-                                                sphx_morton_bits(E.max_runs), E.keys, E.perm);
+    SPHX_HIP(hipGetLastError());
+    *in = MortonIn{E.s.x, E.s.y, E.s.z, E.max_runs > 1 ? E.s.run : nullptr, rbox,
+                   sphx_morton_bits(E.max_runs)};
+    return SPHX_OK;
+}
+
+// Unsorted keys of every particle.
+int sphx_launch_morton(Engine &E, hipStream_t st) {
+    MortonIn in;
+    SPHX_CHECK(morton_in(E, &in, st));
+    k_morton<<<grid_for(E.n, 256), 256, 0, st>>>(in, E.n, E.keys);
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
 }
@@ -412,8 +494,14 @@ void Engine::swap_sorted() {
 
 int Engine::sort_and_permute(hipStream_t st, bool gather_state) {
     if (n == 0) return SPHX_OK;
-    SPHX_CHECK(sphx_launch_morton(*this, st));
-    SPHX_CHECK(sphx_radix_sort(keys, perm, keys2, perm2, hist, n, run_key_bits(max_runs), st));
+    MortonIn in;
+    SPHX_CHECK(morton_in(*this, &in, st));
+    const bool odd = merge_passes(n) & 1;
+    uint64_t *ka = odd ? keys2 : keys, *kb = odd ? keys : keys2;
+    int32_t *va = odd ? perm2 : perm, *vb = odd ? perm : perm2;
+    k_sort_tiles<true><<<grid_for(n, ST_TILE), ST_THREADS, 0, st>>>(in, nullptr, n, 0, ka, va);
+    SPHX_HIP(hipGetLastError());
+    SPHX_CHECK(merge_tiles(ka, va, kb, vb, n, st));
     if (!gather_state) return SPHX_OK;
     double **d[12], **sp[12];
     int32_t **id[4], **isp[4];
@@ -429,16 +517,20 @@ int Engine::sort_and_permute(hipStream_t st, bool gather_state) {
         g.isrc[a] = *id[a];
         g.idst[a] = *isp[a];
     }
-    k_gather<<<grid_for(n, 256), 256, 0, st>>>(g, perm, n);
+    k_gather<<<t.nb, 64, 0, st>>>(g, perm, t);
     SPHX_HIP(hipGetLastError());
     swap_sorted();
+    sorted_boxes = true;
     return SPHX_OK;
 }
 
 int Engine::build_boxes(hipStream_t st, bool with_h) {
     if (n == 0) return SPHX_OK;
     const double *e = p.eps_from_h ? nullptr : s.eps;
-    k_bucket_boxes<<<t.nb, 64, 0, st>>>(t, s.x, s.y, s.z, s.h, e, with_h ? 1 : 0);
+    // right after a sort the gather has left the buckets' boxes
+    if (with_h || !sorted_boxes)
+        k_bucket_boxes<<<t.nb, 64, 0, st>>>(t, s.x, s.y, s.z, s.h, e, with_h ? 1 : 0);
+    sorted_boxes = false;
     k_super_boxes<<<t.ns, 64, 0, st>>>(t, with_h ? 1 : 0);
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
