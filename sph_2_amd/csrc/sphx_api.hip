@@ -380,14 +380,16 @@ int Engine::forces(hipStream_t st, bool predictor, bool with_pot) {
     const bool lists = lists_ready();
     SPHX_CHECK(tmark(st, PH_DENS, 0));
     SPHX_CHECK(build_boxes(st, true));
-    SPHX_CHECK(density_eos(st, lists));
+    // with eps = h the direct sum leaves the softened pairs to the density pass
+    const bool soft = bh_theta == 0.0 && p.eps_from_h && !with_pot;
+    SPHX_CHECK(density_eos(st, lists, soft));
     SPHX_CHECK(tmark(st, PH_DENS, 1));
     SPHX_CHECK(tmark(st, PH_GRAV, 0));
     if (bh_theta > 0.0) {
         if (!bh) bh = sphx_bh_host_new();
         SPHX_CHECK(sphx_bh_run(*this, *bh, bh_theta, with_pot, st, nullptr));
     } else {
-        SPHX_CHECK(sphx_gravity_run(*this, gcfg, with_pot, st));
+        SPHX_CHECK(sphx_gravity_run(*this, gcfg, with_pot, soft, st));
     }
     SPHX_CHECK(tmark(st, PH_GRAV, 1));
     // without the Balsara switch hydro reads nothing of div/curl's output, and
@@ -605,7 +607,7 @@ int Engine::diagnostics(hipStream_t st, bool with_pe, sphx_diag *out) {
     if (with_pe) {
         if (mode == SPHX_MIXED) {
             SPHX_CHECK(build_boxes(st, true));
-            SPHX_CHECK(sphx_gravity_run(*this, gcfg, true, st));
+            SPHX_CHECK(sphx_gravity_run(*this, gcfg, true, false, st));
         } else {
             const double *eps = p.eps_from_h ? s.h : s.eps;
             SPHX_CHECK(plain_gravity(s.x, s.y, s.z, s.m, eps, p.G, n, 0, n, s.gx, s.gy, s.gz,
@@ -946,7 +948,7 @@ extern "C" int sphx_getAcc_g_smth(sphx_ctx *ctx, int mode, int64_t n, const doub
     SPHX_HIP(hipGetLastError());
     SPHX_CHECK(E.sort_and_permute(st, true));
     SPHX_CHECK(E.build_boxes(st, true));
-    SPHX_CHECK(sphx_gravity_run(E, E.gcfg, pot != nullptr, st));
+    SPHX_CHECK(sphx_gravity_run(E, E.gcfg, pot != nullptr, false, st));
     SPHX_CHECK(scatter_out_aos(E, E.s.gx, E.s.gy, E.s.gz, row_beg, row_end, acc, st));
     if (pot) SPHX_CHECK(scatter_out(E, E.s.pot, row_beg, row_end, pot, st));
     return SPHX_OK;

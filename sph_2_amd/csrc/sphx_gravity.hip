@@ -37,7 +37,7 @@ struct GravIO {
     int64_t n;
     // block time steps: only i-blocks holding a particle whose step ends at
     // substep t1 are computed (blk_B == 0: all)
-    const int32_t *bin;
+    const int32_t *bin;  // (SOFT: ax, ay, az hold the softening sums on entry)
     int32_t blk_B;
     int64_t blk_t1;
 };
@@ -172,6 +172,24 @@ __device__ __forceinline__ void near_pair(IState<IPL> &S, float4 j, float ej, in
     }
 }
 
+// A pair of a near tile when the softened pairs' sums come from the density
+// pass (sphx_soft_factor): point masses, no closer than t = eps_i + eps_j.
+template <int IPL>
+__device__ __forceinline__ void clamp_pair(IState<IPL> &S, float4 j, float ej) {
+#pragma unroll
+    for (int p = 0; p < IPL; ++p) {
+        float dx = j.x - S.x[p];
+        float dy = j.y - S.y[p];
+        float dz = j.z - S.z[p];
+        float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+        const float t = S.e[p] + ej;
+        float s = j.w * sphx_clamped_r3(r2, t);
+        S.ax[p] = __builtin_fmaf(s, dx, S.ax[p]);
+        S.ay[p] = __builtin_fmaf(s, dy, S.ay[p]);
+        S.az[p] = __builtin_fmaf(s, dz, S.az[p]);
+    }
+}
+
 // Fold the tile's FP32 partials, scaled by the tile's common mass when the
 // tile was summed without it (scale 1 otherwise), into the Kahan sums.
 template <int IPL>
@@ -202,7 +220,7 @@ __device__ __forceinline__ double block_max(double v, double *red) {
     return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
 }
 
-template <int IPL, int TJ, bool POT>
+template <int IPL, int TJ, bool POT, bool SOFT>
 __global__ __launch_bounds__(256) void k_grav(GravTabs gt, GravIO io) {
     __shared__ float4 jt[TJ];
     __shared__ float je[TJ];
@@ -298,6 +316,9 @@ __global__ __launch_bounds__(256) void k_grav(GravTabs gt, GravIO io) {
         } else if (far) {
 #pragma unroll 8
             for (int q = 0; q < TJ; ++q) far_pair<IPL, POT, false>(S, jt[q]);
+        } else if (SOFT) {
+#pragma unroll 8
+            for (int q = 0; q < TJ; ++q) clamp_pair<IPL>(S, jt[q], je[q]);
         } else {
             for (int q = 0; q < TJ; ++q) near_pair<IPL, POT>(S, jt[q], je[q], j0 + q);
         }
@@ -313,6 +334,9 @@ __global__ __launch_bounds__(256) void k_grav(GravTabs gt, GravIO io) {
         double az = io.G * S.kz[p].value();
         double ph = -io.G * S.kp[p].value();
         if (gt.js == 1) {
+            if (SOFT) {
+                ax += io.G * io.ax[i]; ay += io.G * io.ay[i]; az += io.G * io.az[i];
+            }
             io.ax[i] = ax; io.ay[i] = ay; io.az[i] = az;
             if (POT) io.pot[i] = ph;
         } else {
@@ -322,11 +346,16 @@ __global__ __launch_bounds__(256) void k_grav(GravTabs gt, GravIO io) {
     }
 }
 
+// soft: G times the softening sums in ax, ay, az come first.
 __global__ void k_grav_reduce(const double *__restrict__ part, int js, int64_t n, int64_t p0,
-                              int64_t p1, double *ax, double *ay, double *az, double *pot) {
+                              int64_t p1, double G, int soft, double *ax, double *ay, double *az,
+                              double *pot) {
     int64_t i = p0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p1) return;
     double s[4] = {0, 0, 0, 0};
+    if (soft) {
+        s[0] = G * ax[i]; s[1] = G * ay[i]; s[2] = G * az[i];
+    }
     for (int k = 0; k < js; ++k) {
         const double *pp = part + ((int64_t)k * n + i) * 4;
         s[0] += pp[0]; s[1] += pp[1]; s[2] += pp[2]; s[3] += pp[3];
@@ -336,10 +365,12 @@ __global__ void k_grav_reduce(const double *__restrict__ part, int js, int64_t n
 }
 
 template <int IPL, int TJ>
-int launch_grav(const GravTabs &gt, const GravIO &io, int nblocks, bool pot, hipStream_t st) {
+int launch_grav(const GravTabs &gt, const GravIO &io, int nblocks, bool pot, bool soft,
+                hipStream_t st) {
     dim3 grid((unsigned)(nblocks * gt.js));
-    if (pot) k_grav<IPL, TJ, true><<<grid, 256, 0, st>>>(gt, io);
-    else k_grav<IPL, TJ, false><<<grid, 256, 0, st>>>(gt, io);
+    if (pot) k_grav<IPL, TJ, true, false><<<grid, 256, 0, st>>>(gt, io);
+    else if (soft) k_grav<IPL, TJ, false, true><<<grid, 256, 0, st>>>(gt, io);
+    else k_grav<IPL, TJ, false, false><<<grid, 256, 0, st>>>(gt, io);
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
 }
@@ -403,29 +434,6 @@ __device__ __forceinline__ float sym_rot(float v, int addr) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(addr, __float_as_int(v)));
 }
 
-// The spline-softened force factor of near_pair, without mass or potential;
-// t = eps_i + eps_j is twice the pair's softening e.  Newtonian where
-// r^2 >= t^2, the same test as r^2 >= (4e) e (both products round alike).
-// r^-1 is taken once, before the softening test, and also gives r = r^2 r^-1
-// inside the softening length: a transcendental costs several FP32
-// instructions' issue time, and a wave whose lanes split between the two
-// branches runs both.
-__device__ __forceinline__ float sym_spline_f(float r2, float t) {
-    const float ri = __builtin_amdgcn_rsqf(r2);
-    if (r2 >= t * t) return ri * ri * ri;
-    const float e = 0.5f * t;
-    const float r = r2 > 0.0f ? r2 * ri : 0.0f;
-    const float ie = __builtin_amdgcn_rcpf(e);
-    const float q = r * ie;
-    if (q <= 1.0f) {
-        float q2 = q * q;
-        return ie * ie * ie * (4.0f / 3.0f - 1.2f * q2 + 0.5f * q2 * q);
-    }
-    float w = 2.0f - q;
-    float w2 = w * w;
-    return ri * ri * ri * (1.0f - w2 * w2 * (1.0f - 0.8f * w + w2 * (1.0f / 6.0f)));
-}
-
 // The i particles a lane holds: P of them (8 on the far path, 4 on the near
 // one), with their FP32 force sums of the current j chunk.
 template <int P>
@@ -462,7 +470,9 @@ __device__ __forceinline__ SymJ sym_load(const double *x, const double *y, const
 }
 
 // MODE 0: far, common masses (applied later); 1: far; 2: near; 3: diagonal
-// block (one-sided, spline).
+// block (one-sided, spline).  With the softened pairs' sums from the density
+// pass (sphx_soft_factor), point masses no closer than eps_i + eps_j: 4 near;
+// 5 near, common masses; 6 diagonal; 7 diagonal, common mass.
 template <int MODE, int P>
 __device__ __forceinline__ void sym_pairs(SymIP<P> &S, SymJ &J) {
 #pragma unroll
@@ -475,15 +485,18 @@ __device__ __forceinline__ void sym_pairs(SymIP<P> &S, SymJ &J) {
         if (MODE <= 1) {
             float ri = __builtin_amdgcn_rsqf(r2);
             f = (ri * ri) * ri;
+        } else if (MODE >= 4) {
+            f = sphx_clamped_r3(r2, S.e[p] + J.e);
         } else {
-            f = sym_spline_f(r2, S.e[p] + J.e);
+            f = sphx_spline_f(r2, S.e[p] + J.e);
         }
-        float si = MODE == 0 ? f : J.m * f;
+        constexpr bool COMMON = MODE == 0 || MODE == 5 || MODE == 7;
+        float si = COMMON ? f : J.m * f;
         S.ax[p] = __builtin_fmaf(si, dx, S.ax[p]);
         S.ay[p] = __builtin_fmaf(si, dy, S.ay[p]);
         S.az[p] = __builtin_fmaf(si, dz, S.az[p]);
-        if (MODE != 3) {
-            float sj = MODE == 0 ? f : S.m[p] * f;
+        if (MODE != 3 && MODE < 6) {
+            float sj = COMMON ? f : S.m[p] * f;
             J.fx = __builtin_fmaf(-sj, dx, J.fx);
             J.fy = __builtin_fmaf(-sj, dy, J.fy);
             J.fz = __builtin_fmaf(-sj, dz, J.fz);
@@ -496,9 +509,9 @@ __device__ __forceinline__ void sym_rotate(SymJ &J, int addr) {
     J.x = sym_rot(J.x, addr);
     J.y = sym_rot(J.y, addr);
     J.z = sym_rot(J.z, addr);
-    if (MODE != 0) J.m = sym_rot(J.m, addr);
+    if (MODE != 0 && MODE != 5 && MODE != 7) J.m = sym_rot(J.m, addr);
     if (MODE >= 2) J.e = sym_rot(J.e, addr);
-    if (MODE != 3) {
+    if (MODE != 3 && MODE < 6) {
         J.fx = sym_rot(J.fx, addr);
         J.fy = sym_rot(J.fy, addr);
         J.fz = sym_rot(J.fz, addr);
@@ -521,7 +534,7 @@ __device__ __forceinline__ void sym_pairs_masked(SymIP<P> &S, SymJ &J, unsigned 
             float ri = __builtin_amdgcn_rsqf(r2);
             f = (ri * ri) * ri;
         } else {
-            f = sym_spline_f(r2, S.e[p] + J.e);
+            f = sphx_spline_f(r2, S.e[p] + J.e);
         }
         float si = J.m * f;
         S.ax[p] = __builtin_fmaf(si, dx, S.ax[p]);
@@ -555,6 +568,32 @@ __device__ __forceinline__ void sym_chunk(SymIP<P> &S, SymJ &A, SymJ &B, int add
     }
 }
 
+// The same for a near block pair (MODE 4 or 5), whose sums are the largest: the
+// j sets' FP32 sums are folded every SYM_FOLD steps (SYM_FOLD x 8 pairs) into
+// totals that travel with them by one rotation of SYM_FOLD lanes a fold.  With
+// all 512 terms in one FP32 sum the forces were 20-30 % further from the FP64
+// direct sum.
+constexpr int SYM_FOLD = 16;
+template <int MODE>
+__device__ __forceinline__ void sym_chunk_fold(SymI &S, SymJ &A, SymJ &B, int addr) {
+    const int far = (addr + 4 * (SYM_FOLD - 1)) & 255;  // lane L + SYM_FOLD
+    float ax = 0.0f, ay = 0.0f, az = 0.0f, bx = 0.0f, by = 0.0f, bz = 0.0f;
+#pragma unroll 1
+    for (int q = 0; q < 64 / SYM_FOLD; ++q) {
+        for (int s = 0; s < SYM_FOLD; ++s) {
+            sym_pairs<MODE>(S, A);
+            sym_rotate<MODE>(A, addr);
+            sym_pairs<MODE>(S, B);
+            sym_rotate<MODE>(B, addr);
+        }
+        ax = sym_rot(ax, far) + A.fx; ay = sym_rot(ay, far) + A.fy; az = sym_rot(az, far) + A.fz;
+        bx = sym_rot(bx, far) + B.fx; by = sym_rot(by, far) + B.fy; bz = sym_rot(bz, far) + B.fz;
+        A.fx = A.fy = A.fz = B.fx = B.fy = B.fz = 0.0f;
+    }
+    A.fx = ax; A.fy = ay; A.fz = az;
+    B.fx = bx; B.fy = by; B.fz = bz;
+}
+
 // Block-pair mode of tile J for row I (wave-uniform): 3 diagonal, 2 near
 // (spline path), 0 far with common masses on both sides, 1 far.
 __device__ __forceinline__ int sym_mode(const double *bI, const double *bJ, bool diag) {
@@ -566,10 +605,12 @@ __device__ __forceinline__ int sym_mode(const double *bI, const double *bJ, bool
     return far ? ((bI[7] >= 0.0 && bJ[7] >= 0.0) ? 0 : 1) : 2;
 }
 
-// One segment of row I, restricted to its far block pairs: the i block held
-// as 8 per lane.  Its i-side sums are stored in the segment's slots, or added
-// to what the segment's near pairs stored there before (add).  Every j-side
-// slot belongs to exactly one block pair, near or far.
+// One segment of row I, the i block held as 8 per lane: all its block pairs with
+// SOFT, else only the far ones (the near ones' spline needs registers that the
+// eight i leave no room for).  Its i-side sums are stored in the segment's
+// slots, or added to what the segment's near pairs stored there before (add).
+// Every j-side slot belongs to exactly one block pair, near or far.
+template <bool SOFT>
 __device__ __forceinline__ void sym_segment_far(const SymTabs &T, const double *__restrict__ x,
                                                 const double *__restrict__ y,
                                                 const double *__restrict__ z,
@@ -610,22 +651,30 @@ __device__ __forceinline__ void sym_segment_far(const SymTabs &T, const double *
         const int jb = T.b_beg[J], jc = T.b_cnt[J];
         const double *bJ = T.bbox + 8 * (int64_t)J;
         if (!actI && !T.act[J]) continue;
-        const int mode = sym_mode(bI, bJ, J == I);
-        if (mode > 1) continue;
-        const float si = mode == 0 ? (float)bJ[7] : 1.0f;  // i-side scale: the j block's mass
-        const float sj = mode == 0 ? (float)mI : 1.0f;     // j-side scale: the i block's mass
+        int mode = sym_mode(bI, bJ, J == I);
+        if (!SOFT && mode > 1) continue;
+        const bool same = mI >= 0.0 && bJ[7] >= 0.0;  // common masses on both sides
+        if (SOFT && mode >= 2) mode = mode == 2 ? (same ? 5 : 4) : (same ? 7 : 6);
+        const bool common = mode == 0 || mode == 5 || mode == 7;
+        const float si = common ? (float)bJ[7] : 1.0f;  // i-side scale: the j block's mass
+        const float sj = common ? (float)mI : 1.0f;     // j-side scale: the i block's mass
         const int ce = jc < c0 + T.jspan ? jc : c0 + T.jspan;
         for (int c = c0; c < ce; c += 128) {
             SymJ A = sym_load(x, y, z, m, eps, jb, jc, c + lane, ox, oy, oz);
             SymJ B = sym_load(x, y, z, m, eps, jb, jc, c + 64 + lane, ox, oy, oz);
             if (mode == 0) sym_chunk<0>(S, A, B, addr);
-            else sym_chunk<1>(S, A, B, addr);
+            else if (!SOFT || mode == 1) sym_chunk<1>(S, A, B, addr);
+            else if (mode == 4) sym_chunk_fold<4>(S, A, B, addr);
+            else if (mode == 5) sym_chunk_fold<5>(S, A, B, addr);
+            else if (mode == 6) sym_chunk<6>(S, A, B, addr);
+            else sym_chunk<7>(S, A, B, addr);
+            const bool two = !SOFT || mode < 6;  // the diagonal block is one-sided
             int qa = c + lane, qb = c + 64 + lane;
-            if (qa < jc) {
+            if (two && qa < jc) {
                 int64_t o = roff + (jb + qa - rj0);
                 T.px[o] = sj * A.fx; T.py[o] = sj * A.fy; T.pz[o] = sj * A.fz;
             }
-            if (qb < jc) {
+            if (two && qb < jc) {
                 int64_t o = roff + (jb + qb - rj0);
                 T.px[o] = sj * B.fx; T.py[o] = sj * B.fy; T.pz[o] = sj * B.fz;
             }
@@ -811,11 +860,15 @@ __device__ __forceinline__ bool sym_segment_near(const SymTabs &T, const double 
 // per SIMD: both paths fit 168 VGPRs without spills).  Near work, a few
 // percent of the pairs at 1M particles but a third at 65K, is spread over the
 // same launch as the far work instead of trailing it.
+// SOFT: the softened pairs' sums come from the density pass, so that a near
+// block pair costs four instructions a pair more than a far one instead of the
+// spline's divergent branches, and both run in one pass over the segment.
+template <bool SOFT>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_grav_sym(
     SymTabs T, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, const double *__restrict__ eps) {
-    const bool near = sym_segment_near(T, x, y, z, m, eps);
-    sym_segment_far(T, x, y, z, m, eps, near);
+    const bool near = SOFT ? false : sym_segment_near(T, x, y, z, m, eps);
+    sym_segment_far<SOFT>(T, x, y, z, m, eps, near);
 }
 
 
@@ -1157,7 +1210,7 @@ static int sym_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
     return SPHX_OK;
 }
 
-static int sym_run(Engine &E, hipStream_t st) {
+static int sym_run(Engine &E, bool soft, hipStream_t st) {
     SymHost &H = *E.grav.sym;
     int32_t *d = H.dev_i;
     int s0 = 0, s1 = H.nseg;
@@ -1177,7 +1230,8 @@ static int sym_run(Engine &E, hipStream_t st) {
     k_tile_boxes<<<H.nblocks, 64, 0, st>>>(E.t, d + H.o_runb0, H.nblocks, SYM_B, E.s.m, H.bbox,
                                            blk ? E.s.bin : nullptr, E.blk_B, E.blk_t1, H.act);
     const unsigned pg = (unsigned)((p1 - p0 + 255) / 256);
-    k_grav_sym_zero<<<pg, 256, 0, st>>>(p0, p1, E.s.gx, E.s.gy, E.s.gz);
+    // with soft the sums start from the softened pairs' instead of zero
+    if (!soft) k_grav_sym_zero<<<pg, 256, 0, st>>>(p0, p1, E.s.gx, E.s.gy, E.s.gz);
     SPHX_HIP(hipGetLastError());
     const double *eps = E.p.eps_from_h ? E.s.h : E.s.eps;
     // the kernel-time phase spans the pair launches (and, with several bands,
@@ -1199,7 +1253,8 @@ static int sym_run(Engine &E, hipStream_t st) {
                   H.seg_tj};
         if (!marked) SPHX_CHECK(E.tmark(st, PH_GRAVK, 0));
         marked = true;
-        k_grav_sym<<<(unsigned)(b - a), 64, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
+        if (soft) k_grav_sym<true><<<(unsigned)(b - a), 64, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
+        else k_grav_sym<false><<<(unsigned)(b - a), 64, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
         SPHX_HIP(hipGetLastError());
         if (--left == 0) SPHX_CHECK(E.tmark(st, PH_GRAVK, 1));
         k_grav_sym_reduce<<<pg, 256, 0, st>>>(T, E.p.G, p0, p1, bd.row_lo, bd.row_hi, E.s.gx,
@@ -1269,11 +1324,17 @@ int sphx_gravity_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
     return SPHX_OK;
 }
 
-int sphx_gravity_run(Engine &E, const GravConfig &cfg_in, bool with_pot, hipStream_t st) {
+// soft: E.s.gx..gz hold the softened pairs' sums (sphx_soft_factor) that the
+// density pass of the same forces left there.
+int sphx_gravity_run(Engine &E, const GravConfig &cfg_in, bool with_pot, bool soft, hipStream_t st) {
     if (E.n == 0) return SPHX_OK;
+    if (with_pot && soft) {
+        sphx_set_error("the potential is summed with the spline");
+        return SPHX_ERR_STATE;
+    }
     if (cfg_in.ipl == 8 && !with_pot) {
         SPHX_CHECK(sym_prepare(E, cfg_in, st));
-        return sym_run(E, st);
+        return sym_run(E, soft, st);
     }
     // the symmetric sum carries no potential: that call uses the tiled sum
     const GravConfig cfg = cfg_in.ipl == 8 ? GravConfig{2, 512, 1} : cfg_in;
@@ -1302,13 +1363,13 @@ int sphx_gravity_run(Engine &E, const GravConfig &cfg_in, bool with_pot, hipStre
     int rc;
     SPHX_CHECK(E.tmark(st, PH_GRAVK, 0));
     switch (cfg.ipl * 10000 + cfg.tj) {
-        case 10256: rc = launch_grav<1, 256>(gt, io, nblk, with_pot, st); break;
-        case 10512: rc = launch_grav<1, 512>(gt, io, nblk, with_pot, st); break;
-        case 20256: rc = launch_grav<2, 256>(gt, io, nblk, with_pot, st); break;
-        case 20512: rc = launch_grav<2, 512>(gt, io, nblk, with_pot, st); break;
-        case 21024: rc = launch_grav<2, 1024>(gt, io, nblk, with_pot, st); break;
-        case 40256: rc = launch_grav<4, 256>(gt, io, nblk, with_pot, st); break;
-        case 40512: rc = launch_grav<4, 512>(gt, io, nblk, with_pot, st); break;
+        case 10256: rc = launch_grav<1, 256>(gt, io, nblk, with_pot, soft, st); break;
+        case 10512: rc = launch_grav<1, 512>(gt, io, nblk, with_pot, soft, st); break;
+        case 20256: rc = launch_grav<2, 256>(gt, io, nblk, with_pot, soft, st); break;
+        case 20512: rc = launch_grav<2, 512>(gt, io, nblk, with_pot, soft, st); break;
+        case 21024: rc = launch_grav<2, 1024>(gt, io, nblk, with_pot, soft, st); break;
+        case 40256: rc = launch_grav<4, 256>(gt, io, nblk, with_pot, soft, st); break;
+        case 40512: rc = launch_grav<4, 512>(gt, io, nblk, with_pot, soft, st); break;
         default:
             sphx_set_error("unsupported gravity configuration");
             return SPHX_ERR_ARG;
@@ -1322,7 +1383,7 @@ int sphx_gravity_run(Engine &E, const GravConfig &cfg_in, bool with_pot, hipStre
             p1 = E.rp1;
         }
         k_grav_reduce<<<(unsigned)((p1 - p0 + 255) / 256), 256, 0, st>>>(
-            H.part, cfg.js, E.n, p0, p1, E.s.gx, E.s.gy, E.s.gz, with_pot ? E.s.pot : nullptr);
+            H.part, cfg.js, E.n, p0, p1, E.p.G, soft ? 1 : 0, E.s.gx, E.s.gy, E.s.gz, with_pot ? E.s.pot : nullptr);
         SPHX_HIP(hipGetLastError());
     }
     return SPHX_OK;

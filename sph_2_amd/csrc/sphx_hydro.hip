@@ -1168,6 +1168,25 @@ __device__ __forceinline__ float density_term(float mj, double dx, double dy, do
     return mj * (SPHX_SIGMA_F * h3 * w_shape(g.r, g.hinv, g.q));
 }
 
+// Sums of the softened pairs' gravity (sphx_soft_factor), without G.
+struct SoftSum {
+    KahanF x, y, z;
+    __device__ __forceinline__ void init() { x.init(); y.init(); z.init(); }
+    __device__ __forceinline__ void add(float mj, double dx, double dy, double dz, double r2, double hi,
+                                        double hj) {
+#pragma clang fp contract(off)
+        const float s = -mj * sphx_soft_factor((float)r2, (float)hi + (float)hj);
+        x.add(s * (float)dx);
+        y.add(s * (float)dy);
+        z.add(s * (float)dz);
+    }
+    __device__ __forceinline__ void store(const Soa &s, int i) const {
+        s.gx[i] = x.value();
+        s.gy[i] = y.value();
+        s.gz[i] = z.value();
+    }
+};
+
 // rho and EOS of particle i, and what the pair passes stage of them for a
 // neighbour.
 __device__ __forceinline__ void density_store(const Soa &s, const DensArgs &a, int i,
@@ -1187,6 +1206,7 @@ __device__ __forceinline__ void density_store(const Soa &s, const DensArgs &a, i
 }
 
 // Density and EOS of the particles of bucket b by the candidate walk.
+template <bool SOFT>
 __device__ __forceinline__ void density_bucket(const Tables &t, const Soa &s, const DensArgs &a,
                                                int b) {
     __shared__ double sx[64], sy[64], sz[64], sh[64];
@@ -1201,6 +1221,8 @@ __device__ __forceinline__ void density_bucket(const Tables &t, const Soa &s, co
     const double ib[6] = {t.bxl[b], t.bxh[b], t.byl[b], t.byh[b], t.bzl[b], t.bzh[b]};
     KahanF acc;
     acc.init();
+    SoftSum soft;
+    soft.init();
     int nn = 0;
     int ncand = 0;
     const int r = t.b_run[b];
@@ -1251,8 +1273,9 @@ __device__ __forceinline__ void density_bucket(const Tables &t, const Soa &s, co
             __syncthreads();
             // candidates four at a time, their LDS loads issued before the tests
             // (each pair is met in the same order as one at a time)
-            auto pair = [&](int q, double dx, double dy, double dz, double r2, double tt) {
+            auto pair = [&](int q, double dx, double dy, double dz, double r2, double tt, double hj) {
                     acc.add(density_term(sm[q], dx, dy, dz, r2, tt));
+                    if (SOFT) soft.add(sm[q], dx, dy, dz, r2, hi, hj);
                     ++nn;
                 };
             int q0 = 0;
@@ -1267,27 +1290,29 @@ __device__ __forceinline__ void density_bucket(const Tables &t, const Soa &s, co
                     double dx = xi - cx[u], dy = yi - cy[u], dz = zi - cz[u];
                     double r2 = sphx_r2(dx, dy, dz);
                     double tt = hi + ch[u];
-                    if (mine && r2 <= sphx_sq(tt)) pair(q0 + u, dx, dy, dz, r2, tt);
+                    if (mine && r2 <= sphx_sq(tt)) pair(q0 + u, dx, dy, dz, r2, tt, ch[u]);
                 }
             }
             for (int q = q0; q < k.n; ++q) {
                 double dx = xi - sx[q], dy = yi - sy[q], dz = zi - sz[q];
                 double r2 = sphx_r2(dx, dy, dz);
                 double tt = hi + sh[q];
-                if (mine && r2 <= sphx_sq(tt)) pair(q, dx, dy, dz, r2, tt);
+                if (mine && r2 <= sphx_sq(tt)) pair(q, dx, dy, dz, r2, tt, sh[q]);
             }
         });
     }
     if (ok) {
         density_store(s, a, i, acc);
+        if (SOFT) soft.store(s, i);
         if (a.nsym) a.nsym[i] = nn;
     }
     if (lane == 0 && a.counters)
         atomicAdd((unsigned long long *)&a.counters[CNT_CAND], (unsigned long long)ncand);
 }
 
+template <bool SOFT>
 __global__ __launch_bounds__(64) void k_density(Tables t, Soa s, DensArgs a) {
-    density_bucket(t, s, a, t.boff + xcd_block(blockIdx.x, gridDim.x));
+    density_bucket<SOFT>(t, s, a, t.boff + xcd_block(blockIdx.x, gridDim.x));
 }
 
 // Neighbour lists: the candidates with r_ij^2 <= (h_i + h_j)^2 of every
@@ -1411,6 +1436,7 @@ __device__ __forceinline__ bool bucket_ovf(const int32_t *ovf, int64_t b) {
 // Density and EOS over the lists: the eight gathers of a run of list entries
 // are issued together (the sums keep the list order, the walk's).  Bound: the
 // latency of the gathers (L2-served, 36 of a record's 80 bytes).
+template <bool SOFT>
 __global__ __launch_bounds__(64) void k_density_list(Tables t, Soa s, DensArgs a) {
     const int b = t.boff + xcd_block(blockIdx.x, gridDim.x);
     if (bucket_ovf(a.ovf, b)) return;  // the walk launch takes this bucket
@@ -1429,6 +1455,8 @@ __global__ __launch_bounds__(64) void k_density_list(Tables t, Soa s, DensArgs a
     const int32_t *lp = a.lst + (int64_t)b * SPHX_NBR_MAX * 64;
     KahanF acc;
     acc.init();
+    SoftSum soft;
+    soft.init();
     for (int k0 = 0; k0 < maxlen; k0 += 8) {
         int j[8];
         {
@@ -1462,13 +1490,18 @@ __global__ __launch_bounds__(64) void k_density_list(Tables t, Soa s, DensArgs a
                 const double r2 = sphx_r2(dx, dy, dz);
                 const double tt = hi + h[k];
                 acc.add(density_term(m[k], dx, dy, dz, r2, tt));
+                if (SOFT) soft.add(m[k], dx, dy, dz, r2, hi, h[k]);
             }
         }
     }
-    if (ok) density_store(s, a, i, acc);
+    if (ok) {
+        density_store(s, a, i, acc);
+        if (SOFT) soft.store(s, i);
+    }
 }
 
 // The walk for the buckets whose lists overflowed.
+template <bool SOFT>
 __global__ __launch_bounds__(64) void k_density_ovf(Tables t, Soa s, DensArgs a, int nb) {
     const int lane = threadIdx.x;
     for (int base = blockIdx.x * 64; base < nb; base += gridDim.x * 64) {
@@ -1478,7 +1511,7 @@ __global__ __launch_bounds__(64) void k_density_ovf(Tables t, Soa s, DensArgs a,
         while (m) {
             int q = __builtin_ctzll(m);
             m &= m - 1;
-            density_bucket(t, s, a, t.boff + base + q);
+            density_bucket<SOFT>(t, s, a, t.boff + base + q);
         }
     }
 }
@@ -2201,19 +2234,25 @@ int Engine::fill_records(hipStream_t st) {
     return SPHX_OK;
 }
 
-int Engine::density_eos(hipStream_t st, bool lists) {
+int Engine::density_eos(hipStream_t st, bool lists, bool soft) {
     if (n == 0 || nb_launch() == 0) return SPHX_OK;
     if (!lists) {
         DensArgs a{p.gamma, tmpi, counters, nullptr, nullptr, nullptr};
-        k_density<<<nb_launch(), 64, 0, st>>>(tview(), s, a);
+        if (soft) k_density<true><<<nb_launch(), 64, 0, st>>>(tview(), s, a);
+        else k_density<false><<<nb_launch(), 64, 0, st>>>(tview(), s, a);
         SPHX_HIP(hipGetLastError());
         return SPHX_OK;
     }
     SPHX_CHECK(build_lists(st));
     DensArgs a{p.gamma, tmpi, counters, nbr, prec, nbr_ovf};
     const int nb = (int)nb_launch();
-    k_density_list<<<nb, 64, 0, st>>>(tview(), s, a);
-    k_density_ovf<<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+    if (soft) {
+        k_density_list<true><<<nb, 64, 0, st>>>(tview(), s, a);
+        k_density_ovf<true><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+    } else {
+        k_density_list<false><<<nb, 64, 0, st>>>(tview(), s, a);
+        k_density_ovf<false><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+    }
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
 }

@@ -143,6 +143,50 @@ struct KahanF {
     __device__ __forceinline__ double value() const { return (double)s - (double)c; }
 };
 
+// The spline-softened force factor of a pair, without mass or potential;
+// t = eps_i + eps_j is twice the pair's softening e.  Newtonian where
+// r^2 >= t^2, the same test as r^2 >= (4e) e (both products round alike).
+// r^-1 is taken once, before the softening test, and also gives r = r^2 r^-1
+// inside the softening length: a transcendental costs several FP32
+// instructions' issue time, and a wave whose lanes split between the two
+// branches runs both.
+__device__ __forceinline__ float sphx_spline_f(float r2, float t) {
+    const float ri = __builtin_amdgcn_rsqf(r2);
+    if (r2 >= t * t) return ri * ri * ri;
+    const float e = 0.5f * t;
+    const float r = r2 > 0.0f ? r2 * ri : 0.0f;
+    const float ie = __builtin_amdgcn_rcpf(e);
+    const float q = r * ie;
+    if (q <= 1.0f) {
+        float q2 = q * q;
+        return ie * ie * ie * (4.0f / 3.0f - 1.2f * q2 + 0.5f * q2 * q);
+    }
+    float w = 2.0f - q;
+    float w2 = w * w;
+    return ri * ri * ri * (1.0f - w2 * w2 * (1.0f - 0.8f * w + w2 * (1.0f / 6.0f)));
+}
+
+// Softened pairs apart from the rest.  With softening eps = h the pairs inside
+// the spline, r < t = eps_i + eps_j, are the neighbours r < h_i + h_j that the
+// density pass sums over anyway.  The direct sum then takes every pair as point
+// masses no closer than t, without a branch,
+//   f0(r) = max(r^2, t^2)^(-3/2),
+// and the density pass adds (spline - f0) over the neighbours.  f0 is bounded by
+// the spline's own scale (an eighth of e^-3 against 4/3), so nothing cancels.
+// A near pair's spline cost a wave both divergent branches (about 45 instructions
+// against 18).  Launch of the sum, before -> after: 62 -> 28 us at 2,048
+// particles (tiled), 36 -> 20 at 4,096, 158 -> 104 at 16,384 (symmetric), 361 -> 256
+// at 32,768, 1,089 -> 918 at 65,752, 3,343 -> 3,078 at 131,072; the density pass
+// takes 7 to 13 us more.  Error against FP64 (relative RMS): 2.8e-7 -> 2.6e-7 at
+// 2,048, 8.7e-8 -> 6.1e-8 at 16,384, 4.9e-8 -> 4.1e-8 at 262,144.
+__device__ __forceinline__ float sphx_clamped_r3(float r2, float t) {
+    const float ri = __builtin_amdgcn_rsqf(fmaxf(r2, t * t));
+    return (ri * ri) * ri;
+}
+__device__ __forceinline__ float sphx_soft_factor(float r2, float t) {
+    return sphx_spline_f(r2, t) - sphx_clamped_r3(r2, t);
+}
+
 __device__ __forceinline__ double wave_max_d(double v) {
     for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
     return v;
@@ -455,7 +499,8 @@ struct Engine {
     int build_boxes(hipStream_t st, bool with_h);
     int smoothing(hipStream_t st, bool predictor);
     int build_candidates(hipStream_t st);
-    int density_eos(hipStream_t st, bool lists = false);
+    // soft: also the softened pairs' gravity sums into s.gx..gz (eps = h)
+    int density_eos(hipStream_t st, bool lists = false, bool soft = false);
     // groups per bucket of the smoothing and list walks (1, 2 or 4)
     int smooth_parts() const;
     int list_parts() const;
@@ -520,7 +565,7 @@ void sphx_bh_host_free(BhHost *h);
 int sphx_bh_run(Engine &E, BhHost &H, double theta, bool with_pot, hipStream_t st, BhStats *out);
 
 // launchers implemented in the .hip files
-int sphx_gravity_run(Engine &E, const GravConfig &cfg, bool with_pot, hipStream_t st);
+int sphx_gravity_run(Engine &E, const GravConfig &cfg, bool with_pot, bool soft, hipStream_t st);
 int sphx_gravity_prepare(Engine &E, const GravConfig &cfg, hipStream_t st);
 int sphx_launch_morton(Engine &E, hipStream_t st);
 int sphx_sort_keys(uint64_t *keys, int32_t *vals, uint64_t *keys_tmp, int32_t *vals_tmp, int64_t n,
