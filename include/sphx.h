@@ -394,8 +394,9 @@ int sphx_plan_destroy(sphx_plan *plan);
 
 /* Gravity launch shape of a plan or context: ipl particles per lane (1, 2, 4),
  * j-tile tj (256, 512, 1024), j split js >= 1 (more workgroups for small N);
- * or ipl = 8, the symmetric sum: (8, 512, S) with S block pairs per wave, or
- * (8, 256, 1) / (8, 128, 1) with each block pair split into parts of tj j.
+ * or ipl = 8, the symmetric sum: (8, 512, S) with S block pairs per workgroup
+ * of four waves, each wave a quarter of every block pair ((8, 256, 1) and
+ * (8, 128, 1) are accepted and mean (8, 512, 1)).
  * No reference counterpart: the reference launches acc_g with a fixed
  * <<<ceil(N/256), 256>>> (DRV2:280-281); the autotuner sets this. */
 int sphx_plan_set_gravity_config(sphx_plan *plan, int32_t ipl, int32_t tj, int32_t js);
@@ -519,7 +520,7 @@ int sphx_batch_runs(sphx_batch *b, int64_t *ids, int64_t *sizes, int64_t *steps,
 int sphx_batch_set_cooling_grid(sphx_batch *b, const sphx_cool_grid *grid);
 /* Gravity of the batch's runs from the symmetric direct sum (each pair
  * evaluated once for both particles; block_pairs = 512-particle block pairs
- * per wavefront) instead of the fixed tiled shape.  Its partial sums total
+ * per workgroup) instead of the fixed tiled shape.  Its partial sums total
  * sphx_gravity_symmetric_bytes(n, block_pairs) per run of n particles (about
  * 12 n^2 / 1024 bytes); budget_bytes of device memory are reserved here and
  * the triangle of 512-particle block pairs is summed in bands of rows whose

@@ -1,10 +1,9 @@
 """Launch-shape selection for the gravity kernel.
 
 choose_gravity_config(n) returns (ipl, tj, js): particles per lane, j-tile
-size and j split of the tiled sum, or (8, 512, block pairs per wave) for the
-symmetric sum, or (8, tj, 1) for the symmetric sum with every block pair split
-into parts of tj j particles (tj = 256 or 128: more, shorter waves).  The defaults below keep >= 4 workgroups per CU on the
-256-CU MI355X; ``tune_gravity`` measures the candidates on the device and
+size and j split of the tiled sum, or (8, 512, block pairs per workgroup of four
+waves) for the symmetric sum.  The defaults below keep >= 4 workgroups per CU
+on the 256-CU MI355X; ``tune_gravity`` measures the candidates on the device and
 caches the winner per size class in a JSON file.
 """
 from __future__ import annotations
@@ -15,12 +14,10 @@ import time
 
 CUS = 256
 CANDIDATES = [(1, 256), (1, 512), (2, 256), (2, 512), (2, 1024), (4, 256), (4, 512)]
-# Symmetric sum (ipl 8, blocks of 512): js = block pairs per wave.  Its
+# Symmetric sum (ipl 8, blocks of 512): js = block pairs per workgroup.  Its
 # partial sums (12 B x n^2 / 1024 in all) are summed in row bands of bounded
 # memory, so it is offered at every size the tuner sweeps (up to 8M).
 SYM_SEGMENTS = (1, 2, 4, 8, 16, 32, 64)
-# ... and block pairs split into parts of tj j particles (one part per wave)
-SYM_SPLITS = (256, 128)
 SYM_MAX_N = 1 << 23
 _CACHE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gravity_tuning.json")
 
@@ -139,8 +136,6 @@ def _sweep(libsx, e, n: int, reps: int, res: dict):
     if n <= SYM_MAX_N:
         for S in SYM_SEGMENTS:
             timed((8, 512, S))
-        for tj in SYM_SPLITS:
-            timed((8, tj, 1))
 
 
 def tune_gravity(n: int, seed: int = 0, reps: int = 2, write: bool = True):

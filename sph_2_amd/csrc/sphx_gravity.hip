@@ -378,22 +378,26 @@ int launch_grav(const GravTabs &gt, const GravIO &io, int nblocks, bool pot, boo
 // ---------------------------------------------------------------------------
 // Symmetric direct sum (configuration ipl = 8).  Each pair is evaluated once
 // and applied to both particles (Newton's third law).  The run's particles
-// form blocks of SYM_B; a wave holds one block as its i-set (8 per lane) and
-// walks a segment of the upper triangle of block pairs (row I, blocks
-// J0..J1-1 >= I).  Per 128-particle chunk of block J, two sets of 64 j
+// form blocks of SYM_B; a workgroup of SYM_W waves walks a segment of the upper
+// triangle of block pairs (row I, blocks J0..J1-1 >= I), each wave with block I
+// as its i-set (8 per lane) and its own 128-particle chunk of every block J.
+// Per chunk, two sets of 64 j
 // particles sit one per lane and rotate one lane per step (ds_bpermute, on the
 // LDS pipe) together with their own force accumulators, so after 64 steps
 // every (i, j) pair of the chunk has been met once and each j is back in its
 // lane with its sum over the 512 i.  The j-side sums of row I go to their own
 // slots of a partial buffer and the i-side sums of each segment to theirs;
 // k_grav_sym_reduce adds them in a fixed order, so results do not depend on
-// scheduling.  With tj < SYM_B a segment is a part of one block pair (its
-// j particles [c0, c0 + tj)), so that mid-size runs launch several waves per
-// block pair.  The diagonal block pair (J = I) is summed one-sided.  Far block
+// scheduling.  One wave a segment left a launch of a mid-size run waiting for
+// its last waves (a whole block pair takes one wave alone 175 us) and needed
+// segments split into parts, each with i-side partials of its own; four waves
+// share a segment's partials.
+// The diagonal block pair (J = I) is summed one-sided.  Far block
 // pairs whose blocks each have one common mass use no mass in the pair and
 // scale the chunk sums (rsq + 14 VALU per pair for two interactions).
 // ---------------------------------------------------------------------------
 constexpr int SYM_B = 512;
+constexpr int SYM_W = SYM_B / 128;  // waves of a segment's workgroup
 
 struct SymTabs {
     const int32_t *b_beg, *b_cnt;  // blocks (SYM_B particles; a run's last block partial)
@@ -415,9 +419,6 @@ struct SymTabs {
     const int32_t *r_pbeg;         // first particle of each run
     int64_t n;
     const int32_t *order;          // launch order: group g takes segment order[seg0 + g] (global)
-    const int32_t *seg_c0;         // per segment: first j of each of its blocks (0, or a
-                                   // multiple of jspan when a block pair is split)
-    int32_t jspan;                 // j particles a segment takes of each block (SYM_B, 256, 128)
 };
 
 // The segment a group takes.  Groups start roughly in index order and the
@@ -594,6 +595,33 @@ __device__ __forceinline__ void sym_chunk_fold(SymI &S, SymJ &A, SymJ &B, int ad
     B.fx = bx; B.fy = by; B.fz = bz;
 }
 
+// The segment's i-side sums, P per lane and wave from block particle 64 p0 + on,
+// added over its waves in wave order and stored in (or added to) its slots.
+template <int P>
+__device__ __forceinline__ void sym_store_i(const KahanF *kx, const KahanF *ky, const KahanF *kz, int p0,
+                                            int cnt, int64_t o, double *qx, double *qy, double *qz,
+                                            bool add) {
+    __shared__ double red[SYM_W][64 * P];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    for (int a = 0; a < 3; ++a) {
+        const KahanF *k = a == 0 ? kx : (a == 1 ? ky : kz);
+        double *q = a == 0 ? qx : (a == 1 ? qy : qz);
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < P; ++p) red[w][lane + 64 * p] = k[p].value();
+        __syncthreads();
+        for (int l = threadIdx.x; l < 64 * P; l += 64 * SYM_W) {
+            const int li = 64 * p0 + l;
+            if (li < cnt) {
+                double v = red[0][l];
+#pragma unroll
+                for (int u = 1; u < SYM_W; ++u) v += red[u][l];
+                q[o + li] = add ? q[o + li] + v : v;
+            }
+        }
+    }
+}
+
 // Block-pair mode of tile J for row I (wave-uniform): 3 diagonal, 2 near
 // (spline path), 0 far with common masses on both sides, 1 far.
 __device__ __forceinline__ int sym_mode(const double *bI, const double *bJ, bool diag) {
@@ -616,7 +644,7 @@ __device__ __forceinline__ void sym_segment_far(const SymTabs &T, const double *
                                                 const double *__restrict__ z,
                                                 const double *__restrict__ m,
                                                 const double *__restrict__ eps, bool add) {
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, c = 128 * (threadIdx.x >> 6);
     const int sg = sym_seg(T);
     const int I = T.seg_i[sg], J0 = T.seg_j0[sg], J1 = T.seg_j1[sg];
     const int beg = T.b_beg[I], cnt = T.b_cnt[I];
@@ -645,7 +673,6 @@ __device__ __forceinline__ void sym_segment_far(const SymTabs &T, const double *
     }
     const int64_t roff = T.row_off[I] - T.p_base;
     const int rj0 = T.row_j0[I];
-    const int c0 = T.seg_c0[sg];
 
     for (int J = J0; J < J1; ++J) {
         const int jb = T.b_beg[J], jc = T.b_cnt[J];
@@ -658,8 +685,7 @@ __device__ __forceinline__ void sym_segment_far(const SymTabs &T, const double *
         const bool common = mode == 0 || mode == 5 || mode == 7;
         const float si = common ? (float)bJ[7] : 1.0f;  // i-side scale: the j block's mass
         const float sj = common ? (float)mI : 1.0f;     // j-side scale: the i block's mass
-        const int ce = jc < c0 + T.jspan ? jc : c0 + T.jspan;
-        for (int c = c0; c < ce; c += 128) {
+        if (c < jc) {
             SymJ A = sym_load(x, y, z, m, eps, jb, jc, c + lane, ox, oy, oz);
             SymJ B = sym_load(x, y, z, m, eps, jb, jc, c + 64 + lane, ox, oy, oz);
             if (mode == 0) sym_chunk<0>(S, A, B, addr);
@@ -686,22 +712,7 @@ __device__ __forceinline__ void sym_segment_far(const SymTabs &T, const double *
             }
         }
     }
-#pragma unroll
-    for (int p = 0; p < 8; ++p) {
-        int li = lane + 64 * p;
-        if (li < cnt) {
-            int64_t o = (int64_t)(T.seg0 + sg - T.q_seg0) * SYM_B + li;
-            if (add) {
-                T.qx[o] += kx[p].value();
-                T.qy[o] += ky[p].value();
-                T.qz[o] += kz[p].value();
-            } else {
-                T.qx[o] = kx[p].value();
-                T.qy[o] = ky[p].value();
-                T.qz[o] = kz[p].value();
-            }
-        }
-    }
+    sym_store_i<8>(kx, ky, kz, 0, cnt, (int64_t)(T.seg0 + sg - T.q_seg0) * SYM_B, T.qx, T.qy, T.qz, add);
 }
 
 // The same segment restricted to its near and diagonal block pairs.  The
@@ -718,7 +729,7 @@ __device__ __forceinline__ bool sym_segment_near(const SymTabs &T, const double 
                                                  const double *__restrict__ z,
                                                  const double *__restrict__ m,
                                                  const double *__restrict__ eps) {
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63, c = 128 * (threadIdx.x >> 6);
     const int sg = sym_seg(T);
     const int I = T.seg_i[sg], J0 = T.seg_j0[sg], J1 = T.seg_j1[sg];
     const int beg = T.b_beg[I], cnt = T.b_cnt[I];
@@ -733,8 +744,8 @@ __device__ __forceinline__ bool sym_segment_near(const SymTabs &T, const double 
     const int addr = ((lane + 1) & 63) << 2;  // lane L takes the value of lane L + 1
     const int64_t roff = T.row_off[I] - T.p_base;
     const int rj0 = T.row_j0[I];
-    const int c0 = T.seg_c0[sg];
-    __shared__ float slotbox[4][7];
+    __shared__ float slotboxes[SYM_W][4][7];
+    float(*slotbox)[7] = slotboxes[threadIdx.x >> 6];  // each wave its own copy
 
     for (int h = 0; 256 * h < cnt; ++h) {
         SymIP<4> S;
@@ -764,7 +775,7 @@ __device__ __forceinline__ bool sym_segment_near(const SymTabs &T, const double 
                           wave_max_f(ok ? S.e[p] : 0.0f)};
             if (lane < 7) slotbox[p][lane] = v[lane];
         }
-        __syncthreads();
+        __builtin_amdgcn_wave_barrier();
 
         for (int J = J0; J < J1; ++J) {
             const int jb = T.b_beg[J], jc = T.b_cnt[J];
@@ -772,8 +783,7 @@ __device__ __forceinline__ bool sym_segment_near(const SymTabs &T, const double 
             if (!actI && !T.act[J]) continue;
             const int mode = sym_mode(bI, bJ, J == I);
             if (mode <= 1) continue;
-            const int ce = jc < c0 + T.jspan ? jc : c0 + T.jspan;
-            for (int c = c0; c < ce; c += 128) {
+            if (c < jc) {
                 SymJ A = sym_load(x, y, z, m, eps, jb, jc, c + lane, ox, oy, oz);
                 SymJ B = sym_load(x, y, z, m, eps, jb, jc, c + 64 + lane, ox, oy, oz);
                 int cm = mode;
@@ -842,29 +852,22 @@ __device__ __forceinline__ bool sym_segment_near(const SymTabs &T, const double 
                 }
             }
         }
-#pragma unroll
-        for (int p = 0; p < 4; ++p) {
-            int li = lane + 64 * (4 * h + p);
-            if (li < cnt) {
-                int64_t o = (int64_t)(T.seg0 + sg - T.q_seg0) * SYM_B + li;
-                T.qx[o] = kx[p].value();
-                T.qy[o] = ky[p].value();
-                T.qz[o] = kz[p].value();
-            }
-        }
+        sym_store_i<4>(kx, ky, kz, 4 * h, cnt, (int64_t)(T.seg0 + sg - T.q_seg0) * SYM_B, T.qx, T.qy, T.qz,
+                       false);
     }
     return true;
 }
 
-// One wave per segment: its near block pairs, then its far ones (three waves
-// per SIMD: both paths fit 168 VGPRs without spills).  Near work, a few
+// One workgroup per segment: its near block pairs, then its far ones (three
+// waves per SIMD: both paths fit 168 VGPRs, two values spilled across the
+// block-pair loop).  Near work, a few
 // percent of the pairs at 1M particles but a third at 65K, is spread over the
 // same launch as the far work instead of trailing it.
 // SOFT: the softened pairs' sums come from the density pass, so that a near
 // block pair costs four instructions a pair more than a far one instead of the
 // spline's divergent branches, and both run in one pass over the segment.
 template <bool SOFT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_grav_sym(
+__global__ __launch_bounds__(64 * SYM_W) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_grav_sym(
     SymTabs T, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, const double *__restrict__ eps) {
     const bool near = SOFT ? false : sym_segment_near(T, x, y, z, m, eps);
@@ -979,7 +982,6 @@ __global__ __launch_bounds__(256) void k_pair_probe(float *out, int iters, float
 // length change.
 struct SymHost {
     int seg_len = 0;
-    int seg_tj = 0;                 // j particles per segment and block (SYM_B: whole blocks)
     std::vector<int64_t> sizes;
     int nblocks = 0, nseg = 0;
     std::vector<int32_t> run_seg0;  // first segment of each run (+ total)
@@ -1005,7 +1007,7 @@ struct SymHost {
     };
     std::vector<Band> bands;
     int o_bbeg = 0, o_bcnt = 0, o_runb0 = 0, o_si = 0, o_sj0 = 0, o_sj1 = 0, o_rj0 = 0, o_rns = 0,
-        o_rs0 = 0, o_ord = 0, o_c0 = 0;
+        o_rs0 = 0, o_ord = 0;
 };
 
 void sphx_sym_host_free(SymHost *h) { delete h; }
@@ -1065,11 +1067,8 @@ static int sym_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
     if (!E.grav.sym) E.grav.sym = new SymHost();
     SymHost &H = *E.grav.sym;
     const int S = cfg.js;
-    // tj < SYM_B (with one block pair per segment) splits every block pair
-    // into SYM_B / tj segments of tj j particles each: more, shorter waves
-    const int span = cfg.tj < SYM_B ? cfg.tj : SYM_B;
-    if (H.seg_len == S && H.seg_tj == span && H.sizes == E.run_n) return SPHX_OK;
-    std::vector<int32_t> bbeg, bcnt, runb0, si, sj0, sj1, sc0, rj0, rns, rs0;
+    if (H.seg_len == S && H.sizes == E.run_n) return SPHX_OK;
+    std::vector<int32_t> bbeg, bcnt, runb0, si, sj0, sj1, rj0, rns, rs0;
     std::vector<int64_t> roff;
     std::vector<int32_t> run_seg0;
     int64_t off = 0, plen = 0;
@@ -1090,13 +1089,10 @@ static int sym_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
             plen += (off + nr) - j0;
             rs0.push_back((int32_t)si.size());
             int k = 0;
-            for (int J = I; J < b1; J += S) {
-                for (int c = 0; c < bcnt[J]; c += span, ++k) {
-                    si.push_back(I);
-                    sj0.push_back(J);
-                    sj1.push_back(std::min(b1, J + S));
-                    sc0.push_back(c);
-                }
+            for (int J = I; J < b1; J += S, ++k) {
+                si.push_back(I);
+                sj0.push_back(J);
+                sj1.push_back(std::min(b1, J + S));
             }
             rns.push_back(k);
         }
@@ -1136,8 +1132,7 @@ static int sym_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
     int64_t need_p = 3 * max_slots, need_q = 3 * (int64_t)SYM_B * max_segs;
     // launch order (sym_seg): within each run's part of each band, segments
     // by their distance from the diagonal, nearest first: the k-th segment of
-    // every row of the part (first block pair J0 = I + k S; with split block
-    // pairs, part k mod (SYM_B / tj) of block I + k / (SYM_B / tj)), for k = 0, 1, ...,
+    // every row of the part (first block pair J0 = I + k S), for k = 0, 1, ...,
     // rows in order.  The rows of a part are consecutive and their segments
     // contiguous, so this is a permutation of the part's range, built in one
     // pass (the tables are rebuilt whenever the run set changes).
@@ -1165,7 +1160,7 @@ static int sym_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
     };
     int o_bbeg = put(bbeg), o_bcnt = put(bcnt), o_runb0 = put(runb0), o_si = put(si),
         o_sj0 = put(sj0), o_sj1 = put(sj1), o_rj0 = put(rj0), o_rns = put(rns), o_rs0 = put(rs0),
-        o_ord = put(ord), o_c0 = put(sc0);
+        o_ord = put(ord);
     if ((int64_t)all.size() > H.dev_i_cap) {
         SPHX_CHECK(E.alloc((void **)&H.dev_i, sizeof(int32_t) * (all.size() + 1024)));
         H.dev_i_cap = (int64_t)all.size() + 1024;
@@ -1198,10 +1193,8 @@ static int sym_prepare(Engine &E, const GravConfig &cfg, hipStream_t st) {
     SPHX_HIP(hipStreamSynchronize(st));
     H.o_bbeg = o_bbeg; H.o_bcnt = o_bcnt; H.o_runb0 = o_runb0; H.o_si = o_si; H.o_sj0 = o_sj0;
     H.o_sj1 = o_sj1; H.o_rj0 = o_rj0; H.o_rns = o_rns; H.o_rs0 = o_rs0; H.o_ord = o_ord;
-    H.o_c0 = o_c0;
     H.run_seg0 = run_seg0;
     H.seg_len = S;
-    H.seg_tj = span;
     H.sizes = E.run_n;
     H.nblocks = nb;
     H.nseg = ns;
@@ -1249,12 +1242,11 @@ static int sym_run(Engine &E, bool soft, hipStream_t st) {
         SymTabs T{d + H.o_bbeg, d + H.o_bcnt, d + H.o_runb0, d + H.o_si + a, d + H.o_sj0 + a,
                   d + H.o_sj1 + a, H.row_off, d + H.o_rj0, d + H.o_rns, d + H.o_rs0, H.bbox,
                   part, part + pl, part + 2 * pl, q, q + ql, q + 2 * ql, a, bd.seg_lo, bd.p_base,
-                  blk ? H.act : nullptr, E.s.run, E.t.r_pbeg, E.n, d + H.o_ord, d + H.o_c0 + a,
-                  H.seg_tj};
+                  blk ? H.act : nullptr, E.s.run, E.t.r_pbeg, E.n, d + H.o_ord};
         if (!marked) SPHX_CHECK(E.tmark(st, PH_GRAVK, 0));
         marked = true;
-        if (soft) k_grav_sym<true><<<(unsigned)(b - a), 64, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
-        else k_grav_sym<false><<<(unsigned)(b - a), 64, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
+        if (soft) k_grav_sym<true><<<(unsigned)(b - a), 64 * SYM_W, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
+        else k_grav_sym<false><<<(unsigned)(b - a), 64 * SYM_W, 0, st>>>(T, E.s.x, E.s.y, E.s.z, E.s.m, eps);
         SPHX_HIP(hipGetLastError());
         if (--left == 0) SPHX_CHECK(E.tmark(st, PH_GRAVK, 1));
         k_grav_sym_reduce<<<pg, 256, 0, st>>>(T, E.p.G, p0, p1, bd.row_lo, bd.row_hi, E.s.gx,

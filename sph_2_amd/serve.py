@@ -239,7 +239,7 @@ class Server:
 
     def __init__(self, hbm_budget_bytes: int, max_runs: int = 512, graph: bool = True,
                  cooling: CoolingTable | None = None, symmetric: tuple | None = (4, 0.1)):
-        """symmetric: (block pairs per wave, share of the budget reserved for
+        """symmetric: (block pairs per workgroup, share of the budget reserved for
         the symmetric gravity sum's partials, which it streams in row bands),
         or None for the tiled sum."""
         share = symmetric[1] if symmetric else 0.0
