@@ -1040,20 +1040,30 @@ __device__ __forceinline__ PairGeom pair_geom(double dx, double dy, double dz, d
 // the same instructions (the list passes are then bit-identical to the walks).
 // Their fused multiply-adds are written out: left to the compiler, which
 // products it fuses depends on the loop around them.
-__device__ __forceinline__ void divcurl_pair(double vxi, double vyi, double vzi, double vxj,
-                                             double vyj, double vzj, float mj, double dx,
-                                             double dy, double dz, double r2, double tt,
-                                             KahanF &kd, KahanF &kx, KahanF &ky, KahanF &kz) {
+struct Terms4 {
+    float a, b, c, d;
+};
+__device__ __forceinline__ Terms4 divcurl_terms(double vxi, double vyi, double vzi, double vxj,
+                                                double vyj, double vzj, float mj,
+                                                const PairGeom &g) {
 #pragma clang fp contract(off)
-    PairGeom g = pair_geom(dx, dy, dz, r2, tt);
     float h5 = g.hinv * g.hinv;
     h5 = h5 * h5 * g.hinv;
     float F = SPHX_SIGMA_F * h5 * f_shape(g.q) * mj;
     float vx = (float)(vxi - vxj), vy = (float)(vyi - vyj), vz = (float)(vzi - vzj);
-    kd.add(F * __builtin_fmaf(vz, g.dz, __builtin_fmaf(vx, g.dx, vy * g.dy)));
-    kx.add(F * __builtin_fmaf(vy, g.dz, -(vz * g.dy)));
-    ky.add(F * __builtin_fmaf(vz, g.dx, -(vx * g.dz)));
-    kz.add(F * __builtin_fmaf(vx, g.dy, -(vy * g.dx)));
+    return {F * __builtin_fmaf(vz, g.dz, __builtin_fmaf(vx, g.dx, vy * g.dy)),
+            F * __builtin_fmaf(vy, g.dz, -(vz * g.dy)), F * __builtin_fmaf(vz, g.dx, -(vx * g.dz)),
+            F * __builtin_fmaf(vx, g.dy, -(vy * g.dx))};
+}
+__device__ __forceinline__ void divcurl_pair(double vxi, double vyi, double vzi, double vxj,
+                                             double vyj, double vzj, float mj, double dx,
+                                             double dy, double dz, double r2, double tt,
+                                             KahanF &kd, KahanF &kx, KahanF &ky, KahanF &kz) {
+    const Terms4 t = divcurl_terms(vxi, vyi, vzi, vxj, vyj, vzj, mj, pair_geom(dx, dy, dz, r2, tt));
+    kd.add(t.a);
+    kx.add(t.b);
+    ky.add(t.c);
+    kz.add(t.d);
 }
 
 struct HydroArgs {
@@ -1067,13 +1077,10 @@ struct HydroI {
     float rho, pr, c, f;  // rho, P / rho^2, sound speed, Balsara factor
 };
 
-__device__ __forceinline__ void hydro_pair(const HydroArgs &a, const HydroI &I, double vxj,
-                                           double vyj, double vzj, float mj, float rhoj,
-                                           float prj, float cj, float fj, double dx, double dy,
-                                           double dz, double r2, double tt, KahanF &kx,
-                                           KahanF &ky, KahanF &kz, KahanF &kdu) {
+__device__ __forceinline__ Terms4 hydro_terms(const HydroArgs &a, const HydroI &I, double vxj,
+                                              double vyj, double vzj, float mj, float rhoj, float prj,
+                                              float cj, float fj, double tt, const PairGeom &g) {
 #pragma clang fp contract(off)
-    PairGeom g = pair_geom(dx, dy, dz, r2, tt);
     float h5 = g.hinv * g.hinv;
     h5 = h5 * h5 * g.hinv;
     float F = SPHX_SIGMA_F * h5 * f_shape(g.q);
@@ -1094,10 +1101,19 @@ __device__ __forceinline__ void hydro_pair(const HydroArgs &a, const HydroI &I, 
     }
     float mF = mj * F;
     float sc_ = mF * (I.pr + prj + pij);
-    kx.add(-sc_ * g.dx);
-    ky.add(-sc_ * g.dy);
-    kz.add(-sc_ * g.dz);
-    kdu.add(mF * __builtin_fmaf(0.5f, pij, I.pr) * vr);
+    return {-sc_ * g.dx, -sc_ * g.dy, -sc_ * g.dz, mF * __builtin_fmaf(0.5f, pij, I.pr) * vr};
+}
+__device__ __forceinline__ void hydro_pair(const HydroArgs &a, const HydroI &I, double vxj,
+                                           double vyj, double vzj, float mj, float rhoj,
+                                           float prj, float cj, float fj, double dx, double dy,
+                                           double dz, double r2, double tt, KahanF &kx,
+                                           KahanF &ky, KahanF &kz, KahanF &kdu) {
+    const Terms4 t = hydro_terms(a, I, vxj, vyj, vzj, mj, rhoj, prj, cj, fj, tt,
+                                 pair_geom(dx, dy, dz, r2, tt));
+    kx.add(t.a);
+    ky.add(t.b);
+    kz.add(t.c);
+    kdu.add(t.d);
 }
 
 __device__ __forceinline__ double balsara_f(double dv, double cv, double c, double h) {
@@ -1172,10 +1188,13 @@ __device__ __forceinline__ float density_term(float mj, double dx, double dy, do
 struct SoftSum {
     KahanF x, y, z;
     __device__ __forceinline__ void init() { x.init(); y.init(); z.init(); }
+    static __device__ __forceinline__ float factor(float mj, double r2, double hi, double hj) {
+        return -mj * sphx_soft_factor((float)r2, (float)hi + (float)hj);
+    }
     __device__ __forceinline__ void add(float mj, double dx, double dy, double dz, double r2, double hi,
                                         double hj) {
 #pragma clang fp contract(off)
-        const float s = -mj * sphx_soft_factor((float)r2, (float)hi + (float)hj);
+        const float s = factor(mj, r2, hi, hj);
         x.add(s * (float)dx);
         y.add(s * (float)dy);
         z.add(s * (float)dz);
@@ -1433,17 +1452,39 @@ __device__ __forceinline__ bool bucket_ovf(const int32_t *ovf, int64_t b) {
     return (o.x | o.y | o.z | o.w) != 0;
 }
 
-// Density and EOS over the lists: the eight gathers of a run of list entries
-// are issued together (the sums keep the list order, the walk's).  Bound: the
-// latency of the gathers (L2-served, 36 of a record's 80 bytes).
-template <bool SOFT>
-__global__ __launch_bounds__(64) void k_density_list(Tables t, Soa s, DensArgs a) {
-    const int b = t.boff + xcd_block(blockIdx.x, gridDim.x);
-    if (bucket_ovf(a.ovf, b)) return;  // the walk launch takes this bucket
-    const int lane = threadIdx.x;
-    const int cnt = t.b_cnt[b];
-    const int i = t.b_beg[b] + lane;
-    const bool ok = lane < cnt;
+// Value of v in lane U of this lane's quad.
+template <int U>
+__device__ __forceinline__ float quad_from(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), U * 0x55, 0xf, 0xf, true));
+}
+
+template <int U>
+__device__ __forceinline__ Terms4 quad_from(const Terms4 &t) {
+    return {quad_from<U>(t.a), quad_from<U>(t.b), quad_from<U>(t.c), quad_from<U>(t.d)};
+}
+
+// Density and EOS over the lists, four lanes a particle and 16 particles a
+// wave: a lane evaluates every fourth entry (eight entries a round, their
+// gathers of 36 of a record's 80 bytes issued together), and the terms are
+// added in list order from the quad's lanes, so that the sums are the walk's.
+// Bound: in small runs the chain of the one wave on a SIMD (a VALU instruction
+// every eight cycles or so), in large ones the latency and address rate of the
+// gathers, for which two loads in flight a lane leave 50 registers and eight
+// waves a SIMD.  Against one lane a particle with eight loads in flight (106
+// registers, four waves; with the softening sums up to 131,072): 39 -> 18 us at
+// 4,096 particles, 88 -> 75 at 65,752, 397 -> 344 at 1,048,576.
+template <bool SOFT, bool WALK>
+__global__ __launch_bounds__(64) void k_density_quad(Tables t, Soa s, DensArgs a) {
+    const int g = xcd_block(blockIdx.x, gridDim.x), b = t.boff + (g >> 2);
+    const int lane = threadIdx.x, tl = 16 * (g & 3) + (lane >> 2), u = lane & 3;
+    if (bucket_ovf(a.ovf, b)) {
+        if (!WALK || (g & 3)) return;
+        if (lane == 0 && a.counters) atomicAdd((unsigned long long *)&a.counters[CNT_NBR_OVF], 1ull);
+        density_bucket<SOFT>(t, s, a, b);
+        return;
+    }
+    const bool ok = tl < t.b_cnt[b];
+    const int i = t.b_beg[b] + tl;
     double xi = 0.0, yi = 0.0, zi = 0.0, hi = 0.0;
     int len = 0;
     if (ok) {
@@ -1458,43 +1499,47 @@ __global__ __launch_bounds__(64) void k_density_list(Tables t, Soa s, DensArgs a
     SoftSum soft;
     soft.init();
     for (int k0 = 0; k0 < maxlen; k0 += 8) {
-        int j[8];
-        {
-            int4 u = make_int4(0, 0, 0, 0), v = u;
-            if (k0 < len) {
-                const int4 *p = reinterpret_cast<const int4 *>(lp + nbr_slot(k0, lane));
-                u = p[0];
-                v = p[1];
-            }
-            j[0] = u.x; j[1] = u.y; j[2] = u.z; j[3] = u.w;
-            j[4] = v.x; j[5] = v.y; j[6] = v.z; j[7] = v.w;
-        }
-        double x[8], y[8], z[8], h[8];
-        float m[8];
+        float w[2] = {0.0f, 0.0f}, gx[2] = {0.0f, 0.0f}, gy[2] = {0.0f, 0.0f}, gz[2] = {0.0f, 0.0f};
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            x[k] = y[k] = z[k] = h[k] = 0.0;
-            m[k] = 0.0f;
-            if (k0 + k < len) {
-                const PairRec *q = a.rec + j[k];
-                const double2 u = reinterpret_cast<const double2 *>(q)[0];
-                const double2 v = reinterpret_cast<const double2 *>(q)[1];
-                x[k] = u.x; y[k] = u.y; z[k] = v.x; h[k] = v.y;
-                m[k] = q->m;
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (k0 + k < len) {
-                const double dx = xi - x[k], dy = yi - y[k], dz = zi - z[k];
+        for (int v = 0; v < 2; ++v) {
+            const int k = k0 + 4 * v + u;
+            if (k < len) {
+#pragma clang fp contract(off)
+                const PairRec *q = a.rec + lp[nbr_slot(k, tl)];
+                const double2 p0 = reinterpret_cast<const double2 *>(q)[0];
+                const double2 p1 = reinterpret_cast<const double2 *>(q)[1];
+                const float m = q->m;
+                const double dx = xi - p0.x, dy = yi - p0.y, dz = zi - p1.x;
                 const double r2 = sphx_r2(dx, dy, dz);
-                const double tt = hi + h[k];
-                acc.add(density_term(m[k], dx, dy, dz, r2, tt));
-                if (SOFT) soft.add(m[k], dx, dy, dz, r2, hi, h[k]);
+                w[v] = density_term(m, dx, dy, dz, r2, hi + p1.y);
+                if (SOFT) {
+                    const float f = SoftSum::factor(m, r2, hi, p1.y);
+                    gx[v] = f * (float)dx;
+                    gy[v] = f * (float)dy;
+                    gz[v] = f * (float)dz;
+                }
             }
+        }
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            auto add = [&](int k, float aw, float ax, float ay, float az) {
+                if (k < len) {
+                    acc.add(aw);
+                    if (SOFT) {
+                        soft.x.add(ax);
+                        soft.y.add(ay);
+                        soft.z.add(az);
+                    }
+                }
+            };
+            const int k = k0 + 4 * v;
+            add(k, quad_from<0>(w[v]), quad_from<0>(gx[v]), quad_from<0>(gy[v]), quad_from<0>(gz[v]));
+            add(k + 1, quad_from<1>(w[v]), quad_from<1>(gx[v]), quad_from<1>(gy[v]), quad_from<1>(gz[v]));
+            add(k + 2, quad_from<2>(w[v]), quad_from<2>(gx[v]), quad_from<2>(gy[v]), quad_from<2>(gz[v]));
+            add(k + 3, quad_from<3>(w[v]), quad_from<3>(gx[v]), quad_from<3>(gy[v]), quad_from<3>(gz[v]));
         }
     }
-    if (ok) {
+    if (ok && u == 0) {
         density_store(s, a, i, acc);
         if (SOFT) soft.store(s, i);
     }
@@ -1903,6 +1948,81 @@ __global__ __launch_bounds__(64) void k_dchydro_list(Tables t, Soa s, HydroArgs 
     dchydro_bucket(t, s, a, L, t.boff + xcd_block(blockIdx.x, gridDim.x));
 }
 
+// The same with four lanes a particle (see k_density_quad), the walks of an
+// overflowed bucket included.  37.5 -> 23 us at 4,096 particles, and the
+// overflow launch (4.5 us) gone.
+__global__ __launch_bounds__(64) void k_dchydro_quad(Tables t, Soa s, HydroArgs a, ListArgs L) {
+    const int g = xcd_block(blockIdx.x, gridDim.x), b = t.boff + (g >> 2);
+    const int lane = threadIdx.x, tl = 16 * (g & 3) + (lane >> 2), u = lane & 3;
+    if (bucket_ovf(L.ovf, b)) {
+        if (g & 3) return;
+        divcurl_bucket(t, s, b);
+        hydro_bucket(t, s, a, b, true);
+        return;
+    }
+    const bool ok = tl < t.b_cnt[b];
+    const int i = t.b_beg[b] + tl;
+    RecA me{};
+    HydroI I;
+    I.vx = I.vy = I.vz = 0.0;
+    I.rho = 1.0f; I.pr = 0.0f; I.c = 0.0f; I.f = 1.0f;
+    int len = 0;
+    if (ok) {
+        me = load_rec_a(L.rec, i);
+        uint4 e = load_rec_b(L.rec, i);
+        I.vx = me.vx; I.vy = me.vy; I.vz = me.vz;
+        I.rho = me.rho;
+        I.pr = __uint_as_float(e.x);
+        I.c = __uint_as_float(e.y);
+        len = (int)e.z;
+    }
+    const int maxlen = wave_max_i(len);
+    const int32_t *lp = L.lst + (int64_t)b * SPHX_NBR_MAX * 64;
+    KahanF kd, kx, ky, kz, hx, hy, hz, hdu;
+    kd.init(); kx.init(); ky.init(); kz.init();
+    hx.init(); hy.init(); hz.init(); hdu.init();
+    for (int k0 = 0; k0 < maxlen; k0 += 8) {
+        Terms4 d[2] = {}, h[2] = {};
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            const int k = k0 + 4 * v + u;
+            if (k < len) {
+                const int j = lp[nbr_slot(k, tl)];
+                const RecA o = load_rec_a(L.rec, j);
+                const uint4 e = load_rec_b(L.rec, j);
+                const double dx = me.x - o.x, dy = me.y - o.y, dz = me.z - o.z;
+                const double tt = me.h + o.h;
+                const PairGeom pg = pair_geom(dx, dy, dz, sphx_r2(dx, dy, dz), tt);
+                d[v] = divcurl_terms(me.vx, me.vy, me.vz, o.vx, o.vy, o.vz, o.m, pg);
+                h[v] = hydro_terms(a, I, o.vx, o.vy, o.vz, o.m, o.rho, __uint_as_float(e.x),
+                                   __uint_as_float(e.y), 1.0f, tt, pg);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 2; ++v) {
+            auto add = [&](int k, const Terms4 &p, const Terms4 &q) {
+                if (k < len) {
+                    kd.add(p.a); kx.add(p.b); ky.add(p.c); kz.add(p.d);
+                    hx.add(q.a); hy.add(q.b); hz.add(q.c); hdu.add(q.d);
+                }
+            };
+            const int k = k0 + 4 * v;
+            add(k, quad_from<0>(d[v]), quad_from<0>(h[v]));
+            add(k + 1, quad_from<1>(d[v]), quad_from<1>(h[v]));
+            add(k + 2, quad_from<2>(d[v]), quad_from<2>(h[v]));
+            add(k + 3, quad_from<3>(d[v]), quad_from<3>(h[v]));
+        }
+    }
+    const bool out = ok && u == 0;
+    divcurl_store(s, i, out, kd, kx, ky, kz);
+    if (out) {
+        s.ax[i] = s.gx[i] + hx.value();
+        s.ay[i] = s.gy[i] + hy.value();
+        s.az[i] = s.gz[i] + hz.value();
+        s.du[i] = hdu.value();
+    }
+}
+
 // The walk for the buckets whose lists overflowed: each wave scans 64 flags
 // at a time and walks the flagged buckets of its share.
 __global__ __launch_bounds__(64) void k_divcurl_ovf(Tables t, Soa s, const int32_t *ovf, int nb) {
@@ -2181,6 +2301,14 @@ int sphx_neighbor_pass(Engine &E, int64_t r0, int64_t r1, int32_t *counts, const
 // / 96 / 80 at 4,096, 277 / 164 / 155 at 65,752, 255 / 218 / 224 at 131,072,
 // 330 / 363 / 387 at 262,144.
 int Engine::smooth_parts() const { return nb_launch() <= 384 ? 4 : (nb_launch() <= 1536 ? 2 : 1); }
+// Small runs, whose passes are bounded by launches and by the chain of one
+// wave a SIMD: the list passes walk an overflowed bucket themselves (that costs
+// registers, and the launch it saves 4.5 us), and the div/curl and hydro pass
+// gives a particle four lanes.  One pass with four lanes against one with one
+// lane and its overflow launch: 24.6 against 41 us at 4,096 particles, 37.6
+// against 45 at 32,768, 45 against 44 at 46,341, 56 against 53 at 65,752, 639
+// against 521 at 1,048,576, where the gathers bound it.
+bool Engine::list_small() const { return nb_launch() <= 512; }
 int Engine::list_parts() const { return nb_launch() <= 1536 ? 4 : (nb_launch() <= 3072 ? 2 : 1); }
 
 int Engine::smoothing(hipStream_t st, bool predictor) {
@@ -2246,12 +2374,14 @@ int Engine::density_eos(hipStream_t st, bool lists, bool soft) {
     SPHX_CHECK(build_lists(st));
     DensArgs a{p.gamma, tmpi, counters, nbr, prec, nbr_ovf};
     const int nb = (int)nb_launch();
-    if (soft) {
-        k_density_list<true><<<nb, 64, 0, st>>>(tview(), s, a);
-        k_density_ovf<true><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+    if (list_small()) {
+        if (soft) k_density_quad<true, true><<<4 * nb, 64, 0, st>>>(tview(), s, a);
+        else k_density_quad<false, true><<<4 * nb, 64, 0, st>>>(tview(), s, a);
     } else {
-        k_density_list<false><<<nb, 64, 0, st>>>(tview(), s, a);
-        k_density_ovf<false><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+        if (soft) k_density_quad<true, false><<<4 * nb, 64, 0, st>>>(tview(), s, a);
+        else k_density_quad<false, false><<<4 * nb, 64, 0, st>>>(tview(), s, a);
+        if (soft) k_density_ovf<true><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+        else k_density_ovf<false><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
     }
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
@@ -2286,6 +2416,11 @@ int Engine::divcurl_hydro_lists(hipStream_t st) {
                 p.av_form, p.balsara};
     ListArgs L{nbr, prec, nbr_ovf, fbal};
     const int nb = (int)nb_launch();
+    if (list_small()) {
+        k_dchydro_quad<<<4 * nb, 64, 0, st>>>(tview(), s, a, L);
+        SPHX_HIP(hipGetLastError());
+        return SPHX_OK;
+    }
     k_dchydro_list<<<nb, 64, 0, st>>>(tview(), s, a, L);
     k_dchydro_ovf<<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nbr_ovf, nb);
     SPHX_HIP(hipGetLastError());

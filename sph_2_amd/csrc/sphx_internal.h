@@ -504,6 +504,7 @@ struct Engine {
     // groups per bucket of the smoothing and list walks (1, 2 or 4)
     int smooth_parts() const;
     int list_parts() const;
+    bool list_small() const;  // list passes that walk overflowed buckets themselves
     int build_lists(hipStream_t st);
     int fill_records(hipStream_t st);
     // allocate the lists if they are not; false (and no error) without the memory

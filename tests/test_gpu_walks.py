@@ -77,3 +77,35 @@ def test_lists_of_the_stateless_calls_overflow(gpu):
     acco, duo = oracle.hydro(e.pos, v, rho_o, P, c, h, e.m, dvo, cvo, oracle.Params(balsara=1))
     for a, b in ((dv, dvo), (cv, cvo), (acc, acco), (du, duo)):
         assert np.sqrt(((a - b) ** 2).sum() / (b ** 2).sum()) < 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 17, 63, 32768, 32769, 33001])
+def test_list_passes_equal_the_walks(gpu, n):
+    """The list passes on both sides of 512 buckets (four lanes a particle and
+    the overflowed buckets walked in the same launch; above it the walks in a
+    launch of their own), with partial buckets: the lists give the walks' bits,
+    with lists that overflow and without."""
+    from sph_2_amd.plan import SphPlan
+
+    for wide in (False, True):
+        e = ic.evrard(n, seed=23)
+        kw = {}
+        if wide:
+            e.h = np.where(e.pos[:, 0] > 0.3, 3.0 * e.h, e.h)
+            kw = dict(max_iter=1)
+        outs = []
+        for lists in (True, False):
+            pl = SphPlan(n, **kw)
+            pl.set_cell_level(0)
+            pl.set_neighbor_lists(lists)
+            pl.load(e.pos, e.vel, e.u, e.m, e.h)
+            pl.init()
+            pl.step(1, 1e-4)
+            outs.append(pl.state())
+            c = pl.counters()
+            pl.close()
+            if lists and n > 1000:
+                assert (c["buckets"] <= 512) == (n <= 32768), c
+                assert (c["nbr_overflow"] > 0) == wide, c
+        for f in outs[0]:
+            assert np.array_equal(outs[0][f], outs[1][f]), (f, wide)
