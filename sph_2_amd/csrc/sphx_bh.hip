@@ -26,23 +26,19 @@ constexpr int BH_LEAF = 8;        // particles per leaf at most
 // Cell stack and interaction list capacities per group (one wave).  A deep
 // walk (small opening angle) opens many cells per step, and the larger stack
 // keeps its batches of popped cells large; at larger angles the smaller
-// stack's occupancy wins.  The walk is bound by how many groups a CU holds
-// (LDS) and a SIMD holds (registers): a list of 128 entries and four entries
-// evaluated together give four to five waves per SIMD, where a list of 512
-// and batches of eight gave two to three (4M-particle Plummer sphere, theta
-// 0.3 / 0.5 / 0.7: 45 / 13.8 / 7.5 ms against 60 / 18.1 / 10.1 ms; theta 0.3
-// took 100 ms with the smaller stack).
+// stack's occupancy wins.  A list of 128 entries
+// and four entries evaluated together leave four waves a SIMD, which the pairs'
+// FP32 issue fills (five by spilling took as long); a list of 512 and batches
+// of eight left two to three (the walk as it was then, 4M-particle Plummer
+// sphere, theta 0.3 / 0.5 / 0.7: 60 / 18.1 / 10.1 ms against 45 / 13.8 / 7.5;
+// 100 ms at 0.3 with the smaller stack; now 32.5 / 11.2 / 6.3 ms).
 constexpr int BH_SCAP = 1024;
 constexpr int BH_SCAP_DEEP = 2048;
 constexpr double BH_DEEP_THETA = 0.35;  // the larger stack below this angle
 constexpr int BH_SLACK = 160;     // > 7 x 21 levels of pure depth-first growth
 constexpr int BH_ICAP = 128;
 constexpr int BH_BATCH = 4;       // list entries evaluated together
-// leaf particles a lane lists per round: one round fills the list at most
-constexpr int BH_ROUND = BH_ICAP / 64;
-static_assert(BH_ICAP >= 64 && BH_ICAP % 64 == 0,
-              "a batch of accepted cells (at most 64) must fit the list");
-static_assert(BH_ROUND < 8, "leaf particles per lane and round are scanned in three bits");
+static_assert(BH_ICAP == 128, "the near masks of a full list are two wave ballots");
 static_assert(BH_SCAP > BH_SLACK + 7 * 64, "a full batch must fit above the slack");
 static_assert(BH_SCAP_DEEP > BH_SCAP, "the deep-walk stack is the larger one");
 constexpr int BHT = 256;
@@ -268,16 +264,66 @@ __global__ void k_bh_moments(BhTree T, int32_t l0, int32_t l1, const uint64_t *_
 // when it has at most 64; runs of 64 inside an unsplittable leaf with more.
 // Each particle lands in exactly one group; the list order (atomic append)
 // does not affect any particle's result.
-__global__ void k_bh_groups(BhTree T, int32_t ncell, int32_t *__restrict__ gbeg,
-                            int32_t *__restrict__ gcnt, int32_t *__restrict__ counter) {
+// A group of a cell with many particles sees most of them as single entries:
+// outliers packed over the whole of a large cell, or one small child beside
+// full ones.  A wave alone needs some 130 cycles an entry, so such a group in
+// one wave outlasts all the others.  It goes to several waves, each of which
+// walks the tree and sums its part of the entries: one for every BH_PART
+// particles of the cell (of the cells that begin in a range of them) and
+// BH_OUT for what lies outside (every BH_OUT-th by the cell's first particle).
+// Walk at theta 0.5 over a Plummer sphere, one wave a group -> parts: 3.46 ->
+// 0.42 ms for 65,536 particles, 2.12 -> 1.52 for 524,288.  2,048 particles a
+// wave took 0.65 ms for 131,072, where 1,024 take 0.55 and 512 take 0.59; four
+// waves outside took 1.20 ms for 262,144, eight 0.99 and sixteen 0.86.
+constexpr int BH_PART = 1024, BH_PARTS_MAX = 256, BH_OUT = 16;
+
+// A small run has too few groups to fill the device: all its groups go to
+// several waves (every SHARE-th entry by the cell's first particle), at the
+// price of a tree walk for each.  Evrard sphere with 1 / 2 / 4 / 8 waves: 194 /
+// 126 / 86 / 75 us for 8,192 particles, 287 / 176 / 140 / 208 for 32,768, 338 /
+// 222 / 241 / 353 for 65,536, 385 / 379 / 408 / 671 for 131,072.
+static int bh_share(int64_t n) { return n <= 8192 ? 8 : n <= 32768 ? 4 : n <= 98304 ? 2 : 1; }
+
+struct BhGroups {
+    int32_t *beg, *cnt;  // groups of one wave
+    // items of the others, a wave each: {first particle, particles | items of
+    // the group << 8 in its first | share << 20 | shares - 1 << 24, lo, hi}; a
+    // wave sums the entries of its share in [lo, hi), or outside [hi, lo)
+    int4 *part;
+    int32_t *count;      // [0] groups of one wave, [1] items of the others, [2] the others
+    int share;
+};
+
+__device__ __forceinline__ void bh_add_group(const BhGroups &g, int beg, int cnt, int cell, int ccnt) {
+    const int parts = min(ccnt / BH_PART, BH_PARTS_MAX);
+    if (parts >= 2) {
+        const int all = parts + BH_OUT;
+        const int k = atomicAdd(&g.count[1], all);
+        atomicAdd(&g.count[2], 1);
+        for (int64_t p = 0; p < parts; ++p) {
+            const int lo = cell + (int)(ccnt * p / parts);
+            const int hi = cell + (int)(ccnt * (p + 1) / parts);
+            g.part[k + p] = make_int4(beg, cnt | (p ? 0 : all << 8), lo, hi);
+        }
+        for (int p = 0; p < BH_OUT; ++p)
+            g.part[k + parts + p] = make_int4(beg, cnt | p << 20 | (BH_OUT - 1) << 24, cell + ccnt, cell);
+    } else if (g.share > 1) {
+        const int k = atomicAdd(&g.count[1], g.share);
+        atomicAdd(&g.count[2], 1);
+        for (int p = 0; p < g.share; ++p)
+            g.part[k + p] = make_int4(beg, cnt | (p ? 0 : g.share << 8) | p << 20 | (g.share - 1) << 24, 0, INT32_MAX);
+    } else {
+        const int k = atomicAdd(&g.count[0], 1);
+        g.beg[k] = beg;
+        g.cnt[k] = cnt;
+    }
+}
+
+__global__ void k_bh_groups(BhTree T, int32_t ncell, BhGroups G) {
     int i = blockIdx.x * BHT + threadIdx.x;
     if (i >= ncell) return;
-    int c = T.cnt[i];
-    if (i == 0 && c <= 64) {
-        int g = atomicAdd(counter, 1);
-        gbeg[g] = T.beg[0];
-        gcnt[g] = c;
-    }
+    const int c = T.cnt[i], b = T.beg[i];
+    if (i == 0 && c <= 64) bh_add_group(G, b, c, b, c);
     if (c <= 64) return;
     if (T.child[i] >= 0) {
         // consecutive small children are packed into one group of at most 64
@@ -286,11 +332,7 @@ __global__ void k_bh_groups(BhTree T, int32_t ncell, int32_t *__restrict__ gbeg,
         for (int q = T.child[i]; q < T.child[i] + T.nchild[i]; ++q) {
             int cq = T.cnt[q];
             if (cq > 64 || pc + cq > 64) {
-                if (pc > 0) {
-                    int g = atomicAdd(counter, 1);
-                    gbeg[g] = pb;
-                    gcnt[g] = pc;
-                }
+                if (pc > 0) bh_add_group(G, pb, pc, b, c);
                 pb = -1;
                 pc = 0;
             }
@@ -299,42 +341,34 @@ __global__ void k_bh_groups(BhTree T, int32_t ncell, int32_t *__restrict__ gbeg,
                 pc += cq;
             }
         }
-        if (pc > 0) {
-            int g = atomicAdd(counter, 1);
-            gbeg[g] = pb;
-            gcnt[g] = pc;
-        }
+        if (pc > 0) bh_add_group(G, pb, pc, b, c);
     } else {
-        for (int o = 0; o < c; o += 64) {
-            int g = atomicAdd(counter, 1);
-            gbeg[g] = T.beg[i] + o;
-            gcnt[g] = min(64, c - o);
-        }
+        for (int o = 0; o < c; o += 64) bh_add_group(G, b + o, min(64, c - o), b, 0);
     }
 }
 
-// Exclusive prefix sum over the wave of v, 0 <= v < 2^BITS, called with every
-// lane active: bit b of the lanes' values is one ballot, and the lanes below
-// this one holding it count 2^b each (mbcnt).  Exact integer sums, with no
-// LDS round trip.
-template <int BITS>
-__device__ __forceinline__ int wave_excl_scan(int v, int *total) {
-    int pos = 0, tot = 0;
-#pragma unroll
-    for (int b = 0; b < BITS; ++b) {
-        const uint64_t m = __ballot((v >> b) & 1);
-        const int below = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-        pos += below << b;
-        tot += __popcll(m) << b;
-    }
-    *total = tot;
-    return pos;
+// Inclusive prefix sum over the wave, every lane active: within the rows of 16
+// lanes, then the rows' totals (row_shr 1, 2, 4, 8, row_bcast 15 and 31).
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t u) {
+    int v = (int)u;
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return (uint32_t)v;
+}
+__device__ __forceinline__ uint32_t wave_last(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 struct BhArgs {
     const double *x, *y, *z, *m, *eps;
-    const int32_t *gbeg, *gcnt;   // walk groups
+    const int32_t *gbeg, *gcnt;   // groups of one wave
+    const int4 *part;             // items of the others, npart of them: first in the grid
+    int32_t npart;
+    double4 *psum;                // their sums, 64 an item
     int64_t n;
     double G, theta;
     double *ax, *ay, *az, *pot;
@@ -399,6 +433,23 @@ __device__ __forceinline__ void bh_far(float dx, float dy, float dz, float r2, f
     if (POT) ph = __builtin_fmaf(mj, ri, ph);
 }
 
+// bh_eval without the potential and without a branch: the outer formula with w
+// = 2 - q clamped at zero is the Newtonian one from q = 2 on, so one choice
+// (q <= 1) is left.
+__device__ __forceinline__ void bh_soft(float dx, float dy, float dz, float r2, float t, float mj,
+                                        float &ax, float &ay, float &az) {
+    const float ri = __builtin_amdgcn_rsqf(fmaxf(r2, 1.17549435e-38f));
+    const float ie = 2.0f * __builtin_amdgcn_rcpf(t);
+    const float q = r2 * ri * ie, q2 = q * q;
+    const float in = ie * ie * ie * __builtin_fmaf(q2, __builtin_fmaf(0.5f, q, -1.2f), 4.0f / 3.0f);
+    const float w = fmaxf(2.0f - q, 0.0f), w2 = w * w;
+    const float out = ri * ri * ri * __builtin_fmaf(-w2 * w2, __builtin_fmaf(w2, 1.0f / 6.0f, __builtin_fmaf(-0.8f, w, 1.0f)), 1.0f);
+    const float s = mj * (q <= 1.0f ? in : out);
+    ax = __builtin_fmaf(s, dx, ax);
+    ay = __builtin_fmaf(s, dy, ay);
+    az = __builtin_fmaf(s, dz, az);
+}
+
 template <bool POT>
 __device__ __forceinline__ void bh_pair(float xi, float yi, float zi, float ei, float4 j, float ej,
                                         float &ax, float &ay, float &az, float &ph) {
@@ -407,15 +458,28 @@ __device__ __forceinline__ void bh_pair(float xi, float yi, float zi, float ei, 
     bh_eval<POT>(dx, dy, dz, r2, ei + ej, j.w, ax, ay, az, ph);
 }
 
-template <bool POT, int SCAP>
-__global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
-    __shared__ int32_t stk[SCAP];
-    __shared__ float4 il[BH_ICAP];
-    __shared__ float ie[BH_ICAP];
-    const int lane = threadIdx.x;
-    const int gn = a.gcnt[blockIdx.x];
-    const int64_t i = (int64_t)a.gbeg[blockIdx.x] + lane;
-    const bool ok = lane < gn;
+// Bound: FP32 issue of one wave's pairs (the walk's own instructions are a fifth
+// of it).  So a list's entries are first tested against the group's box, 64 at a
+// time, and four that no particle can see softened are taken without a test (13
+// instructions an entry for 17); softened ones without a branch (34 for some
+// 45); a group of at most 32 or 16 particles gives each two or four lanes; the
+// three counts of a batch are scanned in one word, and opened leaves listed 64
+// particles at a time.  VALU instructions a wave, before -> after: 72,000 ->
+// 51,000 on an Evrard sphere of 1,048,576 particles with eps = h, theta 0.5 (walk
+// 2.33 -> 1.94 ms), 99,900 -> 67,200 on a Plummer sphere of 524,288 (2.68 -> 2.12
+// ms, and 1.52 with the groups in parts and the long walks first).
+//
+// The walk of one group of gn particles, P lanes a particle (P W = 64): lane
+// (sub, p) sums every P-th entry of the list for particle p.  Of the accepted
+// cells and opened leaves it sums those whose first particle lies in [lo, hi).
+template <bool POT, int SCAP, int P>
+__device__ __forceinline__ void bh_walk_group(const BhTree &T, const BhArgs &a, int32_t *stk, float4 *il,
+                                              float *ie, int64_t g0, int gn, int lo, int hi,
+                                              int smask, int sval, double4 *psum) {
+    constexpr int W = 64 / P, STEP = BH_BATCH * P;
+    const int lane = threadIdx.x, sub = lane / W, pl = lane % W;
+    const int64_t i = g0 + pl;
+    const bool ok = pl < gn;
     double xd = ok ? a.x[i] : 0.0, yd = ok ? a.y[i] : 0.0, zd = ok ? a.z[i] : 0.0;
     double lx = wave_min_d(ok ? xd : INFINITY), hx = wave_max_d(ok ? xd : -INFINITY);
     double ly = wave_min_d(ok ? yd : INFINITY), hy = wave_max_d(ok ? yd : -INFINITY);
@@ -423,6 +487,13 @@ __global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
     const double ox = 0.5 * (lx + hx), oy = 0.5 * (ly + hy), oz = 0.5 * (lz + hz);
     const float xi = (float)(xd - ox), yi = (float)(yd - oy), zi = (float)(zd - oz);
     const float ei = ok ? (float)a.eps[i] : 1.0f;
+    // The group's box and largest softening as the pairs see them: an entry at
+    // r >= 2e of the box is at r >= 2e of every particle by the same FP32
+    // operations, each of which keeps order under rounding.
+    const float bx = (float)(lx - ox), cx = (float)(hx - ox);
+    const float by = (float)(ly - oy), cy = (float)(hy - oy);
+    const float bz = (float)(lz - oz), cz = (float)(hz - oz);
+    const float emax = wave_max_f(ok ? fabsf(ei) : 0.0f);
     float ax = 0.f, ay = 0.f, az = 0.f, ph = 0.f;
     KahanF kx, ky, kz, kp;
     kx.init(); ky.init(); kz.init(); kp.init();
@@ -433,41 +504,69 @@ __global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
     int sp = 1;
     __syncthreads();
 
+    // Ballot of the entries q0 + lane of the list that some particle may see softened.
+    auto near_mask = [&](int q0) -> uint64_t {
+        bool near = false;
+        if (q0 + lane < icnt) {
+            const float4 j = il[q0 + lane];
+            const float t = emax + fabsf(ie[q0 + lane]);
+            const float dx = fmaxf(0.0f, fmaxf(bx - j.x, j.x - cx));
+            const float dy = fmaxf(0.0f, fmaxf(by - j.y, j.y - cy));
+            const float dz = fmaxf(0.0f, fmaxf(bz - j.z, j.z - cz));
+            const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+            near = !(r2 >= t * t);
+        }
+        return __ballot(near);
+    };
     auto flush = [&]() {
         __syncthreads();
-        // entries BH_BATCH at a time, their LDS loads issued before the pairs are
-        // evaluated (in list order, as one at a time would)
-        int q = 0;
-        for (; q + BH_BATCH <= icnt; q += BH_BATCH) {
+        // entries STEP at a time, BH_BATCH a lane, their LDS loads issued before the
+        // pairs are evaluated
+        const int full = icnt - icnt % STEP;
+        uint64_t near = near_mask(0);
+        const uint64_t near1 = near_mask(64);
+        for (int q = 0; q < full; q += STEP) {
+            if (q == 64) near = near1;
             float4 j[BH_BATCH];
-            float e[BH_BATCH];
+            float dx[BH_BATCH], dy[BH_BATCH], dz[BH_BATCH], r2[BH_BATCH];
 #pragma unroll
-            for (int k = 0; k < BH_BATCH; ++k) { j[k] = il[q + k]; e[k] = ie[q + k]; }
-            float dx[BH_BATCH], dy[BH_BATCH], dz[BH_BATCH], r2[BH_BATCH], t[BH_BATCH];
-            bool far = true;
+            for (int k = 0; k < BH_BATCH; ++k) j[k] = il[q + k * P + sub];
 #pragma unroll
             for (int k = 0; k < BH_BATCH; ++k) {
                 dx[k] = j[k].x - xi;
                 dy[k] = j[k].y - yi;
                 dz[k] = j[k].z - zi;
                 r2[k] = __builtin_fmaf(dx[k], dx[k], __builtin_fmaf(dy[k], dy[k], dz[k] * dz[k]));
-                t[k] = ei + e[k];
-                far = far && r2[k] >= t[k] * t[k];
             }
-            // lanes past the group's end take part in the vote as far
-            if (__all(far || !ok)) {
+            bool far = true;
+            float t[BH_BATCH];
+            if (near & ((1ull << STEP) - 1)) {
+#pragma unroll
+                for (int k = 0; k < BH_BATCH; ++k) {
+                    t[k] = ei + ie[q + k * P + sub];
+                    far = far && r2[k] >= t[k] * t[k];
+                }
+                // lanes past the group's end take part in the vote as far
+                far = __all(far || !ok);
+            }
+            near >>= STEP;
+            if (far) {
 #pragma unroll
                 for (int k = 0; k < BH_BATCH; ++k) bh_far<POT>(dx[k], dy[k], dz[k], r2[k], j[k].w, ax, ay, az, ph);
             } else {
 #pragma unroll
-                for (int k = 0; k < BH_BATCH; ++k)
-                    bh_eval<POT>(dx[k], dy[k], dz[k], r2[k], t[k], j[k].w, ax, ay, az, ph);
+                for (int k = 0; k < BH_BATCH; ++k) {
+                    if (POT) bh_eval<POT>(dx[k], dy[k], dz[k], r2[k], t[k], j[k].w, ax, ay, az, ph);
+                    else bh_soft(dx[k], dy[k], dz[k], r2[k], t[k], j[k].w, ax, ay, az);
+                }
             }
         }
-        for (; q < icnt; ++q) bh_pair<POT>(xi, yi, zi, ei, il[q], ie[q], ax, ay, az, ph);
-        kx.add(ax); ky.add(ay); kz.add(az); kp.add(ph);
+        for (int q = full + sub; q < icnt; q += P) bh_pair<POT>(xi, yi, zi, ei, il[q], ie[q], ax, ay, az, ph);
+        kx.add(ax); ky.add(ay); kz.add(az);
+        if (POT) kp.add(ph);
         ax = ay = az = ph = 0.f;
         ninter += icnt;
+        maxfill = max(maxfill, icnt);
         icnt = 0;
         __syncthreads();
     };
@@ -477,7 +576,8 @@ __global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
     // at most 7 net entries, so popping at most (cap - slack - sp) / 7 keeps the
     // stack inside cap - slack; past that the walk is pure depth-first (one
     // cell per batch), whose growth is bounded by 7 x the tree depth (<= 147),
-    // inside the slack.
+    // inside the slack.  The particles of opened leaves, eight a cell at most,
+    // take the place of its children above them while they are listed.
     while (sp > 0) {
         int room = (SCAP - BH_SLACK - sp) / 7;
         int take = room < 1 ? 1 : (room < 64 ? room : 64);
@@ -486,11 +586,19 @@ __global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
         int node = lane < take ? stk[base + lane] : -1;
         sp = base;
         __syncthreads();
-        int act = 0, nent = 0, nfr = 0, lnk = 0;
+        // what a lane adds: an accepted cell, leaf particles or children,
+        // from lnk on; the three counts are scanned as fields of one word
+        uint32_t mine = 0;
+        int rem = 0, lnk = 0;
         BhMono mo{};
+        BhLink lk{};
         if (node >= 0) {
             mo = T.mono[node];
-            const BhLink lk = T.link[node];
+            lk = T.link[node];
+        }
+        const int end = lk.beg + lk.cnt;
+        if (node >= 0 && (lo < hi ? lk.beg < hi && end > lo : lk.beg < hi || end > lo)) {
+            const bool own = (lo < hi ? lk.beg >= lo : lk.beg < hi || lk.beg >= lo) && (lk.beg & smask) == sval;
             double dx = fmax(0.0, fmax(lx - mo.cx, mo.cx - hx));
             double dy = fmax(0.0, fmax(ly - mo.cy, mo.cy - hy));
             double dz = fmax(0.0, fmax(lz - mo.cz, mo.cz - hz));
@@ -498,70 +606,89 @@ __global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
             const double d2 = dx * dx + dy * dy + dz * dz;
             const double rhs = (double)lk.size + a.theta * (double)lk.delta;
             if (d2 * (a.theta * a.theta) > rhs * rhs) {
-                act = 1;
+                mine = own ? 1u : 0u;
             } else if (lk.child < 0) {
-                act = 2;
-                nent = lk.cnt;
+                rem = own ? lk.cnt : 0;
                 lnk = lk.beg;
+                mine = (uint32_t)min(rem, 8) << 8;
             } else {
-                act = 3;
-                nfr = lk.nchild;
                 lnk = lk.child;
+                mine = (uint32_t)lk.nchild << 20;
             }
         }
+        uint32_t incl = wave_incl_scan(mine);
+        uint32_t tot = wave_last(incl);
+        const int nacc = tot & 0xff, nch = tot >> 20;
+        int nleaf = (tot >> 8) & 0xfff;
         // accepted cells: at most one entry per lane
-        int tot;
-        int pos = wave_excl_scan<1>(act == 1 ? 1 : 0, &tot);
-        if (icnt + tot > BH_ICAP) flush();
-        if (act == 1) {
-            il[icnt + pos] = make_float4((float)(mo.cx - ox), (float)(mo.cy - oy),
-                                         (float)(mo.cz - oz), mo.mass);
-            ie[icnt + pos] = mo.emax;
+        if (icnt + nacc > BH_ICAP) flush();
+        if (mine & 1u) {
+            const int q = icnt + (int)((incl - mine) & 0xff);
+            il[q] = make_float4((float)(mo.cx - ox), (float)(mo.cy - oy),
+                                (float)(mo.cz - oz), mo.mass);
+            ie[q] = mo.emax;
         }
-        icnt += tot;
-        // particles of opened leaves: rounds of at most BH_ROUND per lane, so
-        // one round never exceeds 64 * BH_ROUND = BH_ICAP entries.  The lane
-        // that opened a leaf only writes its particles' indices into their
-        // list slots; the whole wave then loads the particles, one slot per
-        // lane (same slots, same list order)
-        int rem = act == 2 ? nent : 0;
-        int pb = act == 2 ? lnk : 0;
-        while (__any(rem > 0)) {
-            int tk = rem < BH_ROUND ? rem : BH_ROUND;
-            int lpos = wave_excl_scan<3>(tk, &tot);
-            if (icnt + tot > BH_ICAP) flush();
-            for (int q = 0; q < tk; ++q) ie[icnt + lpos + q] = __int_as_float(pb + q);
+        icnt += nacc;
+        // children onto the stack, the leaf particles' indices above them
+        const int top = sp + nch;
+        {
+            const uint32_t before = incl - mine;
+            const int nq = (mine >> 8 & 0xfff) + (int)(mine >> 20);
+            const int at = mine >> 20 ? sp + (int)(before >> 20) : top + (int)(before >> 8 & 0xfff);
+            if (top + nleaf > SCAP) overflow = 1;
+#pragma unroll
+            for (int q = 0; q < 8; ++q)
+                if (q < nq && at + q < SCAP) stk[at + q] = lnk + q;
+        }
+        sp = min(top, SCAP);
+        while (nleaf > 0) {
             __syncthreads();
-            for (int s = lane; s < tot; s += 64) {
-                const int p = __float_as_int(ie[icnt + s]);
-                il[icnt + s] = make_float4((float)(a.x[p] - ox), (float)(a.y[p] - oy),
-                                           (float)(a.z[p] - oz), (float)a.m[p]);
-                ie[icnt + s] = (float)a.eps[p];
+            nleaf = min(nleaf, SCAP - top);
+            for (int s = 0; s < nleaf;) {
+                if (icnt == BH_ICAP) flush();
+                const int c = min(min(64, nleaf - s), BH_ICAP - icnt);
+                if (lane < c) {
+                    const int p = stk[top + s + lane];
+                    il[icnt + lane] = make_float4((float)(a.x[p] - ox), (float)(a.y[p] - oy),
+                                                  (float)(a.z[p] - oz), (float)a.m[p]);
+                    ie[icnt + lane] = (float)a.eps[p];
+                }
+                icnt += c;
+                s += c;
             }
-            __syncthreads();
-            icnt += tot;
-            rem -= tk;
-            pb += tk;
+            // an unsplittable leaf (coincident particles) holds more than eight
+            rem -= 8;
+            lnk += 8;
+            nleaf = 0;
+            if (__any(rem > 0)) {
+                mine = (uint32_t)max(0, min(rem, 8));
+                incl = wave_incl_scan(mine);
+                nleaf = (int)wave_last(incl);
+                __syncthreads();
+                const int at = top + (int)(incl - mine);
+                if (top + nleaf > SCAP) overflow = 1;
+                for (int q = 0; q < (int)mine; ++q)
+                    if (at + q < SCAP) stk[at + q] = lnk + q;
+            }
         }
-        maxfill = max(maxfill, icnt);
-        // children of opened cells onto the stack
-        int ftot;
-        int fpos = sp + wave_excl_scan<4>(nfr, &ftot);  // 0..8 children
-        if (act == 3) {
-            int c0 = lnk;
-            for (int q = 0; q < nfr; ++q)
-                if (fpos + q < SCAP) stk[fpos + q] = c0 + q;
-        }
-        if (sp + ftot > SCAP) overflow = 1;
-        sp = min(sp + ftot, SCAP);
         __syncthreads();
     }
     flush();
-    if (ok) {
-        a.ax[i] = a.G * kx.value();
-        a.ay[i] = a.G * ky.value();
-        a.az[i] = a.G * kz.value();
-        if (POT) a.pot[i] = -a.G * kp.value();
+    double fx = kx.value(), fy = ky.value(), fz = kz.value(), fp = POT ? kp.value() : 0.0;
+#pragma unroll
+    for (int o = 32; o >= W; o >>= 1) {
+        fx += __shfl_xor(fx, o, 64);
+        fy += __shfl_xor(fy, o, 64);
+        fz += __shfl_xor(fz, o, 64);
+        if (POT) fp += __shfl_xor(fp, o, 64);
+    }
+    if (psum) {
+        if (sub == 0) psum[lane] = make_double4(fx, fy, fz, fp);
+    } else if (ok && sub == 0) {
+        a.ax[i] = a.G * fx;
+        a.ay[i] = a.G * fy;
+        a.az[i] = a.G * fz;
+        if (POT) a.pot[i] = -a.G * fp;
     }
     if (lane == 0) {
         atomicAdd((unsigned long long *)&a.stats[0], (unsigned long long)(ninter * gn));
@@ -573,14 +700,65 @@ __global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
     }
 }
 
+template <bool POT, int SCAP>
+__global__ __launch_bounds__(64) void k_bh_walk(BhTree T, BhArgs a) {
+    __shared__ int32_t stk[SCAP];
+    __shared__ float4 il[BH_ICAP];
+    __shared__ float ie[BH_ICAP];
+    int64_t g0;
+    int gn, lo = 0, hi = INT32_MAX, smask = 0, sval = 0;
+    double4 *psum = nullptr;
+    if ((int)blockIdx.x < a.npart) {
+        const int4 it = a.part[blockIdx.x];
+        g0 = it.x;
+        gn = it.y & 0xff;
+        sval = it.y >> 20 & 15;
+        smask = it.y >> 24 & 15;
+        lo = it.z;
+        hi = it.w;
+        psum = a.psum + 64 * (int64_t)blockIdx.x;
+    } else {
+        // deep cells last in the list, and first here: theirs are the long walks
+        const int g = gridDim.x - 1 - blockIdx.x;
+        g0 = a.gbeg[g];
+        gn = a.gcnt[g];
+    }
+    if (gn > 32) bh_walk_group<POT, SCAP, 1>(T, a, stk, il, ie, g0, gn, lo, hi, smask, sval, psum);
+    else if (gn > 16) bh_walk_group<POT, SCAP, 2>(T, a, stk, il, ie, g0, gn, lo, hi, smask, sval, psum);
+    else bh_walk_group<POT, SCAP, 4>(T, a, stk, il, ie, g0, gn, lo, hi, smask, sval, psum);
+}
+
+// The sums of a group in parts, in the order of the parts.
+template <bool POT>
+__global__ __launch_bounds__(64) void k_bh_join(BhArgs a) {
+    const int4 it = a.part[blockIdx.x];
+    const int parts = it.y >> 8 & 0xfff, gn = it.y & 0xff, lane = threadIdx.x;
+    if (parts == 0 || lane >= gn) return;
+    double x = 0.0, y = 0.0, z = 0.0, p = 0.0;
+    for (int k = 0; k < parts; ++k) {
+        const double4 v = a.psum[64 * ((int64_t)blockIdx.x + k) + lane];
+        x += v.x;
+        y += v.y;
+        z += v.z;
+        p += v.w;
+    }
+    const int64_t i = it.x + lane;
+    a.ax[i] = a.G * x;
+    a.ay[i] = a.G * y;
+    a.az[i] = a.G * z;
+    if (POT) a.pot[i] = -a.G * p;
+}
+
 }  // namespace
 
 // Host side: tree storage (owned here, not by the engine) and the build.
 struct BhHost {
     BhTree T{};
     int64_t cap = 0;
-    int32_t *gbeg = nullptr, *gcnt = nullptr;
+    BhGroups g{};
     int64_t gcap = 0;
+    double4 *psum = nullptr;
+    int64_t icap = 0, pcap = 0;
     int32_t *nk = nullptr, *off = nullptr, *bounds = nullptr, *total = nullptr, *tsum = nullptr;
     int64_t scratch_cap = 0;
     int64_t *stats = nullptr;
@@ -704,35 +882,53 @@ int sphx_bh_run(Engine &E, BhHost &H, double theta, bool with_pot, hipStream_t s
         k_bh_moments<<<(unsigned)((l1 - l0 + BHT - 1) / BHT), BHT, 0, st>>>(
             H.T, l0, l1, E.keys, E.s.x, E.s.y, E.s.z, E.s.m, eps, rbox, cell0);
     }
-    // walk groups
-    int64_t gneed = (int64_t)nodes + n / 64 + 1;
+    // walk groups.  Items of groups in parts: eight groups at most of a cell of
+    // c >= 2 BH_PART particles, at every level, take c / BH_PART + BH_OUT.
+    const int64_t gneed = (int64_t)nodes + n / 64 + 1;
+    H.g.share = bh_share(n);
+    const int64_t pneed = (H.g.share > 1 ? gneed * H.g.share : 1) +
+                          8 * (n / BH_PART) * (BH_OUT / 2 + 1) * (depth + 1);
     if (gneed > H.gcap) {
         int64_t c = std::max<int64_t>(gneed, 2 * H.gcap);
-        SPHX_CHECK(H.alloc((void **)&H.gbeg, sizeof(int32_t) * c));
-        SPHX_CHECK(H.alloc((void **)&H.gcnt, sizeof(int32_t) * c));
+        SPHX_CHECK(H.alloc((void **)&H.g.beg, sizeof(int32_t) * c));
+        SPHX_CHECK(H.alloc((void **)&H.g.cnt, sizeof(int32_t) * c));
         H.gcap = c;
     }
-    SPHX_HIP(hipMemsetAsync(H.total + 1, 0, sizeof(int32_t), st));
-    k_bh_groups<<<(unsigned)((nodes + BHT - 1) / BHT), BHT, 0, st>>>(H.T, nodes, H.gbeg, H.gcnt,
-                                                                      H.total + 1);
+    if (pneed > H.icap) {
+        SPHX_CHECK(H.alloc((void **)&H.g.part, sizeof(int4) * pneed));
+        H.icap = pneed;
+    }
+    H.g.count = H.total + 1;
+    SPHX_HIP(hipMemsetAsync(H.g.count, 0, 3 * sizeof(int32_t), st));
+    k_bh_groups<<<(unsigned)((nodes + BHT - 1) / BHT), BHT, 0, st>>>(H.T, nodes, H.g);
     SPHX_HIP(hipGetLastError());
-    int32_t ngroups = 0;
-    SPHX_HIP(hipMemcpyAsync(&ngroups, H.total + 1, 4, hipMemcpyDeviceToHost, st));
+    int32_t ng[3] = {0, 0, 0};
+    SPHX_HIP(hipMemcpyAsync(ng, H.g.count, sizeof(ng), hipMemcpyDeviceToHost, st));
     SPHX_HIP(hipStreamSynchronize(st));
-    if (ngroups <= 0 || ngroups > gneed) {
+    if (ng[0] < 0 || ng[0] > gneed || ng[1] < 0 || ng[1] > pneed || ng[0] + ng[1] == 0) {
         sphx_set_error("Barnes-Hut group list inconsistent with the tree");
         return SPHX_ERR_STATE;
     }
+    if (ng[1] > H.pcap) {
+        const int64_t c = std::max<int64_t>(ng[1], 2 * H.pcap);
+        SPHX_CHECK(H.alloc((void **)&H.psum, sizeof(double4) * 64 * c));
+        H.pcap = c;
+    }
     SPHX_HIP(hipMemsetAsync(H.stats, 0, sizeof(int64_t) * 4, st));
     SPHX_HIP(hipEventRecord(ev[1], st));
-    BhArgs a{E.s.x, E.s.y, E.s.z, E.s.m, eps, H.gbeg, H.gcnt, n, E.p.G, theta,
+    BhArgs a{E.s.x, E.s.y, E.s.z, E.s.m, eps, H.g.beg, H.g.cnt, H.g.part, ng[1], H.psum, n, E.p.G, theta,
              E.s.gx, E.s.gy, E.s.gz, with_pot ? E.s.pot : nullptr, H.stats,
              E.counters + CNT_BH_OVERFLOW};
     const bool deep = theta < BH_DEEP_THETA;
-    if (with_pot && deep) k_bh_walk<true, BH_SCAP_DEEP><<<(unsigned)ngroups, 64, 0, st>>>(H.T, a);
-    else if (with_pot) k_bh_walk<true, BH_SCAP><<<(unsigned)ngroups, 64, 0, st>>>(H.T, a);
-    else if (deep) k_bh_walk<false, BH_SCAP_DEEP><<<(unsigned)ngroups, 64, 0, st>>>(H.T, a);
-    else k_bh_walk<false, BH_SCAP><<<(unsigned)ngroups, 64, 0, st>>>(H.T, a);
+    const unsigned grid = (unsigned)(ng[0] + ng[1]);
+    if (with_pot && deep) k_bh_walk<true, BH_SCAP_DEEP><<<grid, 64, 0, st>>>(H.T, a);
+    else if (with_pot) k_bh_walk<true, BH_SCAP><<<grid, 64, 0, st>>>(H.T, a);
+    else if (deep) k_bh_walk<false, BH_SCAP_DEEP><<<grid, 64, 0, st>>>(H.T, a);
+    else k_bh_walk<false, BH_SCAP><<<grid, 64, 0, st>>>(H.T, a);
+    if (ng[1] > 0) {
+        if (with_pot) k_bh_join<true><<<(unsigned)ng[1], 64, 0, st>>>(a);
+        else k_bh_join<false><<<(unsigned)ng[1], 64, 0, st>>>(a);
+    }
     SPHX_HIP(hipGetLastError());
     SPHX_HIP(hipEventRecord(ev[2], st));
     if (out) {
@@ -744,7 +940,7 @@ int sphx_bh_run(Engine &E, BhHost &H, double theta, bool with_pot, hipStream_t s
         out->interactions = sv[0];
         out->overflow = sv[1];
         out->max_fill = sv[2];
-        out->groups = ngroups;
+        out->groups = ng[0] + ng[2];
         float b = 0.f, w = 0.f;
         SPHX_HIP(hipEventElapsedTime(&b, ev[0], ev[1]));
         SPHX_HIP(hipEventElapsedTime(&w, ev[1], ev[2]));

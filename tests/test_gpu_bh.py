@@ -114,3 +114,27 @@ def test_bh_potential(gpu, theta, tol_pot, tol_acc):
     acc_o, pot_o = oracle.gravity(p.pos, p.m, p.eps, 1.0, potential=True)
     assert rel_rms(pot, pot_o) < tol_pot
     assert rel_rms(acc, acc_o) < tol_acc
+
+
+@pytest.mark.parametrize("n", [1, 63, 2049, 8192, 8193, 32768, 32769, 98305])
+def test_bh_waves_of_a_group_cover_every_pair(gpu, n):
+    """Groups walked by several waves (eight, four, two or one for a whole run by
+    its size, and parts for outliers beside full cells): every particle is summed
+    once at an opening angle that opens every cell, and its force is the direct
+    sum's to FP32 rounding (1e-5 relative RMS, the bar of the tree that covers
+    every particle)."""
+    from sph_2_amd import libsx
+
+    p = ic.plummer(n, seed=31, eps=0.02)
+    acc, pot, st = libsx.getAcc_g_bh(p.pos, p.m, 1.0, p.eps, 1e-6, return_potential=True,
+                                     return_stats=True)
+    assert st["interactions"] == n * n and st["overflow"] == 0
+    rows = np.unique(np.r_[np.argsort((p.pos ** 2).sum(1))[-40:], np.linspace(0, n - 1, 40).astype(int)])
+    rows = rows[(rows >= 0) & (rows < n)]
+    if n > 1:
+        ref = oracle.gravity(p.pos, p.m, p.eps, 1.0, rows=rows)
+        assert rel_rms(acc[rows], ref) < 1e-5
+    plain = libsx.getAcc_g_bh(p.pos, p.m, 1.0, p.eps, 1e-6)
+    assert rel_rms(plain, acc) < 1e-6 if n > 1 else np.array_equal(plain, acc)
+    again = libsx.getAcc_g_bh(p.pos, p.m, 1.0, p.eps, 1e-6)
+    assert np.array_equal(plain, again)
