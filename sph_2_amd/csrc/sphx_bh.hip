@@ -55,142 +55,98 @@ struct __align__(32) BhLink {
 };
 
 struct BhTree {
-    int32_t *beg, *cnt, *child, *nchild, *level;
-    double *mass, *cx, *cy, *cz, *gx, *gy, *gz, *size, *delta, *emax;
+    int32_t *beg, *cnt, *child, *nchild;
+    double *mass, *emax;
     BhMono *mono;
     BhLink *link;
+    int32_t *ncell;  // cells of each level, BH_LEVELS of them, zero past the deepest
+    int64_t cap;     // cells the arrays hold
 };
+constexpr int BH_LEVELS = 23;
 
 __device__ __forceinline__ int digit_at(uint64_t key, int shift) { return (int)((key >> shift) & 7ull); }
 
-// For each cell of the current level: the nine child boundaries (first index
-// of each child digit) and the number of non-empty children.
-__global__ void k_bh_split(BhTree T, int32_t f0, int32_t fc, const uint64_t *__restrict__ keys,
-                           int level, int32_t *__restrict__ nk, int32_t *__restrict__ bounds) {
-    int t = blockIdx.x * BHT + threadIdx.x;
-    if (t >= fc) return;
-    int i = f0 + t;
-    int b = T.beg[i], c = T.cnt[i];
-    int32_t *bd = bounds + 9 * t;
-    if (c <= BH_LEAF || level >= 21) {
-        nk[t] = 0;
-        bd[0] = -1;
-        return;
+// Cells of a level: [*beg, *beg + returned), as far as the arrays hold them.
+__device__ __forceinline__ int64_t bh_level(const BhTree &T, int level, int64_t *beg) {
+    int64_t b = 0;
+    for (int l = 0; l < level; ++l) b += T.ncell[l];
+    *beg = b;
+    return min((int64_t)T.ncell[level], max((int64_t)0, T.cap - b));
+}
+
+__global__ void k_bh_root(BhTree T, int32_t n, bool fresh, int32_t *__restrict__ gcount,
+                          int64_t *__restrict__ stats) {
+    const int t = threadIdx.x;
+    if (t < 3) gcount[t] = 0;
+    if (t < 4) stats[t] = 0;
+    if (!fresh) return;
+    if (t < BH_LEVELS) T.ncell[t] = t == 0;
+    if (t == 0) {
+        T.beg[0] = 0;
+        T.cnt[0] = n;
     }
-    int shift = 3 * (20 - level);
-    bd[0] = b;
-    bd[8] = b + c;
-    for (int d = 1; d < 8; ++d) {
-        int lo = b, hi = b + c;  // first index with digit >= d
+}
+
+// One level of the build: eight lanes a cell find its child boundaries (first
+// index of each child digit) side by side, a workgroup takes room for its cells'
+// children with one atomic, and the children are written.  The cells' order
+// within a level depends on the atomics; no result does, the walk follows links.
+// Bound: the chain of dependent key loads of a search (20 at the root).  A search
+// by one lane a cell (28 us a level at 1,048,576 particles), three launches of a
+// scan, an emitting one and a wait for the level's count -> one launch a level
+// and the counts left on the device: build of 1,048,576 particles 800 -> 315 us,
+// of 2,000 343 -> 120.
+__global__ __launch_bounds__(BHT) void k_bh_split(BhTree T, const uint64_t *__restrict__ keys, int level) {
+    __shared__ int32_t wsum[BHT / 64], base;
+    const int tid = threadIdx.x, lane = tid & 63, d = tid & 7;
+    int64_t f0;
+    const int64_t fc = bh_level(T, level, &f0), next = f0 + T.ncell[level];
+    const int shift = 3 * (20 - level);
+    for (int64_t t0 = (int64_t)blockIdx.x * (BHT / 8); t0 < fc; t0 += (int64_t)gridDim.x * (BHT / 8)) {
+        const int64_t t = t0 + (tid >> 3), i = f0 + t;
+        int b = 0, c = 0;
+        if (t < fc) {
+            b = T.beg[i];
+            c = T.cnt[i];
+        }
+        const bool leaf = c <= BH_LEAF || level >= 21;
+        int lo = b, hi = leaf || d == 0 ? b : b + c;  // first index with digit >= d
         while (lo < hi) {
-            int mid = (lo + hi) >> 1;
+            const int mid = (lo + hi) >> 1;
             if (digit_at(keys[mid], shift) < d) lo = mid + 1;
             else hi = mid;
         }
-        bd[d] = lo;
-    }
-    int k = 0;
-    for (int d = 0; d < 8; ++d) k += bd[d + 1] > bd[d] ? 1 : 0;
-    nk[t] = k;
-}
-
-// Exclusive scan of fc counts (one workgroup), total written to *total.
-// Exclusive scan of the fc child counts of a level, in three launches of
-// 1024-entry tiles: the tile sums, a scan of the tile sums (writing the
-// total), then each tile's scan on top of its offset.
-constexpr int BH_SCAN_TILE = 1024;
-
-__global__ __launch_bounds__(256) void k_bh_scan_tiles(const int32_t *__restrict__ in, int32_t fc,
-                                                       int32_t *__restrict__ tsum) {
-    __shared__ int32_t red[256];
-    const int t = blockIdx.x, tid = threadIdx.x;
-    const int64_t b = (int64_t)t * BH_SCAN_TILE;
-    int s = 0;
-    for (int k = tid; k < BH_SCAN_TILE; k += 256)
-        if (b + k < fc) s += in[b + k];
-    red[tid] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (tid < o) red[tid] += red[tid + o];
+        int end = __shfl_down(lo, 1, 8);
+        if (d == 7) end = b + c;
+        const bool has = !leaf && end > lo;
+        const uint64_t m = __ballot(has);
+        const int mine = (int)((m >> (lane & 56)) & 0xff);
+        if (lane == 0) wsum[tid >> 6] = __popcll(m);
         __syncthreads();
-    }
-    if (tid == 0) tsum[t] = red[0];
-}
-
-__global__ __launch_bounds__(1024) void k_bh_scan_sums(int32_t *__restrict__ tsum, int ntiles,
-                                                       int32_t *__restrict__ total) {
-    __shared__ int32_t part[1024];
-    const int tid = threadIdx.x;
-    const int per = (ntiles + 1023) / 1024;
-    const int b = min(ntiles, tid * per), e = min(ntiles, b + per);
-    int s = 0;
-    for (int i = b; i < e; ++i) s += tsum[i];
-    part[tid] = s;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-        int v = tid >= off ? part[tid - off] : 0;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
-    }
-    int run = tid > 0 ? part[tid - 1] : 0;
-    for (int i = b; i < e; ++i) {
-        int v = tsum[i];
-        tsum[i] = run;
-        run += v;
-    }
-    if (tid == 1023) *total = part[1023];
-}
-
-__global__ __launch_bounds__(256) void k_bh_scan_apply(const int32_t *__restrict__ in, int32_t fc,
-                                                       const int32_t *__restrict__ tsum,
-                                                       int32_t *__restrict__ out) {
-    __shared__ int32_t part[256];
-    const int t = blockIdx.x, tid = threadIdx.x;
-    const int64_t b = (int64_t)t * BH_SCAN_TILE + 4 * tid;  // four consecutive entries per thread
-    int v[4], s = 0;
-    for (int k = 0; k < 4; ++k) {
-        v[k] = b + k < fc ? in[b + k] : 0;
-        s += v[k];
-    }
-    part[tid] = s;
-    __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
-        int u = tid >= off ? part[tid - off] : 0;
-        __syncthreads();
-        part[tid] += u;
-        __syncthreads();
-    }
-    int run = tsum[t] + (tid > 0 ? part[tid - 1] : 0);
-    for (int k = 0; k < 4; ++k) {
-        if (b + k < fc) out[b + k] = run;
-        run += v[k];
-    }
-}
-
-__global__ void k_bh_emit(BhTree T, int32_t f0, int32_t fc, const int32_t *__restrict__ off,
-                          const int32_t *__restrict__ bounds, int32_t base, int level) {
-    int t = blockIdx.x * BHT + threadIdx.x;
-    if (t >= fc) return;
-    int i = f0 + t;
-    const int32_t *bd = bounds + 9 * t;
-    if (bd[0] < 0) {
-        T.child[i] = -1;
-        T.nchild[i] = 0;
-        return;
-    }
-    int o = base + off[t];
-    int k = 0;
-    for (int d = 0; d < 8; ++d) {
-        if (bd[d + 1] > bd[d]) {
-            T.beg[o + k] = bd[d];
-            T.cnt[o + k] = bd[d + 1] - bd[d];
-            T.level[o + k] = level + 1;
-            ++k;
+        if (tid == 0) {
+            int s = 0;
+            for (int w = 0; w < BHT / 64; ++w) {
+                const int v = wsum[w];
+                wsum[w] = s;
+                s += v;
+            }
+            base = s ? atomicAdd(&T.ncell[level + 1], s) : 0;
         }
+        __syncthreads();
+        const int64_t first = next + base + wsum[tid >> 6] + __popcll(m & ((1ull << (lane & 56)) - 1));
+        if (has) {
+            const int64_t o = first + __popc(mine & ((1 << d) - 1));
+            if (o < T.cap) {
+                T.beg[o] = lo;
+                T.cnt[o] = end - lo;
+            }
+        }
+        if (t < fc && d == 0) {
+            T.child[i] = leaf ? -1 : (int32_t)first;
+            T.nchild[i] = __popc(mine);
+        }
+        __syncthreads();
     }
-    T.child[i] = o;
-    T.nchild[i] = k;
 }
 
 __device__ __forceinline__ uint32_t compact3(uint64_t v) {
@@ -205,58 +161,63 @@ __device__ __forceinline__ uint32_t compact3(uint64_t v) {
 }
 
 // Moments of the cells of one level (children are one level deeper and done).
-__global__ void k_bh_moments(BhTree T, int32_t l0, int32_t l1, const uint64_t *__restrict__ keys,
-                             const double *__restrict__ x, const double *__restrict__ y,
-                             const double *__restrict__ z, const double *__restrict__ m,
-                             const double *__restrict__ eps, const double *__restrict__ rbox,
-                             double cell0) {
-    int i = l0 + blockIdx.x * BHT + threadIdx.x;
-    if (i >= l1) return;
-    double M = 0.0, sx = 0.0, sy = 0.0, sz = 0.0, em = 0.0;
-    if (T.child[i] < 0) {
-        for (int q = T.beg[i]; q < T.beg[i] + T.cnt[i]; ++q) {
-            double mq = m[q];
-            M += mq;
-            sx += mq * x[q]; sy += mq * y[q]; sz += mq * z[q];
-            em = fmax(em, eps[q]);
+__global__ __launch_bounds__(BHT) void k_bh_moments(BhTree T, int level, const uint64_t *__restrict__ keys,
+                                                    const double *__restrict__ x,
+                                                    const double *__restrict__ y,
+                                                    const double *__restrict__ z,
+                                                    const double *__restrict__ m,
+                                                    const double *__restrict__ eps,
+                                                    const double *__restrict__ rbox) {
+    int64_t l0;
+    const int64_t nl = bh_level(T, level, &l0);
+    const double ext = fmax(rbox[1] - rbox[0], fmax(rbox[3] - rbox[2], rbox[5] - rbox[4]));
+    // cell0 = side of a level-21 cell
+    const double cell0 = ext > 0.0 ? ext * (1.0 + 0x1p-30) / (double)(1ull << 21) : 1.0;
+    const double side = cell0 * (double)(1ull << (21 - level));
+    for (int64_t t = (int64_t)blockIdx.x * BHT + threadIdx.x; t < nl; t += (int64_t)gridDim.x * BHT) {
+        const int64_t i = l0 + t;
+        const int b = T.beg[i], cnt = T.cnt[i], child = T.child[i], nchild = T.nchild[i];
+        double M = 0.0, sx = 0.0, sy = 0.0, sz = 0.0, em = 0.0;
+        if (child < 0) {
+            for (int q = b; q < b + cnt; ++q) {
+                double mq = m[q];
+                M += mq;
+                sx += mq * x[q]; sy += mq * y[q]; sz += mq * z[q];
+                em = fmax(em, eps[q]);
+            }
+        } else if ((int64_t)child + nchild <= T.cap) {
+            for (int c = child; c < child + nchild; ++c) {
+                double mc = T.mass[c];
+                const BhMono mo = T.mono[c];
+                M += mc;
+                sx += mc * mo.cx; sy += mc * mo.cy; sz += mc * mo.cz;
+                em = fmax(em, T.emax[c]);
+            }
         }
-    } else {
-        for (int c = T.child[i]; c < T.child[i] + T.nchild[i]; ++c) {
-            double mc = T.mass[c];
-            M += mc;
-            sx += mc * T.cx[c]; sy += mc * T.cy[c]; sz += mc * T.cz[c];
-            em = fmax(em, T.emax[c]);
-        }
+        double cx = M > 0.0 ? sx / M : 0.0, cy = M > 0.0 ? sy / M : 0.0, cz = M > 0.0 ? sz / M : 0.0;
+        uint64_t pre = level > 0 ? keys[b] >> (3 * (21 - level)) : 0ull;
+        double gx = rbox[0] + (compact3(pre >> 2) + 0.5) * side;
+        double gy = rbox[2] + (compact3(pre >> 1) + 0.5) * side;
+        double gz = rbox[4] + (compact3(pre) + 0.5) * side;
+        double dl = sqrt((cx - gx) * (cx - gx) + (cy - gy) * (cy - gy) + (cz - gz) * (cz - gz));
+        T.mass[i] = M;
+        T.emax[i] = em;
+        BhMono mo;
+        mo.cx = cx; mo.cy = cy; mo.cz = cz;
+        mo.mass = (float)M;
+        mo.emax = (float)em;
+        T.mono[i] = mo;
+        BhLink lk;
+        // rounded up so that the FP32 opening test is never looser than the FP64 one
+        lk.size = __double2float_ru(side);
+        lk.delta = __double2float_ru(dl);
+        lk.child = child;
+        lk.nchild = nchild;
+        lk.beg = b;
+        lk.cnt = cnt;
+        lk.pad0 = lk.pad1 = 0;
+        T.link[i] = lk;
     }
-    double cx = M > 0.0 ? sx / M : 0.0, cy = M > 0.0 ? sy / M : 0.0, cz = M > 0.0 ? sz / M : 0.0;
-    int l = T.level[i];
-    double side = cell0 * (double)(1ull << (21 - l));   // cell0 = side of a level-21 cell
-    uint64_t pre = l > 0 ? keys[T.beg[i]] >> (3 * (21 - l)) : 0ull;
-    double gx = rbox[0] + (compact3(pre >> 2) + 0.5) * side;
-    double gy = rbox[2] + (compact3(pre >> 1) + 0.5) * side;
-    double gz = rbox[4] + (compact3(pre) + 0.5) * side;
-    T.mass[i] = M;
-    T.cx[i] = cx; T.cy[i] = cy; T.cz[i] = cz;
-    T.gx[i] = gx; T.gy[i] = gy; T.gz[i] = gz;
-    T.size[i] = side;
-    double dl = sqrt((cx - gx) * (cx - gx) + (cy - gy) * (cy - gy) + (cz - gz) * (cz - gz));
-    T.delta[i] = dl;
-    T.emax[i] = em;
-    BhMono mo;
-    mo.cx = cx; mo.cy = cy; mo.cz = cz;
-    mo.mass = (float)M;
-    mo.emax = (float)em;
-    T.mono[i] = mo;
-    BhLink lk;
-    // rounded up so that the FP32 opening test is never looser than the FP64 one
-    lk.size = __double2float_ru(side);
-    lk.delta = __double2float_ru(dl);
-    lk.child = T.child[i];
-    lk.nchild = T.nchild[i];
-    lk.beg = T.beg[i];
-    lk.cnt = T.cnt[i];
-    lk.pad0 = lk.pad1 = 0;
-    T.link[i] = lk;
 }
 
 // Walk groups: the children (cnt <= 64) of a cell with more than 64
@@ -276,6 +237,7 @@ __global__ void k_bh_moments(BhTree T, int32_t l0, int32_t l1, const uint64_t *_
 // wave took 0.65 ms for 131,072, where 1,024 take 0.55 and 512 take 0.59; four
 // waves outside took 1.20 ms for 262,144, eight 0.99 and sixteen 0.86.
 constexpr int BH_PART = 1024, BH_PARTS_MAX = 256, BH_OUT = 16;
+static_assert(BH_PART > BH_PARTS_MAX, "no part of a cell's range is empty");
 
 // A small run has too few groups to fill the device: all its groups go to
 // several waves (every SHARE-th entry by the cell's first particle), at the
@@ -297,14 +259,13 @@ struct BhGroups {
 __device__ __forceinline__ void bh_add_group(const BhGroups &g, int beg, int cnt, int cell, int ccnt) {
     const int parts = min(ccnt / BH_PART, BH_PARTS_MAX);
     if (parts >= 2) {
-        const int all = parts + BH_OUT;
+        // no range is empty: a part has at least BH_PART > BH_PARTS_MAX particles
+        const int all = parts + BH_OUT, step = (ccnt + parts - 1) / parts;
         const int k = atomicAdd(&g.count[1], all);
         atomicAdd(&g.count[2], 1);
-        for (int64_t p = 0; p < parts; ++p) {
-            const int lo = cell + (int)(ccnt * p / parts);
-            const int hi = cell + (int)(ccnt * (p + 1) / parts);
-            g.part[k + p] = make_int4(beg, cnt | (p ? 0 : all << 8), lo, hi);
-        }
+        for (int p = 0; p < parts; ++p)
+            g.part[k + p] = make_int4(beg, cnt | (p ? 0 : all << 8), cell + min(ccnt, p * step),
+                                      cell + min(ccnt, (p + 1) * step));
         for (int p = 0; p < BH_OUT; ++p)
             g.part[k + parts + p] = make_int4(beg, cnt | p << 20 | (BH_OUT - 1) << 24, cell + ccnt, cell);
     } else if (g.share > 1) {
@@ -319,13 +280,12 @@ __device__ __forceinline__ void bh_add_group(const BhGroups &g, int beg, int cnt
     }
 }
 
-__global__ void k_bh_groups(BhTree T, int32_t ncell, BhGroups G) {
-    int i = blockIdx.x * BHT + threadIdx.x;
-    if (i >= ncell) return;
+__device__ __forceinline__ void bh_cell_groups(const BhTree &T, int64_t i, const BhGroups &G) {
     const int c = T.cnt[i], b = T.beg[i];
     if (i == 0 && c <= 64) bh_add_group(G, b, c, b, c);
     if (c <= 64) return;
     if (T.child[i] >= 0) {
+        if ((int64_t)T.child[i] + T.nchild[i] > T.cap) return;  // to be built again
         // consecutive small children are packed into one group of at most 64
         // (their union stays inside this cell's cube)
         int pb = -1, pc = 0;
@@ -345,6 +305,14 @@ __global__ void k_bh_groups(BhTree T, int32_t ncell, BhGroups G) {
     } else {
         for (int o = 0; o < c; o += 64) bh_add_group(G, b + o, min(64, c - o), b, 0);
     }
+}
+
+// Over the levels 0 to top, those that have been split.
+__global__ __launch_bounds__(BHT) void k_bh_groups(BhTree T, int top, BhGroups G) {
+    int64_t beg;
+    const int64_t n = bh_level(T, top, &beg) + beg;
+    for (int64_t i = (int64_t)blockIdx.x * BHT + threadIdx.x; i < min(n, T.cap); i += (int64_t)gridDim.x * BHT)
+        bh_cell_groups(T, i, G);
 }
 
 // Inclusive prefix sum over the wave, every lane active: within the rows of 16
@@ -735,6 +703,7 @@ __global__ __launch_bounds__(64) void k_bh_join(BhArgs a) {
     const int parts = it.y >> 8 & 0xfff, gn = it.y & 0xff, lane = threadIdx.x;
     if (parts == 0 || lane >= gn) return;
     double x = 0.0, y = 0.0, z = 0.0, p = 0.0;
+#pragma unroll 8
     for (int k = 0; k < parts; ++k) {
         const double4 v = a.psum[64 * ((int64_t)blockIdx.x + k) + lane];
         x += v.x;
@@ -759,8 +728,6 @@ struct BhHost {
     int64_t gcap = 0;
     double4 *psum = nullptr;
     int64_t icap = 0, pcap = 0;
-    int32_t *nk = nullptr, *off = nullptr, *bounds = nullptr, *total = nullptr, *tsum = nullptr;
-    int64_t scratch_cap = 0;
     int64_t *stats = nullptr;
     std::vector<void *> owned;
     ~BhHost() {
@@ -782,18 +749,14 @@ static int bh_alloc_nodes(BhHost &H, int64_t need) {
     if (need <= H.cap) return SPHX_OK;
     int64_t cap = std::max<int64_t>(need, 2 * H.cap);
     BhTree T{};
-    int32_t **ip[] = {&T.beg, &T.cnt, &T.child, &T.nchild, &T.level};
-    double **dp[] = {&T.mass, &T.cx, &T.cy, &T.cz, &T.gx, &T.gy, &T.gz, &T.size, &T.delta, &T.emax};
+    int32_t **ip[] = {&T.beg, &T.cnt, &T.child, &T.nchild};
+    double **dp[] = {&T.mass, &T.emax};
     for (int32_t **q : ip) SPHX_CHECK(H.alloc((void **)q, sizeof(int32_t) * cap));
     for (double **q : dp) SPHX_CHECK(H.alloc((void **)q, sizeof(double) * cap));
     SPHX_CHECK(H.alloc((void **)&T.mono, sizeof(BhMono) * cap));
     SPHX_CHECK(H.alloc((void **)&T.link, sizeof(BhLink) * cap));
-    if (H.cap > 0) {
-        int32_t *oi[] = {H.T.beg, H.T.cnt, H.T.child, H.T.nchild, H.T.level};
-        int32_t *ni[] = {T.beg, T.cnt, T.child, T.nchild, T.level};
-        for (int k = 0; k < 5; ++k)
-            SPHX_HIP(hipMemcpy(ni[k], oi[k], sizeof(int32_t) * H.cap, hipMemcpyDeviceToDevice));
-    }
+    SPHX_CHECK(H.alloc((void **)&T.ncell, sizeof(int32_t) * (BH_LEVELS + 3)));
+    T.cap = cap;
     H.T = T;
     H.cap = cap;
     return SPHX_OK;
@@ -820,101 +783,74 @@ int sphx_bh_run(Engine &E, BhHost &H, double theta, bool with_pot, hipStream_t s
     } evfree{ev};
     SPHX_HIP(hipEventRecord(ev[0], st));
     SPHX_CHECK(bh_alloc_nodes(H, std::max<int64_t>(1024, n / 2)));
-    if (!H.total) {
-        SPHX_CHECK(H.alloc((void **)&H.total, sizeof(int32_t) * 4));
-        SPHX_CHECK(H.alloc((void **)&H.stats, sizeof(int64_t) * 4));
-    }
-    // root
-    int32_t root[5] = {0, (int32_t)n, -1, 0, 0};
-    SPHX_HIP(hipMemcpyAsync(H.T.beg, &root[0], 4, hipMemcpyHostToDevice, st));
-    SPHX_HIP(hipMemcpyAsync(H.T.cnt, &root[1], 4, hipMemcpyHostToDevice, st));
-    SPHX_HIP(hipMemcpyAsync(H.T.level, &root[4], 4, hipMemcpyHostToDevice, st));
-    std::vector<int32_t> lev{0, 1};
-    int32_t nodes = 1;
-    for (int level = 0; level < 21; ++level) {
-        int32_t f0 = lev[level], fc = lev[level + 1] - lev[level];
-        if (fc <= 0) break;
-        if (fc > H.scratch_cap) {
-            int64_t c = std::max<int64_t>(fc, 2 * H.scratch_cap);
-            SPHX_CHECK(H.alloc((void **)&H.nk, sizeof(int32_t) * c));
-            SPHX_CHECK(H.alloc((void **)&H.off, sizeof(int32_t) * c));
-            SPHX_CHECK(H.alloc((void **)&H.bounds, sizeof(int32_t) * 9 * c));
-            SPHX_CHECK(H.alloc((void **)&H.tsum, sizeof(int32_t) * ((c + BH_SCAN_TILE - 1) / BH_SCAN_TILE)));
-            H.scratch_cap = c;
-        }
-        unsigned g = (unsigned)((fc + BHT - 1) / BHT);
-        k_bh_split<<<g, BHT, 0, st>>>(H.T, f0, fc, E.keys, level, H.nk, H.bounds);
-        const int ntiles = (int)((fc + BH_SCAN_TILE - 1) / BH_SCAN_TILE);
-        k_bh_scan_tiles<<<ntiles, 256, 0, st>>>(H.nk, fc, H.tsum);
-        k_bh_scan_sums<<<1, 1024, 0, st>>>(H.tsum, ntiles, H.total);
-        k_bh_scan_apply<<<ntiles, 256, 0, st>>>(H.nk, fc, H.tsum, H.off);
-        int32_t tot = 0;
-        SPHX_HIP(hipMemcpyAsync(&tot, H.total, 4, hipMemcpyDeviceToHost, st));
-        SPHX_HIP(hipStreamSynchronize(st));
-        if ((int64_t)nodes + tot > H.cap) SPHX_CHECK(bh_alloc_nodes(H, (int64_t)nodes + tot));
-        k_bh_emit<<<g, BHT, 0, st>>>(H.T, f0, fc, H.off, H.bounds, nodes, level);
-        SPHX_HIP(hipGetLastError());
-        nodes += tot;
-        lev.push_back(nodes);
-        if (tot == 0) break;
-    }
-    // leaves of the deepest level (never split) get child = -1
-    {
-        int32_t f0 = lev[lev.size() - 2], fc = lev.back() - f0;
-        if (fc > 0 && (int)lev.size() - 2 >= 21) {
-            std::vector<int32_t> neg(fc, -1), zero(fc, 0);
-            SPHX_HIP(hipMemcpyAsync(H.T.child + f0, neg.data(), 4 * fc, hipMemcpyHostToDevice, st));
-            SPHX_HIP(hipMemcpyAsync(H.T.nchild + f0, zero.data(), 4 * fc, hipMemcpyHostToDevice, st));
-            SPHX_HIP(hipStreamSynchronize(st));
-        }
-    }
-    int depth = (int)lev.size() - 2;
-    // moments bottom-up; the run box gives the cell geometry
+    if (!H.stats) SPHX_CHECK(H.alloc((void **)&H.stats, sizeof(int64_t) * 4));
     const double *rbox = E.bbox + 6 * (int64_t)E.t.ns;
-    double hb[6];
-    SPHX_HIP(hipMemcpyAsync(hb, rbox, sizeof(hb), hipMemcpyDeviceToHost, st));
-    SPHX_HIP(hipStreamSynchronize(st));
-    double ext = std::max(hb[1] - hb[0], std::max(hb[3] - hb[2], hb[5] - hb[4]));
-    double cell0 = ext > 0.0 ? ext * (1.0 + 0x1p-30) / (double)(1ull << 21) : 1.0;
-    for (int l = depth; l >= 0; --l) {
-        int32_t l0 = lev[l], l1 = lev[l + 1];
-        if (l1 <= l0) continue;
-        k_bh_moments<<<(unsigned)((l1 - l0 + BHT - 1) / BHT), BHT, 0, st>>>(
-            H.T, l0, l1, E.keys, E.s.x, E.s.y, E.s.z, E.s.m, eps, rbox, cell0);
+    // Levels 0 to top are built, summed and cut into groups without waiting for
+    // their counts, seven levels more than a uniform cloud takes (an empty level
+    // costs 5 us, a wait 20).  A deeper tree is split on, summed and cut again,
+    // and built anew where the arrays do not hold its cells.
+    int top = 6, from = 0;
+    for (int64_t c = 8; c < n; c *= 8) ++top;
+    top = std::min(top, 21);
+    int32_t ncell[BH_LEVELS], ng[3] = {0, 0, 0};
+    int64_t nodes = 0;
+    for (;;) {
+        // at most 8^level cells, of the nodes that the arrays hold
+        auto blocks = [&](int level, int per) {
+            const int64_t c = level < 7 ? (int64_t)1 << (3 * level) : H.cap;
+            return (unsigned)std::min<int64_t>((std::min(c, H.cap) + per - 1) / per, 4096);
+        };
+        const int64_t gneed = H.cap + n / 64 + 1;
+        // Items of groups in parts: eight groups at most of a cell of c >= 2 BH_PART
+        // particles, at every level, take c / BH_PART + BH_OUT.
+        H.g.share = bh_share(n);
+        const int64_t pneed = (H.g.share > 1 ? gneed * H.g.share : 1) +
+                              8 * (n / BH_PART) * (BH_OUT / 2 + 1) * (top + 1);
+        if (gneed > H.gcap) {
+            SPHX_CHECK(H.alloc((void **)&H.g.beg, sizeof(int32_t) * gneed));
+            SPHX_CHECK(H.alloc((void **)&H.g.cnt, sizeof(int32_t) * gneed));
+            H.gcap = gneed;
+        }
+        if (pneed > H.icap) {
+            SPHX_CHECK(H.alloc((void **)&H.g.part, sizeof(int4) * pneed));
+            H.icap = pneed;
+        }
+        H.g.count = H.T.ncell + BH_LEVELS;
+        k_bh_root<<<1, 64, 0, st>>>(H.T, (int32_t)n, from == 0, H.g.count, H.stats);
+        for (int l = from; l <= top; ++l) k_bh_split<<<blocks(l, BHT / 8), BHT, 0, st>>>(H.T, E.keys, l);
+        for (int l = top; l >= 0; --l)
+            k_bh_moments<<<blocks(l, BHT), BHT, 0, st>>>(H.T, l, E.keys, E.s.x, E.s.y, E.s.z, E.s.m, eps, rbox);
+        k_bh_groups<<<blocks(7, BHT), BHT, 0, st>>>(H.T, top, H.g);
+        SPHX_HIP(hipGetLastError());
+        int32_t back[BH_LEVELS + 3];
+        SPHX_HIP(hipMemcpyAsync(back, H.T.ncell, sizeof(back), hipMemcpyDeviceToHost, st));
+        SPHX_HIP(hipStreamSynchronize(st));
+        std::copy(back, back + BH_LEVELS, ncell);
+        std::copy(back + BH_LEVELS, back + BH_LEVELS + 3, ng);
+        nodes = 0;
+        for (int32_t c : ncell) nodes += c;
+        if (nodes <= H.cap && (top == 21 || ncell[top + 1] == 0)) {
+            if (ng[0] < 0 || ng[0] > gneed || ng[1] < 0 || ng[1] > pneed || ng[0] + ng[1] == 0) {
+                sphx_set_error("Barnes-Hut group list inconsistent with the tree");
+                return SPHX_ERR_STATE;
+            }
+            break;
+        }
+        from = top + 1;
+        if (nodes > H.cap) {
+            SPHX_CHECK(bh_alloc_nodes(H, nodes + nodes / 4));
+            from = 0;
+        }
+        top = std::min(top + 4, 21);
     }
-    // walk groups.  Items of groups in parts: eight groups at most of a cell of
-    // c >= 2 BH_PART particles, at every level, take c / BH_PART + BH_OUT.
-    const int64_t gneed = (int64_t)nodes + n / 64 + 1;
-    H.g.share = bh_share(n);
-    const int64_t pneed = (H.g.share > 1 ? gneed * H.g.share : 1) +
-                          8 * (n / BH_PART) * (BH_OUT / 2 + 1) * (depth + 1);
-    if (gneed > H.gcap) {
-        int64_t c = std::max<int64_t>(gneed, 2 * H.gcap);
-        SPHX_CHECK(H.alloc((void **)&H.g.beg, sizeof(int32_t) * c));
-        SPHX_CHECK(H.alloc((void **)&H.g.cnt, sizeof(int32_t) * c));
-        H.gcap = c;
-    }
-    if (pneed > H.icap) {
-        SPHX_CHECK(H.alloc((void **)&H.g.part, sizeof(int4) * pneed));
-        H.icap = pneed;
-    }
-    H.g.count = H.total + 1;
-    SPHX_HIP(hipMemsetAsync(H.g.count, 0, 3 * sizeof(int32_t), st));
-    k_bh_groups<<<(unsigned)((nodes + BHT - 1) / BHT), BHT, 0, st>>>(H.T, nodes, H.g);
-    SPHX_HIP(hipGetLastError());
-    int32_t ng[3] = {0, 0, 0};
-    SPHX_HIP(hipMemcpyAsync(ng, H.g.count, sizeof(ng), hipMemcpyDeviceToHost, st));
-    SPHX_HIP(hipStreamSynchronize(st));
-    if (ng[0] < 0 || ng[0] > gneed || ng[1] < 0 || ng[1] > pneed || ng[0] + ng[1] == 0) {
-        sphx_set_error("Barnes-Hut group list inconsistent with the tree");
-        return SPHX_ERR_STATE;
-    }
+    // levels up to the first empty one
+    int depth = 1;
+    while (depth < 21 && ncell[depth] > 0) ++depth;
     if (ng[1] > H.pcap) {
         const int64_t c = std::max<int64_t>(ng[1], 2 * H.pcap);
         SPHX_CHECK(H.alloc((void **)&H.psum, sizeof(double4) * 64 * c));
         H.pcap = c;
     }
-    SPHX_HIP(hipMemsetAsync(H.stats, 0, sizeof(int64_t) * 4, st));
     SPHX_HIP(hipEventRecord(ev[1], st));
     BhArgs a{E.s.x, E.s.y, E.s.z, E.s.m, eps, H.g.beg, H.g.cnt, H.g.part, ng[1], H.psum, n, E.p.G, theta,
              E.s.gx, E.s.gy, E.s.gz, with_pot ? E.s.pot : nullptr, H.stats,

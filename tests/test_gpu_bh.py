@@ -138,3 +138,24 @@ def test_bh_waves_of_a_group_cover_every_pair(gpu, n):
     assert rel_rms(plain, acc) < 1e-6 if n > 1 else np.array_equal(plain, acc)
     again = libsx.getAcc_g_bh(p.pos, p.m, 1.0, p.eps, 1e-6)
     assert np.array_equal(plain, again)
+
+
+@pytest.mark.parametrize("n,each", [(9, 9), (900, 9), (9000, 9), (9000, 100), (40000, 2)])
+def test_bh_deep_trees(gpu, n, each):
+    """Clusters of coincident particles: chains of cells down to the deepest
+    level, more levels and more cells than the build starts with, and leaves
+    that hold more than eight.  Every particle is summed once (an angle of 1e-7
+    opens the deepest cells too, whose side is 2^-21 of the box's: s / theta is
+    4.8 box sides)."""
+    from sph_2_amd import libsx
+
+    c = ic.plummer(max(2, n // each), seed=32, eps=0.05)
+    pos = np.repeat(c.pos, each, axis=0)[:n]
+    m = np.full(n, 1.0 / n)
+    eps = np.full(n, 0.05)
+    acc, st = libsx.getAcc_g_bh(pos, m, 1.0, eps, 1e-7, return_stats=True)
+    assert st["interactions"] == n * n and st["overflow"] == 0
+    assert each <= 8 or st["depth"] == 21 or n == 9
+    rows = np.linspace(0, n - 1, 50).astype(int)
+    ref = oracle.gravity(pos, m, eps, 1.0, rows=rows)
+    assert np.sqrt(((acc[rows] - ref) ** 2).sum()) < 1e-5 * max(1.0, np.sqrt((ref ** 2).sum()))
