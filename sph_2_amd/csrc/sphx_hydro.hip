@@ -151,8 +151,8 @@ __device__ __forceinline__ void seg_box(bool mine, double x, double y, double z,
 }
 
 // The particles a walk group takes: a whole bucket (P = 1) or, in runs too
-// small to fill the device with one wave per bucket, a half or a quarter of
-// one, so that there are P times the groups and each meets fewer candidates.
+// small to fill the device with one wave per bucket, a half, a quarter or an
+// eighth of one, so that there are P times the groups and each meets fewer candidates.
 // A group holds T = 64 / P targets, lane L the target L mod T; its P lanes per
 // target are slices that take a P-th of every batch of candidates each.  A
 // part walks the candidates of its own box, exactly as a segment does, so every
@@ -1439,17 +1439,17 @@ __global__ __launch_bounds__(64) void k_lists(Tables t, Soa s, DensArgs a) {
         q->len = nn;
         q->pad = 0;
     }
-    // four flags per bucket, one per quarter
+    // eight flags per bucket, one per eighth
     const uint64_t o = __ballot(ok && nn > SPHX_NBR_MAX);
-    if (lane < 4 / P) a.ovf[4 * b + (4 / P) * ws.part + lane] = o ? 1 : 0;
+    if (lane < 8 / P) a.ovf[8 * b + (8 / P) * ws.part + lane] = o ? 1 : 0;
     if (lane == 0 && a.counters)
         atomicAdd((unsigned long long *)&a.counters[CNT_CAND], (unsigned long long)ncand);
 }
 
-// Whether a quarter of bucket b has a list that overflowed.
+// Whether an eighth of bucket b has a list that overflowed.
 __device__ __forceinline__ bool bucket_ovf(const int32_t *ovf, int64_t b) {
-    const int4 o = reinterpret_cast<const int4 *>(ovf)[b];
-    return (o.x | o.y | o.z | o.w) != 0;
+    const int4 o = reinterpret_cast<const int4 *>(ovf)[2 * b], p = reinterpret_cast<const int4 *>(ovf)[2 * b + 1];
+    return (o.x | o.y | o.z | o.w | p.x | p.y | p.z | p.w) != 0;
 }
 
 // Value of v in lane U of this lane's quad.
@@ -2291,15 +2291,17 @@ int sphx_neighbor_pass(Engine &E, int64_t r0, int64_t r1, int32_t *counts, const
     return SPHX_OK;
 }
 
-// Small runs walk a half or a quarter of a bucket per group: with one wave per
-// bucket most SIMDs would hold a single wave or none, and a group's chain of
+// Small runs walk a half, a quarter or an eighth of a bucket per group: with one
+// wave per bucket most SIMDs would hold a single wave or none, and a group's chain of
 // loads, tests and LDS round trips sets the time.  Smaller groups gather more
 // candidate buckets in all, which costs more once the chip is full.  Measured,
 // one / two / four groups a bucket, on a collapsing Evrard sphere (us, boxes
-// included): smoothing 77 / 46 / 40 at 4,096 particles, 119 / 77 / 91 at 32,768,
+// included, the density pass as it was then): smoothing 77 / 46 / 40 at 4,096 particles, 119 / 77 / 91 at 32,768,
 // 159 / 112 / 149 at 65,752, 146 / 165 / 238 at 131,072; lists and density 154
 // / 96 / 80 at 4,096, 277 / 164 / 155 at 65,752, 255 / 218 / 224 at 131,072,
-// 330 / 363 / 387 at 262,144.
+// 330 / 363 / 387 at 262,144.  Four / eight groups: lists and density 66 / 57 at
+// 4,096, 88 / 81 at 16,384, 108 / 112 at 24,576; smoothing 33 / 28 at 2,048, 36 /
+// 36 at 4,096, 51 / 56 at 8,192 (left at four).
 int Engine::smooth_parts() const { return nb_launch() <= 384 ? 4 : (nb_launch() <= 1536 ? 2 : 1); }
 // Small runs, whose passes are bounded by launches and by the chain of one
 // wave a SIMD: the list passes walk an overflowed bucket themselves (that costs
@@ -2309,7 +2311,10 @@ int Engine::smooth_parts() const { return nb_launch() <= 384 ? 4 : (nb_launch() 
 // against 45 at 32,768, 45 against 44 at 46,341, 56 against 53 at 65,752, 639
 // against 521 at 1,048,576, where the gathers bound it.
 bool Engine::list_small() const { return nb_launch() <= 512; }
-int Engine::list_parts() const { return nb_launch() <= 1536 ? 4 : (nb_launch() <= 3072 ? 2 : 1); }
+int Engine::list_parts() const {
+    const unsigned nb = nb_launch();
+    return nb <= 256 ? 8 : nb <= 1536 ? 4 : nb <= 3072 ? 2 : 1;
+}
 
 int Engine::smoothing(hipStream_t st, bool predictor) {
     if (n == 0 || nb_launch() == 0) return SPHX_OK;
@@ -2346,7 +2351,8 @@ int Engine::build_lists(hipStream_t st) {
     }
     DensArgs a{p.gamma, tmpi, counters, nbr, prec, nbr_ovf};
     const int nb = (int)nb_launch(), parts = list_parts();
-    if (parts == 4) k_lists<4><<<nb * 4, 64, 0, st>>>(tview(), s, a);
+    if (parts == 8) k_lists<8><<<nb * 8, 64, 0, st>>>(tview(), s, a);
+    else if (parts == 4) k_lists<4><<<nb * 4, 64, 0, st>>>(tview(), s, a);
     else if (parts == 2) k_lists<2><<<nb * 2, 64, 0, st>>>(tview(), s, a);
     else k_lists<1><<<nb, 64, 0, st>>>(tview(), s, a);
     SPHX_HIP(hipGetLastError());

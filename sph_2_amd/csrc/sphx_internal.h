@@ -406,7 +406,7 @@ struct Engine {
     bool want_lists = false;
     bool use_lists = true;      // tuning knob: the walks give the same bits
     int32_t *nbr = nullptr;     // nbr_bcap buckets x SPHX_NBR_MAX x 64
-    int32_t *nbr_ovf = nullptr; // four per bucket (one per quarter)
+    int32_t *nbr_ovf = nullptr; // eight per bucket (one per eighth)
     int64_t nbr_bcap = 0;
     PairRec *prec = nullptr;    // per particle of capacity
     float *fbal = nullptr;      // per particle of capacity

@@ -1,6 +1,6 @@
-"""The candidate walks at the sizes where their shape changes (a quarter, a half
-or a whole bucket per group: 384 / 385, 1,536 / 1,537 and 3,072 / 3,073 buckets),
-with a partial last bucket, and where the FP32 screen of the FP64 distance test
+"""The candidate walks at the sizes where their shape changes (an eighth, a
+quarter, a half or a whole bucket per group: 256 / 257, 384 / 385, 1,536 / 1,537
+and 3,072 / 3,073 buckets), with a partial last bucket, and where the FP32 screen of the FP64 distance test
 is hardest: coordinates far from the origin, units far from one, distances that
 equal the radius.  Counts and smoothing lengths bit for bit the oracle's."""
 import numpy as np
@@ -12,7 +12,7 @@ from sph_2_amd import ic
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 63, 65, 1000, 24576, 24577, 98304, 98305, 196608, 196650])
+@pytest.mark.parametrize("n", [1, 63, 65, 1000, 16384, 16385, 24576, 24577, 98304, 98305, 196608, 196650])
 def test_walk_shapes(gpu, n):
     from sph_2_amd import libsx
 
