@@ -590,7 +590,7 @@ def serve_stream(a, runs: int, verbose: bool = False) -> dict:
         "arrival_rate_per_s": a.rate, "hbm_budget_gb": a.hbm_gb,
         "graph_replay": bool(a.serve_graph),
         "gravity": ("tiled" if sym is None else
-                    f"symmetric ({sym[0]} block pairs per wave, {sym[1]:.0%} of the budget for "
+                    f"symmetric ({sym[0]} block pairs per segment, {sym[1]:.0%} of the budget for "
                     f"its partial sums)")}
     return out
 

@@ -345,7 +345,7 @@ int sphx_global_dt_noalloc(int device, int64_t n, const double *h, const double 
                            double c_cfl, double dt_min, double dt_max, double *out, void *stream);
 
 /* Morton keys (21 bits per axis, 63-bit key) over the bounding box of pos,
- * then a stable LSD radix sort; keys_out[i] and perm_out[i] = original index of
+ * then a stable merge sort; keys_out[i] and perm_out[i] = original index of
  * the i-th smallest key.  Synchronous. */
 int sphx_morton_sort(sphx_ctx *ctx, int64_t n, const double *pos, uint64_t *keys_out,
                      int32_t *perm_out, void *stream);

@@ -33,7 +33,7 @@ def _size_class(n: int) -> str:
 
 def _default(n: int):
     """The shape of a size the table holds no entry for: from 1M particles the
-    symmetric sum with 16 block pairs per wave (its partial sums are summed in
+    symmetric sum with 16 block pairs per segment (its partial sums are summed in
     row bands of bounded memory), below that the tiled kernel with enough j
     split for four workgroups per CU."""
     if (1 << 20) <= n <= SYM_MAX_N:
@@ -102,7 +102,7 @@ def tune_cells(n: int, seed: int = 0, steps: int = 3):
 def pick(res: dict):
     """The fastest shape, except that among shapes within 1 % of it the one
     needing the least extra memory wins: a tiled shape (none), else the
-    symmetric sum with the most block pairs per wave (fewest partial sums),
+    symmetric sum with the most block pairs per segment (fewest partial sums),
     whole block pairs before split ones."""
     t_best = min(res.values())
     near = [k for k, v in res.items() if v <= 1.01 * t_best]

@@ -1777,11 +1777,10 @@ extern "C" int sphx_plan_destroy(sphx_plan *plan) {
 
 // Gravity launch configuration of a plan (used by the autotuner).
 // Tiled sum: ipl 1/2/4 particles per lane, j tiles of 256/512/1024, js j
-// splits (1..64).  Symmetric sum: ipl 8, tj 512, js = block pairs per wave
-// (1..4096).
+// splits (1..64).  Symmetric sum: ipl 8, tj 512, js = block pairs per
+// segment (1..4096).
 static bool gravity_config_ok(int32_t ipl, int32_t tj, int32_t js) {
-    // symmetric sum: js block pairs per wave, or (js = 1) a block pair split
-    // into 512 / tj parts of tj j particles
+    // symmetric sum: js block pairs per segment; tj 256 and 128 with js = 1 mean 512
     if (ipl == 8) return (tj == 512 && js >= 1 && js <= 4096) || ((tj == 256 || tj == 128) && js == 1);
     return (ipl == 1 || ipl == 2 || ipl == 4) && (tj == 256 || tj == 512 || tj == 1024) &&
            js >= 1 && js <= 64 && !(ipl == 1 && tj == 1024) && !(ipl == 4 && tj == 1024);
