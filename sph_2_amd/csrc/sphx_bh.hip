@@ -432,10 +432,10 @@ __device__ __forceinline__ void bh_pair(float xi, float yi, float zi, float ei, 
 // instructions an entry for 17); softened ones without a branch (34 for some
 // 45); a group of at most 32 or 16 particles gives each two or four lanes; the
 // three counts of a batch are scanned in one word, and opened leaves listed 64
-// particles at a time.  VALU instructions a wave, before -> after: 72,000 ->
-// 51,000 on an Evrard sphere of 1,048,576 particles with eps = h, theta 0.5 (walk
-// 2.33 -> 1.94 ms), 99,900 -> 67,200 on a Plummer sphere of 524,288 (2.68 -> 2.12
-// ms, and 1.52 with the groups in parts and the long walks first).
+// particles at a time.  VALU instructions of the launch, with the groups in
+// parts, before -> after: 1.65 -> 1.22 x 10^9 on an Evrard sphere of 1,048,576
+// particles with eps = h, theta 0.5 (2.33 -> 1.85 ms), 1.15 -> 0.79 x 10^9 on a
+// Plummer sphere of 524,288 (2.68 -> 1.48 ms).
 //
 // The walk of one group of gn particles, P lanes a particle (P W = 64): lane
 // (sub, p) sums every P-th entry of the list for particle p.  Of the accepted
