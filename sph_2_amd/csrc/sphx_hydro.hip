@@ -241,9 +241,11 @@ __device__ __forceinline__ WalkFrame walk_frame(const double *gb, double reach) 
     const int be = (int)(((unsigned long long)__double_as_longlong(reach) >> 52) & 0x7ffull);
     const bool fine = reach > 0.0 && be >= 543 && be <= 1523;
     f.sc = fine ? __longlong_as_double((long long)(2046 - be) << 52) : 0.0;
-    f.ex = __double2float_ru(0.5 * (gb[1] - gb[0]) * f.sc * (1.0 + 0x1p-40));
-    f.ey = __double2float_ru(0.5 * (gb[3] - gb[2]) * f.sc * (1.0 + 0x1p-40));
-    f.ez = __double2float_ru(0.5 * (gb[5] - gb[4]) * f.sc * (1.0 + 0x1p-40));
+    // from the centre as it was rounded: far from the origin it is off the box's
+    // middle by as much as the particles' own spacing there
+    f.ex = __double2float_ru(fmax(gb[1] - f.ox, f.ox - gb[0]) * f.sc * (1.0 + 0x1p-40));
+    f.ey = __double2float_ru(fmax(gb[3] - f.oy, f.oy - gb[2]) * f.sc * (1.0 + 0x1p-40));
+    f.ez = __double2float_ru(fmax(gb[5] - f.oz, f.oz - gb[4]) * f.sc * (1.0 + 0x1p-40));
     return f;
 }
 // Bound on |r^2 - S^2| below which the FP32 value may have the wrong sign:

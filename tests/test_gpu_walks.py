@@ -109,3 +109,35 @@ def test_list_passes_equal_the_walks(gpu, n):
                 assert (c["nbr_overflow"] > 0) == wide, c
         for f in outs[0]:
             assert np.array_equal(outs[0][f], outs[1][f]), (f, wide)
+
+
+def _capped_ok(call, *a, **kw):
+    import warnings
+
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", RuntimeWarning)  # the odd particle finds no length
+        return call(*a, **kw)
+
+
+@pytest.mark.parametrize("shift", [0.0, 2.0 ** 46, 2.0 ** 51, 2.0 ** 52])
+def test_far_offsets(gpu, shift):
+    """Particles so far from the origin that the middle of a group's box is
+    rounded by a good part of the search radius: a lattice whose pairs lie on the
+    radius, and a sphere."""
+    from sph_2_amd import libsx
+
+    g = np.arange(14.0)
+    pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3) + shift
+    m = np.full(len(pos), 1.0 / len(pos))
+    for r in (2.0, 3.0):
+        hh = np.full(len(pos), 0.5 * r)
+        cnt = libsx.getDensity(pos, m, hh, return_count=True)[1]
+        assert np.array_equal(cnt, oracle.density(pos, m, hh)[1])
+        for h_mode in (0, 2):
+            h, k, it = _capped_ok(libsx.smoothing_h, pos, hh, h_mode=h_mode)
+            ho, ko, ito, _ = oracle.smoothing(pos, hh, p=oracle.Params(h_mode=h_mode))
+            assert np.array_equal(h, ho) and np.array_equal(k, ko) and np.array_equal(it, ito)
+    e = ic.evrard(3000, seed=34)
+    pos, h0 = 64.0 * e.pos + shift * np.array([1.0, -0.75, 0.875]), 64.0 * e.h
+    cnt = libsx.getDensity(pos, e.m, h0, return_count=True)[1]
+    assert np.array_equal(cnt, oracle.density(pos, e.m, h0)[1])
