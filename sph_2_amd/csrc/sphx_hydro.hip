@@ -228,7 +228,8 @@ struct WalkLds {
 // two that brings the search radius near one, so that FP32 neither over- nor
 // underflows at any scale of the run.  A radius whose square comes near the
 // ends of the FP64 range (below 2^-480, above 2^500), where r^2 itself is
-// rounded coarsely, leaves sc = 0, and every batch is tested in FP64.
+// rounded coarsely, and a box or radius that is not finite leave sc = 0: every
+// candidate is then kept and every batch tested in FP64.
 struct WalkFrame {
     double ox, oy, oz, sc;
     float ex, ey, ez;
@@ -246,6 +247,10 @@ __device__ __forceinline__ WalkFrame walk_frame(const double *gb, double reach) 
     f.ex = __double2float_ru(fmax(gb[1] - f.ox, f.ox - gb[0]) * f.sc * (1.0 + 0x1p-40));
     f.ey = __double2float_ru(fmax(gb[3] - f.oy, f.oy - gb[2]) * f.sc * (1.0 + 0x1p-40));
     f.ez = __double2float_ru(fmax(gb[5] - f.oz, f.oz - gb[4]) * f.sc * (1.0 + 0x1p-40));
+    if (!(f.ex < INFINITY && f.ey < INFINITY && f.ez < INFINITY)) {
+        f.sc = f.ox = f.oy = f.oz = 0.0;
+        f.ex = f.ey = f.ez = 0.0f;
+    }
     return f;
 }
 // Bound on |r^2 - S^2| below which the FP32 value may have the wrong sign:
@@ -259,10 +264,10 @@ __device__ __forceinline__ float walk_band(double S, double M) {
 }
 
 // Calls the sink for the candidates of the group's box gb within `reach` (HH:
-// reach + h_j), in increasing order.  Sink: chunk(hc) before the candidates of
-// a chunk (hc: their largest h), cand(x, y, z, h) for each candidate of the
-// lane's slice of a batch, batch(L, base, n) after it.  Returns the number of
-// candidate buckets.
+// reach + h_j), in increasing order.  Sink: chunk(hc, exact) before the candidates
+// of a chunk (hc: their largest h; exact: the FP32 values say nothing), cand(x, y,
+// z, h) for each candidate of the lane's slice of a batch, batch(L, base, n) after
+// it.  Returns the number of candidate buckets.
 template <int P, bool HH, class Sink>
 __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<HH> &L, int r,
                                          int lane, const double *gb, double reach,
@@ -276,7 +281,8 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
         double hmax = 0.0;
         if (HH) hmax = wave_max_d(hc);
         hc = 0.0;
-        sink.chunk(hmax);
+        const bool exact = !(f.sc > 0.0);
+        sink.chunk(hmax, exact);
         // |relative coordinate| of a particle in reach is at most e + reach; its
         // rounding and that of the distance widen the test by 2^-20
         const float rr = __double2float_ru((reach + hmax) * f.sc);
@@ -330,7 +336,8 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
             ra = ra * (1.0f + 0x1p-20f);
             // a NaN coordinate fails here as it fails every distance test
             const bool finite = fabsf(rx) < INFINITY && fabsf(ry) < INFINITY && fabsf(rz) < INFINITY;
-            const bool keep = lane < c0.n && finite && (dx * dx + dy * dy) + dz * dz <= ra * ra;
+            const bool keep =
+                lane < c0.n && (exact || (finite && (dx * dx + dy * dy) + dz * dz <= ra * ra));
             const uint64_t m = __ballot(keep);
             if (m) {
                 if (keep) {
@@ -423,18 +430,19 @@ struct CountSink {
     WalkTarget p;
     float nS2, band;
     Exact exact;
+    bool all;  // every batch in FP64
     int kc;
     uint32_t m0, m1;
     float amin;
     __device__ __forceinline__ CountSink(const WalkFrame &f, bool act, double xi, double yi, double zi,
                                          double S, Exact ex)
-        : exact(ex), kc(0) {
+        : exact(ex), all(false), kc(0) {
         p.set(f, act, xi, yi, zi);
         const double Ss = S * f.sc, M = fmax(fmax(f.ex, f.ey), f.ez) + 2.0;
         nS2 = act ? -(float)(Ss * Ss) : 1.0f;
         band = act ? (f.sc > 0.0 ? walk_band(Ss, M) : INFINITY) : -1.0f;
     }
-    __device__ __forceinline__ void chunk(double) {}
+    __device__ __forceinline__ void chunk(double, bool ex) { all = ex; }
     __device__ __forceinline__ void begin() { m0 = m1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { m0 = m1; m1 = 0u; }
     __device__ __forceinline__ void cand(float cx, float cy, float cz, float) {
@@ -445,7 +453,7 @@ struct CountSink {
     }
     template <class LDS>
     __device__ __forceinline__ void batch(const LDS &L, int base, int n, int q0) {
-        if (__any(amin <= band)) {
+        if (all || __any(amin <= band)) {
             int c = 0;
             for (int k = 0; k < 64 / P; ++k)
                 if (q0 + k < n && band >= 0.0f && exact(L.j[base + q0 + k])) ++c;
@@ -700,6 +708,7 @@ template <int P>
 struct WindowSink {
     WalkTarget p;
     float nW1, dW, band;
+    bool all = false;  // every batch in FP64
     double xi, yi, zi, W0, W1;
     const Soa *s;
     double *col;
@@ -719,7 +728,7 @@ struct WindowSink {
         dW = (float)(s1 * s1 - s0 * s0);
         band = act ? (f.sc > 0.0 ? walk_band(s1, M) : INFINITY) : -1.0f;
     }
-    __device__ __forceinline__ void chunk(double) {}
+    __device__ __forceinline__ void chunk(double, bool ex) { all = ex; }
     __device__ __forceinline__ void begin() { a0 = a1 = b0 = b1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { a0 = a1; b0 = b1; a1 = b1 = 0u; }
     __device__ __forceinline__ void cand(float cx, float cy, float cz, float) {
@@ -733,7 +742,7 @@ struct WindowSink {
     template <class LDS>
     __device__ __forceinline__ void batch(const LDS &L, int base_, int n, int q0) {
         constexpr int Q = 64 / P;
-        if (__any(amin <= band)) {
+        if (all || __any(amin <= band)) {
             a0 = a1 = b0 = b1 = 0u;
             for (int k = 0; k < Q; ++k) {
                 if (P == 1 && k == 32) word();
@@ -1346,6 +1355,7 @@ template <int P>
 struct ListSink {
     WalkTarget p;
     float fh, band;
+    bool all;  // every batch in FP64
     double xi, yi, zi, hi, hS, sc, e;
     const Soa *s;
     int32_t *lst;  // the target's first run of the block: entry k at nbr_slot(k, 0)
@@ -1356,11 +1366,12 @@ struct ListSink {
     __device__ __forceinline__ ListSink(const WalkFrame &f, bool act_, double x, double y, double z,
                                         double h, double hS_, const Soa *s_, int32_t *lst_, int lane_,
                                         int nn_)
-        : fh(act_ ? (float)(h * f.sc) : 0.0f), xi(x), yi(y), zi(z), hi(h), hS(hS_), sc(f.sc),
+        : fh(act_ ? (float)(h * f.sc) : 0.0f), all(false), xi(x), yi(y), zi(z), hi(h), hS(hS_), sc(f.sc),
           e(fmax(fmax(f.ex, f.ey), f.ez)), s(s_), lst(lst_), lane(lane_), nn(nn_), act(act_) {
         p.set(f, act, x, y, z);
     }
-    __device__ __forceinline__ void chunk(double hc) {
+    __device__ __forceinline__ void chunk(double hc, bool ex) {
+        all = ex;
         const double S = (hi + hc) * sc, M = e + 1.001 * (hS + hc) * sc;
         band = act ? (sc > 0.0 ? walk_band(S, M) : INFINITY) : -1.0f;
     }
@@ -1376,7 +1387,7 @@ struct ListSink {
     template <class LDS>
     __device__ __forceinline__ void batch(const LDS &L, int base, int n, int q0) {
         constexpr int Q = 64 / P;
-        if (__any(amin <= band)) {
+        if (all || __any(amin <= band)) {
             m0 = m1 = 0u;
             for (int k = 0; k < Q; ++k) {
                 if (P == 1 && k == 32) word();

@@ -119,6 +119,65 @@ def _capped_ok(call, *a, **kw):
         return call(*a, **kw)
 
 
+@pytest.mark.parametrize("h_mode", [0, 2, 5])
+@pytest.mark.parametrize("where", [(np.inf, 0.1, 0.1), (0.1, -np.inf, 0.1), (np.inf, -np.inf, np.inf)])
+def test_infinite_position_beside_valid_rows(gpu, where, h_mode):
+    """A particle at infinity has no neighbours and is nobody's: the other rows,
+    those of its own group among them, are what they are without it."""
+    from sph_2_amd import libsx
+
+    e = ic.evrard(700, seed=31)
+    pos = e.pos.copy()
+    pos[333] = where
+    rows = np.delete(np.arange(e.n), 333)
+    h, k, it = _capped_ok(libsx.smoothing_h, pos, e.h, h_mode=h_mode)
+    ho, ko, ito, _ = oracle.smoothing(pos, e.h, p=oracle.Params(h_mode=h_mode), rows=rows)
+    assert np.array_equal(h[rows], ho) and np.array_equal(k[rows], ko) and np.array_equal(it[rows], ito)
+    rho, cnt = libsx.getDensity(pos, e.m, e.h, return_count=True)
+    rho_o, cnt_o = oracle.density(pos, e.m, e.h, rows=rows)
+    assert np.array_equal(cnt[rows], cnt_o)
+    assert np.max(np.abs(rho[rows] / rho_o - 1.0)) < 1e-6
+
+
+@pytest.mark.parametrize("huge", [1e10, np.inf])
+def test_huge_h_beside_valid_rows(gpu, huge):
+    """One particle with a huge or infinite h: everybody's neighbour, with no
+    weight, and no more to the rows beside it."""
+    from sph_2_amd import libsx
+
+    e = ic.evrard(700, seed=32)
+    h = e.h.copy()
+    h[100] = huge
+    rho, cnt = libsx.getDensity(e.pos, e.m, h, return_count=True)
+    rho_o, cnt_o = oracle.density(e.pos, e.m, h)
+    assert np.array_equal(cnt, cnt_o)
+    ok = np.arange(e.n) != 100
+    assert np.max(np.abs(rho[ok] / rho_o[ok] - 1.0)) < 1e-6
+    assert rho[100] == pytest.approx(rho_o[100], rel=1e-5, abs=1e-30)
+    if huge < np.inf:
+        # far particles, one of which only that h reaches
+        pos = e.pos.copy()
+        pos[200] = (0.0, 1.5 * huge, 0.0)
+        pos[201] = (0.5 * huge, 0.0, 0.0)
+        cnt = libsx.getDensity(pos, e.m, h, return_count=True)[1]
+        assert np.array_equal(cnt, oracle.density(pos, e.m, h)[1])
+
+
+@pytest.mark.parametrize("h_mode", [0, 2, 5])
+def test_infinite_start_beside_valid_rows(gpu, h_mode):
+    """A particle whose iteration starts from an infinite length, and the rows
+    of its group."""
+    from sph_2_amd import libsx
+
+    e = ic.evrard(700, seed=33)
+    h0 = e.h.copy()
+    h0[400] = np.inf
+    rows = np.delete(np.arange(e.n), 400)
+    h, k, it = _capped_ok(libsx.smoothing_h, e.pos, h0, h_mode=h_mode)
+    ho, ko, ito, _ = oracle.smoothing(e.pos, h0, p=oracle.Params(h_mode=h_mode), rows=rows)
+    assert np.array_equal(h[rows], ho) and np.array_equal(k[rows], ko) and np.array_equal(it[rows], ito)
+
+
 @pytest.mark.parametrize("shift", [0.0, 2.0 ** 46, 2.0 ** 51, 2.0 ** 52])
 def test_far_offsets(gpu, shift):
     """Particles so far from the origin that the middle of a group's box is
