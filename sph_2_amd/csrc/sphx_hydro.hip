@@ -229,7 +229,7 @@ struct WalkLds {
 // underflows at any scale of the run.  A radius whose square comes near the
 // ends of the FP64 range (below 2^-480, above 2^500), where r^2 itself is
 // rounded coarsely, and a box or radius that is not finite leave sc = 0: every
-// candidate is then kept and every batch tested in FP64.
+// candidate is then tested in FP64, a bucket at a time.
 struct WalkFrame {
     double ox, oy, oz, sc;
     float ex, ey, ez;
@@ -265,9 +265,9 @@ __device__ __forceinline__ float walk_band(double S, double M) {
 
 // Calls the sink for the candidates of the group's box gb within `reach` (HH:
 // reach + h_j), in increasing order.  Sink: chunk(hc, exact) before the candidates
-// of a chunk (hc: their largest h; exact: the FP32 values say nothing), cand(x, y,
-// z, h) for each candidate of the lane's slice of a batch, batch(L, base, n) after
-// it.  Returns the number of candidate buckets.
+// of a chunk (hc: their largest h; exact: every batch is to be tested in FP64),
+// cand(x, y, z, h) for each candidate of the lane's slice of a batch, batch(L,
+// base, n) after it.  Returns the number of candidate buckets.
 template <int P, bool HH, class Sink>
 __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<HH> &L, int r,
                                          int lane, const double *gb, double reach,
@@ -281,11 +281,25 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
         double hmax = 0.0;
         if (HH) hmax = wave_max_d(hc);
         hc = 0.0;
-        const bool exact = !(f.sc > 0.0);
-        sink.chunk(hmax, exact);
         // |relative coordinate| of a particle in reach is at most e + reach; its
         // rounding and that of the distance widen the test by 2^-20
         const float rr = __double2float_ru((reach + hmax) * f.sc);
+        // a candidate's h so far above the group's own that squares in FP32 come
+        // near its range, or the far coordinate, is decided in FP64 as well
+        const bool exact = !(f.sc > 0.0 && rr < 1.0e15f);
+        sink.chunk(hmax, exact);
+        if (exact) {  // (inside the compaction it cost k_lists 2-4 %, here nothing)
+            for (int k = 0; k < nl; ++k) {
+                const int2 e = L.bl[k];
+                L.j[lane] = e.x + lane;
+                __builtin_amdgcn_wave_barrier();
+                sink.begin();
+                sink.batch(L, 0, e.y, q0);
+                __builtin_amdgcn_wave_barrier();
+            }
+            nl = 0;
+            return;
+        }
         const float mx = f.ex + 0x1p-20f * (f.ex + rr), my = f.ey + 0x1p-20f * (f.ey + rr),
                     mz = f.ez + 0x1p-20f * (f.ez + rr);
         struct Cand {
@@ -336,8 +350,7 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
             ra = ra * (1.0f + 0x1p-20f);
             // a NaN coordinate fails here as it fails every distance test
             const bool finite = fabsf(rx) < INFINITY && fabsf(ry) < INFINITY && fabsf(rz) < INFINITY;
-            const bool keep =
-                lane < c0.n && (exact || (finite && (dx * dx + dy * dy) + dz * dz <= ra * ra));
+            const bool keep = lane < c0.n && finite && (dx * dx + dy * dy) + dz * dz <= ra * ra;
             const uint64_t m = __ballot(keep);
             if (m) {
                 if (keep) {
@@ -430,19 +443,18 @@ struct CountSink {
     WalkTarget p;
     float nS2, band;
     Exact exact;
-    bool all;  // every batch in FP64
     int kc;
     uint32_t m0, m1;
     float amin;
     __device__ __forceinline__ CountSink(const WalkFrame &f, bool act, double xi, double yi, double zi,
                                          double S, Exact ex)
-        : exact(ex), all(false), kc(0) {
+        : exact(ex), kc(0) {
         p.set(f, act, xi, yi, zi);
         const double Ss = S * f.sc, M = fmax(fmax(f.ex, f.ey), f.ez) + 2.0;
         nS2 = act ? -(float)(Ss * Ss) : 1.0f;
-        band = act ? (f.sc > 0.0 ? walk_band(Ss, M) : INFINITY) : -1.0f;
+        band = f.sc > 0.0 ? (act ? walk_band(Ss, M) : -1.0f) : INFINITY;
     }
-    __device__ __forceinline__ void chunk(double, bool ex) { all = ex; }
+    __device__ __forceinline__ void chunk(double, bool) {}
     __device__ __forceinline__ void begin() { m0 = m1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { m0 = m1; m1 = 0u; }
     __device__ __forceinline__ void cand(float cx, float cy, float cz, float) {
@@ -453,10 +465,10 @@ struct CountSink {
     }
     template <class LDS>
     __device__ __forceinline__ void batch(const LDS &L, int base, int n, int q0) {
-        if (all || __any(amin <= band)) {
+        if (__any(amin <= band)) {
             int c = 0;
             for (int k = 0; k < 64 / P; ++k)
-                if (q0 + k < n && band >= 0.0f && exact(L.j[base + q0 + k])) ++c;
+                if (q0 + k < n && !(nS2 > 0.0f) && exact(L.j[base + q0 + k])) ++c;
             kc += c;
         } else {
             kc += __popc(m0) + __popc(m1);
@@ -708,7 +720,6 @@ template <int P>
 struct WindowSink {
     WalkTarget p;
     float nW1, dW, band;
-    bool all = false;  // every batch in FP64
     double xi, yi, zi, W0, W1;
     const Soa *s;
     double *col;
@@ -726,9 +737,9 @@ struct WindowSink {
         // r^2 = 0 is inside a window from 0, where the band cannot be trusted to
         // tell: every value within it is tested in FP64
         dW = (float)(s1 * s1 - s0 * s0);
-        band = act ? (f.sc > 0.0 ? walk_band(s1, M) : INFINITY) : -1.0f;
+        band = f.sc > 0.0 ? (act ? walk_band(s1, M) : -1.0f) : INFINITY;
     }
-    __device__ __forceinline__ void chunk(double, bool ex) { all = ex; }
+    __device__ __forceinline__ void chunk(double, bool) {}
     __device__ __forceinline__ void begin() { a0 = a1 = b0 = b1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { a0 = a1; b0 = b1; a1 = b1 = 0u; }
     __device__ __forceinline__ void cand(float cx, float cy, float cz, float) {
@@ -742,13 +753,13 @@ struct WindowSink {
     template <class LDS>
     __device__ __forceinline__ void batch(const LDS &L, int base_, int n, int q0) {
         constexpr int Q = 64 / P;
-        if (all || __any(amin <= band)) {
+        if (__any(amin <= band)) {
             a0 = a1 = b0 = b1 = 0u;
             for (int k = 0; k < Q; ++k) {
                 if (P == 1 && k == 32) word();
                 a1 <<= 1;
                 b1 <<= 1;
-                if (band >= 0.0f && q0 + k < n) {
+                if (!(nW1 > 0.0f) && q0 + k < n) {
                     const int j = L.j[base_ + q0 + k];
                     const double r2 = sphx_r2(xi - s->x[j], yi - s->y[j], zi - s->z[j]);
                     a1 |= r2 <= W1 ? 1u : 0u;
@@ -1355,7 +1366,6 @@ template <int P>
 struct ListSink {
     WalkTarget p;
     float fh, band;
-    bool all;  // every batch in FP64
     double xi, yi, zi, hi, hS, sc, e;
     const Soa *s;
     int32_t *lst;  // the target's first run of the block: entry k at nbr_slot(k, 0)
@@ -1366,14 +1376,13 @@ struct ListSink {
     __device__ __forceinline__ ListSink(const WalkFrame &f, bool act_, double x, double y, double z,
                                         double h, double hS_, const Soa *s_, int32_t *lst_, int lane_,
                                         int nn_)
-        : fh(act_ ? (float)(h * f.sc) : 0.0f), all(false), xi(x), yi(y), zi(z), hi(h), hS(hS_), sc(f.sc),
+        : fh(act_ ? (float)(h * f.sc) : 0.0f), xi(x), yi(y), zi(z), hi(h), hS(hS_), sc(f.sc),
           e(fmax(fmax(f.ex, f.ey), f.ez)), s(s_), lst(lst_), lane(lane_), nn(nn_), act(act_) {
         p.set(f, act, x, y, z);
     }
     __device__ __forceinline__ void chunk(double hc, bool ex) {
-        all = ex;
         const double S = (hi + hc) * sc, M = e + 1.001 * (hS + hc) * sc;
-        band = act ? (sc > 0.0 ? walk_band(S, M) : INFINITY) : -1.0f;
+        band = ex ? INFINITY : (act ? walk_band(S, M) : -1.0f);
     }
     __device__ __forceinline__ void begin() { m0 = m1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { m0 = m1; m1 = 0u; }
@@ -1387,7 +1396,7 @@ struct ListSink {
     template <class LDS>
     __device__ __forceinline__ void batch(const LDS &L, int base, int n, int q0) {
         constexpr int Q = 64 / P;
-        if (all || __any(amin <= band)) {
+        if (__any(amin <= band)) {
             m0 = m1 = 0u;
             for (int k = 0; k < Q; ++k) {
                 if (P == 1 && k == 32) word();

@@ -139,7 +139,7 @@ def test_infinite_position_beside_valid_rows(gpu, where, h_mode):
     assert np.max(np.abs(rho[rows] / rho_o - 1.0)) < 1e-6
 
 
-@pytest.mark.parametrize("huge", [1e10, np.inf])
+@pytest.mark.parametrize("huge", [1e10, 1e18, 1e19, 1e25, 1e100, 1e200, np.inf])
 def test_huge_h_beside_valid_rows(gpu, huge):
     """One particle with a huge or infinite h: everybody's neighbour, with no
     weight, and no more to the rows beside it."""
