@@ -506,6 +506,9 @@ struct SmoothArgs {
     int64_t *counters;
     double hstep;      // RULE 2: the step as a fraction of h_prev (2 x the reference's coeff)
     double hmin;       // RULE 5: the floor on h after eleven steps (0: none)
+    // step rules: the counts that a window's ends are aimed at and the slack
+    // either side of them (hwin 0: no window holds this band)
+    int32_t hwin, wlo, whi, wslack;
 };
 
 // One walk over the candidates of the group's active targets: for each segment
@@ -703,16 +706,21 @@ struct StepIter {
 // up to w0 plus the window's, and between two crossings of the band all passes
 // fall on one side, decided by one distance.
 //
-// Bound: the walks, which every pass took before.  Now there are two to four a
-// group, whatever the passes: the first pass's count, then the window, +- 10 %
-// about the radius that this count makes nngb neighbours likely at; it holds 39
-// +- 6 of 64, so that 64 slots seldom overflow (the window is then narrowed);
-// they take 512 B a target.  A target left without a
-// window (more than 64 particles at one distance, a start that is not a
-// positive number) is walked pass by pass.
+// Bound: the walks, which every pass took before.  Now there are two or three a
+// group, whatever the passes: the first pass's count, and windows whose ends are
+// aimed, from the counts at the last ones, at the band and a quarter of the spare
+// slots beyond it on either side (45 and 83 neighbours for the band 59 to 69), or
+// halved in between.  A window takes nup - ndown + 2 distances at least, of
+// HW_CAP.  Walks of a target on an Evrard sphere of 16,384, from 1.3 times the
+// length (102 passes for all of these): 2.03 on average and 4 at most for the band
+// 59 to 69, 2.41 and 5 for 44 to 84, 3.4 and 9 for 36 to 92; with both ends
+// scaled together about the middle of the band they were passes and 16 walks
+// more for most targets from bands of 41 counts on.  A wider band, a target left
+// without a window (more than 64 particles at one distance, a start that is not a
+// positive number) is walked pass by pass.  The slots take 512 B a target.
 constexpr int HW_CAP = 64;
-constexpr double HW_WIN = 0.1;
-constexpr int HW_WALKS = 16;
+constexpr int HW_WALKS = 8;
+constexpr int HW_SPARE = 4;  // with fewer slots to spare the search takes too long
 
 // Collects the window: base counts r^2 <= W0, the indices of the candidates
 // with W0 < r^2 <= W1 go to the target's column (the first HW_CAP of them).
@@ -857,20 +865,21 @@ __global__ __launch_bounds__(64) void k_smoothing_steps(Tables t, Soa s, SmoothA
     // the first pass settles most targets of a run in progress, and tells the
     // others where the band is
     const int k0 = count(ok, sr);
-    double w0 = 0.0, w1 = 0.0, win = HW_WIN;
+    double w0 = 0.0, w1 = 0.0;
     if (ok) {
         q.pass(k0, a);
         const double c0 = sr * sphx_h_factor(a.nngb, k0);
-        w0 = c0 * (1.0 - win);
-        w1 = c0 * (1.0 + win);
+        w0 = a.wlo > 0 ? c0 * sphx_h_factor(a.wlo, a.nngb) : 0.0;
+        w1 = c0 * sphx_h_factor(a.whi, a.nngb);
     }
 
     // the window
     double *col = hw + tl;
     double lo = 0.0, hi = INFINITY;  // radii known to hold < ndown, and > nup (or the run)
+    double u = INFINITY, v = 0.0;    // and the next ones known not to
     int base = 0, inw = 0;
     bool sel = false, whole = false;
-    bool open = ok && !q.done && fin && sr > 0.0 && sr < INFINITY && w1 < INFINITY;
+    bool open = a.hwin && ok && !q.done && fin && sr > 0.0 && sr < INFINITY && w1 < INFINITY;
     for (int walk = 0; walk < HW_WALKS && __any(open); ++walk) {
         // r^2 bounds of the window; 0 itself is inside a window from 0
         const double W0 = w0 > 0.0 ? sphx_sq(w0) : -1.0, W1 = sphx_sq(w1);
@@ -894,22 +903,27 @@ __global__ __launch_bounds__(64) void k_smoothing_steps(Tables t, Soa s, SmoothA
             if (base > a.nup && w0 < hi) hi = w0;
             if (hi_ok && w1 < hi) hi = w1;
             if (tot < a.ndown && !whole && w1 > lo) lo = w1;
+            if (!lo_ok && w0 < u) u = w0;
+            if (!hi_ok && w1 > v) v = w1;
             if (lo_ok && hi_ok && inw <= HW_CAP) {
                 sel = true;
                 open = false;
             } else {
-                // radii expected to hold nngb, from the counts at the window's ends
-                const double cb = w0 * sphx_h_factor(a.nngb, base);
-                const double ct = w1 * sphx_h_factor(a.nngb, tot);
-                double nw0, nw1;
-                if (lo_ok && hi_ok) {  // too many to keep
-                    win *= 0.5;
-                    nw0 = ct * (1.0 - win);
-                    nw1 = ct * (1.0 + win);
-                } else {
-                    nw0 = (lo_ok ? ct : cb) * (1.0 - win);
-                    nw1 = (hi_ok ? cb : ct) * (1.0 + win);
+                // an end that is not near enough: the middle of the radii between
+                // which it must lie, once both are known, before that aimed anew
+                // from its own count (the lower one from the upper's where its
+                // own says too little)
+                double nw0 = w0, nw1 = w1;
+                if (!lo_ok || base < a.wlo - a.wslack) {
+                    nw0 = 8 * (int64_t)base > a.wlo ? w0 * sphx_h_factor(a.wlo, base)
+                                                    : w1 * sphx_h_factor(a.wlo, tot);
+                    if (lo > 0.0 && u < INFINITY) nw0 = 0.5 * (lo + u);
                 }
+                if (!hi_ok || tot - a.wslack > a.whi) {
+                    nw1 = w1 * sphx_h_factor(a.whi, tot);
+                    if (v > 0.0 && hi < INFINITY) nw1 = 0.5 * (v + hi);
+                }
+                if (a.wlo == 0) nw0 = 0.0;
                 w0 = fmax(lo, nw0);
                 w1 = fmin(hi, nw1);
                 open = w0 < w1 && w1 < INFINITY;
@@ -2341,7 +2355,14 @@ int Engine::list_parts() const {
 int Engine::smoothing(hipStream_t st, bool predictor) {
     if (n == 0 || nb_launch() == 0) return SPHX_OK;
     SmoothArgs a{p.nngb, p.ndown, p.nup, p.max_iter, (predictor && p.h_predictor) ? 1 : 0,
-                 d_run, h_iters, counters, sphx_h_step(p.h_mode), p.h_min};
+                 d_run, h_iters, counters, sphx_h_step(p.h_mode), p.h_min, 0, 0, 0, 0};
+    const int64_t need = (int64_t)p.nup - p.ndown + 2;
+    if (p.ndown >= 1 && need <= HW_CAP - HW_SPARE) {
+        a.hwin = 1;
+        a.wslack = (int)(HW_CAP - need) / 4;
+        a.wlo = std::max(p.ndown - 1 - a.wslack, 0);
+        a.whi = (int)std::min<int64_t>((int64_t)p.nup + 1 + a.wslack, INT32_MAX);
+    }
     const int parts = smooth_parts();
     auto launch = [&](auto k4, auto k2, auto k1) {
         if (parts == 4) k4<<<nb_launch() * 4, 64, 0, st>>>(tview(), s, a);

@@ -48,3 +48,47 @@ def test_step_rules_match_the_oracle(gpu, name, h_mode):
     assert np.array_equal(h, ho)
     assert np.array_equal(k, ko)
     assert np.array_equal(it, ito)
+
+
+@pytest.mark.parametrize("h_mode", [2, 4, 5])
+@pytest.mark.parametrize("nngb,ndown,nup", [(64, 44, 84), (64, 35, 93), (64, 35, 94), (64, 20, 110),
+                                            (200, 170, 230), (32, 1, 33), (32, 0, 40), (500, 480, 520)])
+def test_bands(gpu, nngb, ndown, nup, h_mode):
+    """Bands that nearly fill the window's 64 distances, the widest that takes one
+    (35 to 93), those that take none, and other neighbour numbers."""
+    import warnings
+
+    from sph_2_amd import libsx
+
+    e = ic.evrard(900, seed=6)
+    h0 = e.h * np.geomspace(0.5, 2.0, e.n) * (nngb / 64.0) ** (1.0 / 3.0)
+    kw = dict(h_mode=h_mode, nngb=nngb, ndown=ndown, nup=nup)
+    ho, ko, ito, _ = oracle.smoothing(e.pos, h0, p=oracle.Params(**kw))
+    with warnings.catch_warnings():
+        warnings.simplefilter("ignore", RuntimeWarning)
+        h, k, it = libsx.smoothing_h(e.pos, h0, **kw)
+    assert np.array_equal(h, ho) and np.array_equal(k, ko) and np.array_equal(it, ito)
+
+
+def test_wide_band_costs_no_more(gpu):
+    """From 1.3 times the length the passes are many for any band.  A band of 41
+    counts, which the window still holds, takes about what the narrow one takes;
+    searching for its window in vain took a walk for each of 100 passes."""
+    import time
+
+    from sph_2_amd import libsx
+
+    e = ic.evrard(16384, seed=6)
+    h0 = 1.3 * libsx.smoothing_h(e.pos, e.h)[0]
+
+    def best(**kw):
+        t = []
+        for _ in range(6):
+            t0 = time.perf_counter()
+            libsx.smoothing_h(e.pos, h0, h_mode=2, max_iter=200, **kw)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    narrow = best(nngb=64, ndown=59, nup=69)
+    wide = best(nngb=64, ndown=44, nup=84)
+    assert wide < 2.5 * narrow, (wide, narrow)
