@@ -2382,7 +2382,7 @@ int Engine::smoothing(hipStream_t st, bool predictor) {
 static unsigned ovf_grid(unsigned nb) { return std::min(256u, (nb + 63) / 64); }
 
 bool Engine::lists_ready() const {
-    return use_lists && nbr && prec && fbal && nbr_ovf && nbr_bcap >= t.nb;
+    return use_lists && nbr && prec && fbal && nbr_ovf && nbr_bcap >= t.nb && nbr_pcap >= n;
 }
 
 // The lists and the geometric half of the records.

@@ -407,10 +407,10 @@ struct Engine {
     bool use_lists = true;      // tuning knob: the walks give the same bits
     int32_t *nbr = nullptr;     // nbr_bcap buckets x SPHX_NBR_MAX x 64
     int32_t *nbr_ovf = nullptr; // eight per bucket (one per eighth)
-    int64_t nbr_bcap = 0;
-    PairRec *prec = nullptr;    // per particle of capacity
-    float *fbal = nullptr;      // per particle of capacity
-    bool no_list_mem = false;   // ensure_lists found no memory for them at this capacity
+    int64_t nbr_bcap = 0, nbr_pcap = 0;  // buckets and particles they have room for
+    PairRec *prec = nullptr;    // per particle
+    float *fbal = nullptr;      // per particle
+    int64_t no_list_mem = INT64_MAX;  // ensure_lists found no memory for this many particles
     int alloc_lists(int64_t capacity);
     bool lists_ready() const;
     int32_t *cand_off = nullptr, *cand_cnt = nullptr, *cand = nullptr;
@@ -509,6 +509,9 @@ struct Engine {
     int fill_records(hipStream_t st);
     // allocate the lists if they are not; false (and no error) without the memory
     bool ensure_lists();
+    // give back lists that ensure_lists allocated: all, or large ones
+    void free_lists();
+    void trim_lists();
     int gravity(hipStream_t st, bool with_pot);
     int divcurl(hipStream_t st, bool lists = false);
     int hydro(hipStream_t st, bool lists = false);
