@@ -1225,6 +1225,7 @@ struct SoftSum {
     KahanF x, y, z;
     __device__ __forceinline__ void init() { x.init(); y.init(); z.init(); }
     static __device__ __forceinline__ float factor(float mj, double r2, double hi, double hj) {
+#pragma clang fp contract(off)
         return -mj * sphx_soft_factor((float)r2, (float)hi + (float)hj);
     }
     __device__ __forceinline__ void add(float mj, double dx, double dy, double dz, double r2, double hi,

@@ -149,8 +149,10 @@ struct KahanF {
 // r^-1 is taken once, before the softening test, and also gives r = r^2 r^-1
 // inside the softening length: a transcendental costs several FP32
 // instructions' issue time, and a wave whose lanes split between the two
-// branches runs both.
+// branches runs both.  Here and below the fused multiply-adds are written out, so
+// that every kernel gives a pair the same bits whatever loop it stands in.
 __device__ __forceinline__ float sphx_spline_f(float r2, float t) {
+#pragma clang fp contract(off)
     const float ri = __builtin_amdgcn_rsqf(r2);
     if (r2 >= t * t) return ri * ri * ri;
     const float e = 0.5f * t;
@@ -159,11 +161,12 @@ __device__ __forceinline__ float sphx_spline_f(float r2, float t) {
     const float q = r * ie;
     if (q <= 1.0f) {
         float q2 = q * q;
-        return ie * ie * ie * (4.0f / 3.0f - 1.2f * q2 + 0.5f * q2 * q);
+        return ie * ie * ie * __builtin_fmaf(0.5f * q2, q, __builtin_fmaf(-1.2f, q2, 4.0f / 3.0f));
     }
     float w = 2.0f - q;
     float w2 = w * w;
-    return ri * ri * ri * (1.0f - w2 * w2 * (1.0f - 0.8f * w + w2 * (1.0f / 6.0f)));
+    const float p = __builtin_fmaf(w2, 1.0f / 6.0f, __builtin_fmaf(-0.8f, w, 1.0f));
+    return ri * ri * ri * __builtin_fmaf(-(w2 * w2), p, 1.0f);
 }
 
 // Softened pairs apart from the rest.  With softening eps = h the pairs inside
@@ -180,11 +183,14 @@ __device__ __forceinline__ float sphx_spline_f(float r2, float t) {
 // takes 7 to 13 us more.  Error against FP64 (relative RMS): 2.8e-7 -> 2.6e-7 at
 // 2,048, 8.7e-8 -> 6.1e-8 at 16,384, 4.9e-8 -> 4.1e-8 at 262,144.
 __device__ __forceinline__ float sphx_clamped_r3(float r2, float t) {
+#pragma clang fp contract(off)
     const float ri = __builtin_amdgcn_rsqf(fmaxf(r2, t * t));
     return (ri * ri) * ri;
 }
 __device__ __forceinline__ float sphx_soft_factor(float r2, float t) {
-    return sphx_spline_f(r2, t) - sphx_clamped_r3(r2, t);
+#pragma clang fp contract(off)
+    const float ri = __builtin_amdgcn_rsqf(fmaxf(r2, t * t));
+    return __builtin_fmaf(-(ri * ri), ri, sphx_spline_f(r2, t));
 }
 
 __device__ __forceinline__ double wave_max_d(double v) {
