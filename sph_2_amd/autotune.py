@@ -10,7 +10,6 @@ from __future__ import annotations
 
 import json
 import os
-import time
 
 CUS = 256
 CANDIDATES = [(1, 256), (1, 512), (2, 256), (2, 512), (2, 1024), (4, 256), (4, 512)]
@@ -102,52 +101,53 @@ def tune_cells(n: int, seed: int = 0, steps: int = 3):
 def pick(res: dict):
     """The fastest shape, except that among shapes within 1 % of it the one
     needing the least extra memory wins: a tiled shape (none), else the
-    symmetric sum with the most block pairs per segment (fewest partial sums),
-    whole block pairs before split ones."""
+    symmetric sum with the most block pairs per segment (fewest partial sums)."""
     t_best = min(res.values())
     near = [k for k, v in res.items() if v <= 1.01 * t_best]
     tiled = [k for k in near if k[0] != 8]
     if tiled:
         return min(tiled, key=res.get)
-    return max(near, key=lambda k: (k[2], k[1]))
+    return max(near, key=lambda k: k[2])
 
 
-def _sweep(libsx, e, n: int, reps: int, res: dict):
-    """Time every candidate shape (stateless call, mean of reps after one
-    warm-up) into res."""
-    import torch
-
-    def timed(cfg):
-        libsx.set_gravity_config(*cfg)
-        libsx.getAcc_g_smth(e.pos, e.m, 1.0, e.h)
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-        for _ in range(reps):
-            libsx.getAcc_g_smth(e.pos, e.m, 1.0, e.h)
-        torch.cuda.synchronize()
-        res[cfg] = (time.perf_counter() - t0) / reps
-
+def _shapes(n: int):
     for ipl, tj in CANDIDATES:
         blocks = (n + 256 * ipl - 1) // (256 * ipl)
         for js in (1, 2, 4, 8, 16):
             if js > 1 and blocks * js > 16 * CUS:
                 break
-            timed((ipl, tj, js))
+            yield ipl, tj, js
     if n <= SYM_MAX_N:
         for S in SYM_SEGMENTS:
-            timed((8, 512, S))
+            yield 8, 512, S
 
 
-def tune_gravity(n: int, seed: int = 0, reps: int = 2, write: bool = True):
-    """Time every candidate shape on an Evrard sphere of n particles."""
-    from . import ic, libsx
+def tune_gravity(n: int, seed: int = 0, reps: int | None = None, write: bool = True):
+    """Time every candidate shape on an Evrard sphere of n particles: the gravity
+    phase (seconds) of the steps of a resident run, whose kernels a shape is
+    chosen for.  (A stateless call with a softening of its own sums the softened
+    pairs with the spline, and its time is its copies and its sort as well.)"""
+    import torch
 
+    from . import ic
+    from .plan import SphPlan
+
+    reps = reps or max(2, min(20, (1 << 21) // n))
     e = ic.evrard(n, seed=seed)
     res = {}
-    try:
-        _sweep(libsx, e, n, reps, res)
-    finally:
-        libsx.set_gravity_config()  # back to the tuned shapes
+    pl = SphPlan(n)
+    pl.load(e.pos, e.vel, e.u, e.m, e.h)
+    pl.init()
+    for cfg in _shapes(n):
+        pl.set_gravity_config(*cfg)
+        pl.step(1, 1e-6)
+        torch.cuda.synchronize()
+        pl.set_timing(True)
+        pl.step(reps, 1e-6)
+        ms, cnt = pl.timing()["gravity"]
+        pl.set_timing(False)
+        res[cfg] = 1e-3 * ms / max(cnt, 1)
+    pl.close()
     best = pick(res)
     if write:
         try:

@@ -56,3 +56,17 @@ def test_symmetric_blocks(gpu, n):
 @pytest.mark.parametrize("cfg", [(1, 256, 16), (8, 512, 1)])
 def test_soft_gravity_by_the_walk(gpu, cfg, lists):
     _check(6000, cfg, lists=lists, wide=True)
+
+
+def test_tuner_times_the_steps_of_a_plan(gpu, monkeypatch):
+    """The shape table is for the kernels of a resident run, not for those of the
+    stateless call."""
+    from sph_2_amd import autotune, libsx
+
+    def never(*a, **kw):
+        raise AssertionError("stateless gravity call")
+
+    monkeypatch.setattr(libsx, "getAcc_g_smth", never)
+    best, res = autotune.tune_gravity(1500, reps=1, write=False)
+    assert ",".join(map(str, best)) in res and all(v > 0.0 for v in res.values())
+    assert {"1,256,1", "2,1024,4", "8,512,1", "8,512,64"} <= set(res)
