@@ -713,7 +713,8 @@ struct StepIter {
 // halved in between.  A window takes nup - ndown + 2 distances at least, of
 // HW_CAP.  Walks of a target on an Evrard sphere of 16,384, from 1.3 times the
 // length (102 passes for all of these): 2.03 on average and 4 at most for the band
-// 59 to 69, 2.41 and 5 for 44 to 84, 3.4 and 9 for 36 to 92; with both ends
+// 59 to 69, 2.41 and 5 for 44 to 84, 3.4 and 9 for 36 to 92 (and from a third of
+// the length to three times it 2.7 and 7 for the first); with both ends
 // scaled together about the middle of the band they were passes and 16 walks
 // more for most targets from bands of 41 counts on.  A wider band, a target left
 // without a window (more than 64 particles at one distance, a start that is not a
@@ -910,22 +911,26 @@ __global__ __launch_bounds__(64) void k_smoothing_steps(Tables t, Soa s, SmoothA
                 open = false;
             } else {
                 // an end that is not near enough: the middle of the radii between
-                // which it must lie, once both are known, before that aimed anew
-                // from its own count (the lower one from the upper's where its
-                // own says too little)
+                // which it must lie, once both are known (at last the one that
+                // is known to do), before that aimed anew from its own count (the
+                // lower one from the upper's where its own says too little)
                 double nw0 = w0, nw1 = w1;
                 if (!lo_ok || base < a.wlo - a.wslack) {
-                    nw0 = 8 * (int64_t)base > a.wlo ? w0 * sphx_h_factor(a.wlo, base)
+                    nw0 = 2 * (int64_t)base > a.wlo ? w0 * sphx_h_factor(a.wlo, base)
                                                     : w1 * sphx_h_factor(a.wlo, tot);
-                    if (lo > 0.0 && u < INFINITY) nw0 = 0.5 * (lo + u);
+                    if (lo > 0.0 && u < INFINITY) nw0 = walk >= 4 && !lo_ok ? lo : 0.5 * (lo + u);
                 }
                 if (!hi_ok || tot - a.wslack > a.whi) {
                     nw1 = w1 * sphx_h_factor(a.whi, tot);
-                    if (v > 0.0 && hi < INFINITY) nw1 = 0.5 * (v + hi);
+                    if (v > 0.0 && hi < INFINITY) nw1 = walk >= 4 && !hi_ok ? hi : 0.5 * (v + hi);
                 }
                 if (a.wlo == 0) nw0 = 0.0;
                 w0 = fmax(lo, nw0);
                 w1 = fmin(hi, nw1);
+                if (!(w0 < w1) && lo < hi && hi < INFINITY) {  // both in one gap
+                    w0 = lo + (hi - lo) / 3.0;
+                    w1 = hi - (hi - lo) / 3.0;
+                }
                 open = w0 < w1 && w1 < INFINITY;
                 if (open) base = inw = 0;
             }

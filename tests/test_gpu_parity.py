@@ -284,8 +284,8 @@ def test_gravity_symmetric(gpu, evr, n, masses, eps):
     the oracle: far block pairs with one common mass, with mixed masses, near
     and diagonal block pairs, partial blocks (n = 3001: a last block of 441,
     whose second half of 256 is partial; 2200: a last block of 152, with no
-    second half; 300: one partial block), segment lengths 1, 3 and 64, and
-    block pairs split into parts of 256 and 128 j particles."""
+    second half; 300: one partial block), segment lengths 1, 3 and 64; the
+    shapes (8, 256, 1) and (8, 128, 1) mean (8, 512, 1)."""
     from sph_2_amd import libsx
 
     rng = np.random.default_rng(n)
@@ -294,12 +294,15 @@ def test_gravity_symmetric(gpu, evr, n, masses, eps):
     e = evr["h"][:n] if eps == "h" else np.full(n, eps)
     acc_o = oracle.gravity(pos, m, e, 1.0)
     try:
-        for tj, S in ((512, 1), (512, 3), (512, 64), (256, 1), (128, 1)):
-            libsx.set_gravity_config(8, tj, S)
+        for S in (1, 3, 64):
+            libsx.set_gravity_config(8, 512, S)
             acc = libsx.getAcc_g_smth(pos, m, 1.0, e)
-            assert rel_rms(acc, acc_o) < 1e-5, (tj, S)
+            assert rel_rms(acc, acc_o) < 1e-5, S
             assert np.max(np.linalg.norm(acc - acc_o, axis=1) /
-                          np.linalg.norm(acc_o, axis=1)) < 1e-4, (tj, S)
+                          np.linalg.norm(acc_o, axis=1)) < 1e-4, S
+            for tj in (256, 128) if S == 1 else ():
+                libsx.set_gravity_config(8, tj, 1)
+                assert np.array_equal(libsx.getAcc_g_smth(pos, m, 1.0, e), acc), tj
             # the potential call falls back to the tiled sum
             acc2, pot = libsx.getAcc_g_smth(pos, m, 1.0, e, return_potential=True)
             assert rel_rms(acc2, acc_o) < 1e-5

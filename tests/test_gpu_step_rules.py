@@ -92,3 +92,27 @@ def test_wide_band_costs_no_more(gpu):
     narrow = best(nngb=64, ndown=59, nup=69)
     wide = best(nngb=64, ndown=44, nup=84)
     assert wide < 2.5 * narrow, (wide, narrow)
+
+
+def test_far_starts_cost_no_more(gpu):
+    """Starts from a third of the length to three times it find their windows too:
+    some 1.5 times what starts from the guess take, where one target walked pass by
+    pass (400 of them) takes five."""
+    import time
+
+    from sph_2_amd import libsx
+
+    e = ic.evrard(98304, seed=17)
+    h0 = e.h.copy()
+    h0[::7] *= np.geomspace(1.0 / 3.0, 3.0, len(h0[::7]))
+
+    def best(h):
+        t = []
+        for _ in range(6):
+            t0 = time.perf_counter()
+            libsx.smoothing_h(e.pos, h, h_mode=5)
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    near, far = best(e.h), best(h0)
+    assert far < 3.0 * near, (far, near)
