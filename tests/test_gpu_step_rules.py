@@ -116,3 +116,44 @@ def test_far_starts_cost_no_more(gpu):
 
     near, far = best(e.h), best(h0)
     assert far < 3.0 * near, (far, near)
+
+
+@pytest.mark.parametrize("h_mode", [2, 4, 5])
+@pytest.mark.parametrize("n", [24576, 24577, 98304, 98305])
+def test_step_rules_at_every_group_size(gpu, n, h_mode):
+    """A quarter, a half and a whole bucket per group (384 / 385 and 1,536 / 1,537
+    buckets, the last one partial), from the guess, from starts up to three times
+    off among them with 80 particles on one point, and (rules with one) from the eq.
+    31 start of a step later: sampled rows, the clustered ones among them."""
+    import warnings
+
+    from sph_2_amd import libsx
+
+    e = ic.evrard(n, seed=17)
+    # (10,001 passes for h_mode 5's clustered rows: one of them)
+    rows = np.unique(np.r_[0:32 if h_mode == 5 else 64, 40, np.linspace(0, n - 1, 160).astype(int)])
+    p = oracle.Params(h_mode=h_mode)
+
+    def check(pos, h0, **kw):
+        ho, ko, ito, _ = oracle.smoothing(pos, h0, p=p, rows=rows, **kw)
+        with warnings.catch_warnings():
+            warnings.simplefilter("ignore", RuntimeWarning)
+            if kw:
+                out = libsx._smoothing(pos, h0, kw["k_prev"], kw["divV"], kw["dt"], None, None,
+                                       "mixed", 0, h_mode=h_mode)
+            else:
+                out = libsx.smoothing_h(pos, h0, h_mode=h_mode)
+        for got, want in zip(out, (ho, ko, ito)):
+            assert np.array_equal(got[rows], want)
+        return out
+
+    check(e.pos, e.h)
+    pos, h0 = e.pos.copy(), e.h.copy()
+    h0[::7] *= np.geomspace(1.0 / 3.0, 3.0, len(h0[::7]))
+    pos[32:112] = pos[32]
+    check(pos, h0)
+    if h_mode != 5:
+        h, k, _ = libsx.smoothing_h(e.pos, e.h)
+        r = np.sqrt((e.pos ** 2).sum(axis=1))
+        vel = -0.8 / (0.3 + r)[:, None] * e.pos
+        check(e.pos + 1e-3 * vel, h, k_prev=k, divV=-0.8 * (0.9 + 2.0 * r) / (0.3 + r) ** 2, dt=1e-3)
