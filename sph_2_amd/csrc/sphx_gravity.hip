@@ -139,7 +139,7 @@ __device__ __forceinline__ void near_pair(IState<IPL> &S, float4 j, float ej, in
         float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
         const float t = S.e[p] + ej;  // 2e; r^2 >= t^2 is r^2 >= (4e) e
         float f, ph;
-        // r^-1 once for both branches (as in sym_spline_f)
+        // r^-1 once for both branches (as in sphx_spline_f)
         const float ri = __builtin_amdgcn_rsqf(r2);
         if (r2 >= t * t) {
             f = ri * ri * ri;

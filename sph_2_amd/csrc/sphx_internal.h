@@ -507,7 +507,7 @@ struct Engine {
     int build_candidates(hipStream_t st);
     // soft: also the softened pairs' gravity sums into s.gx..gz (eps = h)
     int density_eos(hipStream_t st, bool lists = false, bool soft = false);
-    // groups per bucket of the smoothing and list walks (1, 2 or 4)
+    // groups per bucket of the smoothing (1, 2, 4) and list walks (1, 2, 4, 8)
     int smooth_parts() const;
     int list_parts() const;
     bool list_small() const;  // list passes that walk overflowed buckets themselves
