@@ -246,3 +246,28 @@ def test_large_lists_are_given_back(gpu):
     taken = free - gpu.cuda.mem_get_info()[0]
     assert taken < 4.5e9, taken
     assert L.sphx_ctx_destroy(ctx) == 0
+
+
+def test_overflowing_lists_are_walked_by_the_whole_device(gpu):
+    """Eight times the neighbours, so that every list overflows: the walks that
+    take their place cost a few times the list passes (2 to 4 here), not the
+    fiftyfold that 17 waves took for 1,028 buckets."""
+    import time
+
+    from sph_2_amd import libsx
+
+    e = ic.evrard(65752, seed=3)
+    v = np.random.default_rng(1).standard_normal((e.n, 3))
+
+    def best(f):
+        t = []
+        for _ in range(4):
+            t0 = time.perf_counter()
+            f()
+            t.append(time.perf_counter() - t0)
+        return min(t)
+
+    rho = libsx.getDensity(e.pos, e.m, e.h)
+    for f in (lambda h: libsx.getDensity(e.pos, e.m, h), lambda h: libsx.div_curlVel(e.pos, v, rho, e.m, h)):
+        narrow, wide = best(lambda: f(e.h)), best(lambda: f(2.0 * e.h))
+        assert wide < 8.0 * narrow, (wide, narrow)
