@@ -337,7 +337,8 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
         };
         // two buckets' loads are in flight while a third is compacted
         Cand c0 = load(0), c1 = load(1);
-        for (int k = 0; k < nl; ++k) {
+        int lim = nl;
+        for (int k = 0; k < lim; ++k) {
             const Cand c2 = load(k + 2);
             const float rx = (float)((c0.x - f.ox) * f.sc), ry = (float)((c0.y - f.oy) * f.sc),
                         rz = (float)((c0.z - f.oz) * f.sc);
@@ -363,7 +364,10 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
                     L.j[at] = c0.beg + lane;
                 }
                 const int nt = tail + __popcll(m);
-                if ((nt ^ tail) & 64) batch(tail & 64, 64);
+                if ((nt ^ tail) & 64) {
+                    batch(tail & 64, 64);
+                    lim = sink.full() ? 0 : lim;
+                }
                 tail = nt & 127;
             }
             c0 = c1;
@@ -415,6 +419,7 @@ __device__ __forceinline__ int tile_walk(const Tables &t, const Soa &s, WalkLds<
             ncand += __popcll(bmask);
             __builtin_amdgcn_wave_barrier();
             if (nl > TW_LIST - 64) walk();
+            if (sink.full()) return ncand;
         }
     }
     if (nl) walk();
@@ -456,6 +461,7 @@ struct CountSink {
         band = f.sc > 0.0 ? (act ? walk_band(Ss, M) : -1.0f) : INFINITY;
     }
     __device__ __forceinline__ void chunk(double, bool) {}
+    __device__ __forceinline__ bool full() const { return false; }
     __device__ __forceinline__ void begin() { m0 = m1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { m0 = m1; m1 = 0u; }
     __device__ __forceinline__ void cand(float cx, float cy, float cz, float) {
@@ -750,6 +756,7 @@ struct WindowSink {
         band = f.sc > 0.0 ? (act ? walk_band(s1, M) : -1.0f) : INFINITY;
     }
     __device__ __forceinline__ void chunk(double, bool) {}
+    __device__ __forceinline__ bool full() const { return false; }
     __device__ __forceinline__ void begin() { a0 = a1 = b0 = b1 = 0u; amin = INFINITY; }
     __device__ __forceinline__ void word() { a0 = a1; b0 = b1; a1 = b1 = 0u; }
     __device__ __forceinline__ void cand(float cx, float cy, float cz, float) {
@@ -1394,6 +1401,7 @@ struct ListSink {
     bool act;
     uint32_t m0, m1;
     float amin;
+    __device__ __forceinline__ bool full() const { return __any(nn > SPHX_NBR_MAX); }
     __device__ __forceinline__ ListSink(const WalkFrame &f, bool act_, double x, double y, double z,
                                         double h, double hS_, const Soa *s_, int32_t *lst_, int lane_,
                                         int nn_)
@@ -1588,28 +1596,20 @@ __global__ __launch_bounds__(64) void k_density_quad(Tables t, Soa s, DensArgs a
     }
 }
 
-// Calls f for the overflowed ones of a wave's buckets, which are spread over the
-// launch: runs whose lists all overflow (wide h, many neighbours) keep every wave
-// busy.  With 64 consecutive buckets a wave, density with 500 neighbours took 23 ms
-// at 65,752 particles, of which the walks spread out take 0.5.
+// Calls f for the wave's bucket if its lists overflowed.  A wave a bucket: runs
+// whose lists all overflow (wide h, many neighbours) fill the device.  With 64
+// consecutive buckets a wave, density with 500 neighbours took 23 ms at 65,752
+// particles, of which these walks take 0.5.
 template <class F>
-__device__ __forceinline__ void for_overflowed(const Tables &t, const int32_t *ovf, int nb, F f) {
-    const int step = gridDim.x;
-    for (int64_t base = blockIdx.x; base < nb; base += 64 * (int64_t)step) {
-        const int64_t b = base + (int64_t)threadIdx.x * step;
-        uint64_t m = __ballot(b < nb && bucket_ovf(ovf, t.boff + b));
-        while (m) {
-            const int q = __builtin_ctzll(m);
-            m &= m - 1;
-            f(t.boff + (int)base + q * step);
-        }
-    }
+__device__ __forceinline__ void if_overflowed(const Tables &t, const int32_t *ovf, F f) {
+    const int b = t.boff + xcd_block(blockIdx.x, gridDim.x);
+    if (bucket_ovf(ovf, b)) f(b);
 }
 
 // The walk for the buckets whose lists overflowed.
 template <bool SOFT>
-__global__ __launch_bounds__(64) void k_density_ovf(Tables t, Soa s, DensArgs a, int nb) {
-    for_overflowed(t, a.ovf, nb, [&](int b) {
+__global__ __launch_bounds__(64) void k_density_ovf(Tables t, Soa s, DensArgs a) {
+    if_overflowed(t, a.ovf, [&](int b) {
         if (threadIdx.x == 0 && a.counters) atomicAdd((unsigned long long *)&a.counters[CNT_NBR_OVF], 1ull);
         density_bucket<SOFT>(t, s, a, b);
     });
@@ -2077,20 +2077,20 @@ __global__ __launch_bounds__(64) void k_dchydro_quad(Tables t, Soa s, HydroArgs 
     }
 }
 
-__global__ __launch_bounds__(64) void k_divcurl_ovf(Tables t, Soa s, const int32_t *ovf, int nb) {
-    for_overflowed(t, ovf, nb, [&](int b) { divcurl_bucket(t, s, b); });
+__global__ __launch_bounds__(64) void k_divcurl_ovf(Tables t, Soa s, const int32_t *ovf) {
+    if_overflowed(t, ovf, [&](int b) { divcurl_bucket(t, s, b); });
 }
 
-__global__ __launch_bounds__(64) void k_hydro_ovf(Tables t, Soa s, HydroArgs a, const int32_t *ovf,
-                                                  int nb) {
-    for_overflowed(t, ovf, nb, [&](int b) { hydro_bucket(t, s, a, b, false); });
+__global__ __launch_bounds__(64) void k_hydro_ovf(Tables t, Soa s, HydroArgs a,
+                                                  const int32_t *ovf) {
+    if_overflowed(t, ovf, [&](int b) { hydro_bucket(t, s, a, b, false); });
 }
 
 // The overflow walks of the fused pass, div/curl and then hydro (which without
 // the Balsara switch reads nothing of it), in one launch.
 __global__ __launch_bounds__(64) void k_dchydro_ovf(Tables t, Soa s, HydroArgs a,
-                                                    const int32_t *ovf, int nb) {
-    for_overflowed(t, ovf, nb, [&](int b) {
+                                                    const int32_t *ovf) {
+    if_overflowed(t, ovf, [&](int b) {
         divcurl_bucket(t, s, b);
         hydro_bucket(t, s, a, b, true);
     });
@@ -2371,10 +2371,6 @@ int Engine::smoothing(hipStream_t st, bool predictor) {
     return SPHX_OK;
 }
 
-// Launch shape of the overflow walks: a wave a bucket, as far as that fills the
-// device (four a SIMD); most of them find nothing to do.
-static unsigned ovf_grid(unsigned nb) { return std::min(4096u, nb); }
-
 bool Engine::lists_ready() const {
     return use_lists && nbr && prec && fbal && nbr_ovf && nbr_bcap >= t.nb && nbr_pcap >= n;
 }
@@ -2423,8 +2419,8 @@ int Engine::density_eos(hipStream_t st, bool lists, bool soft) {
     } else {
         if (soft) k_density_quad<true, false><<<4 * nb, 64, 0, st>>>(tview(), s, a);
         else k_density_quad<false, false><<<4 * nb, 64, 0, st>>>(tview(), s, a);
-        if (soft) k_density_ovf<true><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
-        else k_density_ovf<false><<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nb);
+        if (soft) k_density_ovf<true><<<nb, 64, 0, st>>>(tview(), s, a);
+        else k_density_ovf<false><<<nb, 64, 0, st>>>(tview(), s, a);
     }
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
@@ -2435,8 +2431,7 @@ int Engine::divcurl(hipStream_t st, bool lists) {
     if (lists) {
         ListArgs L{nbr, prec, nbr_ovf, fbal};
         k_divcurl_list<<<nb_launch(), 64, 0, st>>>(tview(), s, L);
-        k_divcurl_ovf<<<ovf_grid(nb_launch()), 64, 0, st>>>(tview(), s, nbr_ovf,
-                                                           (int)nb_launch());
+        k_divcurl_ovf<<<nb_launch(), 64, 0, st>>>(tview(), s, nbr_ovf);
         if (p.balsara) {
             int64_t p0 = rrun >= 0 ? rp0 : 0, p1 = rrun >= 0 ? rp1 : n;
             if (p1 > p0)
@@ -2465,7 +2460,7 @@ int Engine::divcurl_hydro_lists(hipStream_t st) {
         return SPHX_OK;
     }
     k_dchydro_list<<<nb, 64, 0, st>>>(tview(), s, a, L);
-    k_dchydro_ovf<<<ovf_grid(nb), 64, 0, st>>>(tview(), s, a, nbr_ovf, nb);
+    k_dchydro_ovf<<<nb, 64, 0, st>>>(tview(), s, a, nbr_ovf);
     SPHX_HIP(hipGetLastError());
     return SPHX_OK;
 }
@@ -2477,8 +2472,7 @@ int Engine::hydro(hipStream_t st, bool lists) {
     if (lists) {
         ListArgs L{nbr, prec, nbr_ovf, fbal};
         k_hydro_list<<<nb_launch(), 64, 0, st>>>(tview(), s, a, L);
-        k_hydro_ovf<<<ovf_grid(nb_launch()), 64, 0, st>>>(tview(), s, a, nbr_ovf,
-                                                         (int)nb_launch());
+        k_hydro_ovf<<<nb_launch(), 64, 0, st>>>(tview(), s, a, nbr_ovf);
     } else {
         k_hydro<<<nb_launch(), 64, 0, st>>>(tview(), s, a);
     }
