@@ -203,8 +203,8 @@ def test_far_offsets(gpu, shift):
 
 
 def test_large_lists_are_given_back(gpu):
-    """The stateless calls hold the neighbour lists of small runs only: after a
-    density of 5,000,000 particles (3 GB of lists, 1.3 GB of particle arrays) the
+    """The stateless calls hold the neighbour lists of small runs only: after
+    div/curl of 5,000,000 particles (3 GB of lists, 1.3 GB of particle arrays) the
     device has that memory again, and smaller calls in the same context, whose
     lists are made anew, give what a context of their own gives."""
     import ctypes as C
@@ -215,32 +215,37 @@ def test_large_lists_are_given_back(gpu):
     st = _lib.stream_handle()
     rng = np.random.default_rng(2)
 
-    def density(ctx, n):
+    def divcurl(ctx, n):
         pos, m = _lib.dev(rng.random((n, 3))), _lib.dev(np.full(n, 1.0 / n))
+        v = _lib.dev(rng.standard_normal((n, 3)))
         h = _lib.dev(np.full(n, 0.62 * (64.0 / (4.19 * n)) ** (1.0 / 3.0)))
-        rho = gpu.empty(n, dtype=gpu.float64, device="cuda")
-        args = [a.data_ptr() for a in (pos, m, h)]
-        assert L.sphx_getDensity(ctx, _lib.MIXED, n, *args, 0, n, rho.data_ptr(), None, st) == 0
+        div, curl = (gpu.empty(n, dtype=gpu.float64, device="cuda") for _ in range(2))
+        args = [a.data_ptr() for a in (pos, v, m, m, h)]  # (rho: any)
+
+        def call(c, a, b):
+            assert L.sphx_div_curlVel(c, _lib.MIXED, n, *args, 0, n, a.data_ptr(), b.data_ptr(), st) == 0
+
+        call(ctx, div, curl)
         gpu.cuda.synchronize()
         own = C.c_void_p()
         assert L.sphx_ctx_create(0, C.byref(own)) == 0
-        want = gpu.empty_like(rho)
-        assert L.sphx_getDensity(own, _lib.MIXED, n, *args, 0, n, want.data_ptr(), None, st) == 0
+        want = gpu.empty_like(div), gpu.empty_like(curl)
+        call(own, *want)
         gpu.cuda.synchronize()
         assert L.sphx_ctx_destroy(own) == 0
-        assert gpu.equal(rho, want)
+        assert gpu.equal(div, want[0]) and gpu.equal(curl, want[1])
 
     ctx = C.c_void_p()
     assert L.sphx_ctx_create(0, C.byref(ctx)) == 0
-    density(ctx, 2000)
+    divcurl(ctx, 2000)
     gpu.cuda.empty_cache()
     free = gpu.cuda.mem_get_info()[0]
-    density(ctx, 5_000_000)
+    divcurl(ctx, 5_000_000)
     gpu.cuda.empty_cache()
     taken = free - gpu.cuda.mem_get_info()[0]
     assert taken < 2.0e9, taken
     for n in (1080, 2000, 100_000, 1_000_001):
-        density(ctx, n)
+        divcurl(ctx, n)
     gpu.cuda.synchronize()
     gpu.cuda.empty_cache()
     taken = free - gpu.cuda.mem_get_info()[0]
